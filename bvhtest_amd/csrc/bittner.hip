@@ -590,39 +590,81 @@ __device__ uint32_t decide(PatchRec *r, uint32_t k, uint32_t round, uint64_t *lo
   return REC_WON;
 }
 
+// Sixteen lanes per patch for the kernels that touch every node of a patch:
+// lane j holds node j, so the patch's node ids, their locks and the writes
+// are one round trip each instead of ten in a row (a chunk has a few hundred
+// to a few thousand patches, far too few to hide a chain of loads per
+// thread).  1M triangles, 627 patches: k_commitFirst 13.3 -> 4.8 us,
+// k_apply 11.1 -> 4.8 us.
+constexpr uint32_t kPatchLanes = 16, kPatchBlock = 256, kPatchesPerBlock = kPatchBlock / kPatchLanes;
+
 // Round 1 over every patch (the reservations were made by k_search).
-__global__ __launch_bounds__(256) void k_commitFirst(PatchRec *__restrict__ recs, uint32_t K, uint64_t *locks,
-                                                     uint32_t *__restrict__ marks, uint32_t *__restrict__ skipped,
-                                                     uint32_t *__restrict__ stats, uint32_t *__restrict__ pending,
-                                                     uint32_t *__restrict__ numPending) {
-  const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-  if (k >= K) return;
-  PatchRec *r = recs + k;
-  if (r->ok != REC_PENDING) return;
-  if (decide(r, k, 1, locks, marks, skipped, stats) == REC_PENDING) pending[atomicAdd(numPending, 1u)] = k;
+__global__ __launch_bounds__(kPatchBlock) void k_commitFirst(PatchRec *__restrict__ recs, uint32_t K, uint64_t *locks,
+                                                             uint32_t *__restrict__ marks,
+                                                             uint32_t *__restrict__ skipped,
+                                                             uint32_t *__restrict__ stats,
+                                                             uint32_t *__restrict__ pending,
+                                                             uint32_t *__restrict__ numPending) {
+  const uint32_t k = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes, j = threadIdx.x % kPatchLanes;
+  const bool in = k < K;  // every lane stays for the ballots
+  PatchRec *r = recs + (in ? k : 0);
+  const uint32_t ok = in ? r->ok : (uint32_t)REC_NONE;
+  const uint32_t n = in && j < (uint32_t)kNNode ? r->node[j] : NONE;
+  const uint32_t moved = in && j < 2 ? r->moved[j] : NONE;
+  const bool open = ok == REC_PENDING, use = open && n != NONE;
+  const uint64_t mine = lockKey(1, k);
+  const uint64_t v = use ? __hip_atomic_load(locks + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : mine;
+  const uint32_t group = threadIdx.x & 63u & ~(kPatchLanes - 1);
+  const bool lost = ((__ballot((v >> 32) == 0) >> group) & 0xFFFFu) != 0;  // node of an applied patch
+  const bool holdAll = ((__ballot(v != mine) >> group) & 0xFFFFu) == 0;
+  if (!open) return;
+  if (!lost && holdAll) {
+    if (use)
+      atomicMin(reinterpret_cast<unsigned long long *>(locks + n), (unsigned long long)lockKey(kRoundWin, k));
+    if (j < 2) marks[moved] = k;  // moved roots are patch nodes: one applied patch each
+    if (j == 0) r->ok = REC_WON;
+  } else if (j == 0) {
+    if (lost) {
+      r->ok = REC_LOST;
+      skipped[k] += 1;
+      atomicAdd(stats + ST_CONFLICT, 1u);
+    } else {
+      pending[atomicAdd(numPending, 1u)] = k;
+    }
+  }
 }
 
 // Rounds 2.. over the (few) undecided patches, in one workgroup.  At most
 // `num + 1` rounds are needed; patches still undecided after that bound
 // (never, unless memory ordering is broken) are dropped and counted.
 //
-// Up to kTailBlock patches (one per thread), the rounds run in LDS and
-// registers: the nodes of the undecided patches go into an LDS hash table
-// holding, per node, whether a winner took it (round 1's from its global
-// lock, read once) and the lowest rank reserving it this round, and each
-// thread keeps its patch's table slots in registers.  A round is then LDS
-// atomics and barriers instead of global atomics and loads.  The decisions
-// are those of the global rounds: in round r a patch reserves every node no
-// winner took, wins if it holds them all, loses if a winner took one, and
-// waits otherwise.  Global locks keep their round-1 values (k_apply
-// releases them all).
+// Up to kTailCap patches (two per thread, every node a table slot of its own
+// at worst), the rounds run in LDS and registers: the nodes of the undecided
+// patches go into an LDS hash table holding, per node, whether a winner took
+// it (round 1's from its global lock, read once) and the lowest rank
+// reserving it this round, and each thread keeps its patches' table slots in
+// registers.  A round is two barriers: a patch with a taken node loses, the
+// others reserve their nodes; a patch that holds them all wins and takes
+// them.  (A losing patch no longer reserves, which decides its neighbours no
+// later.)  The reservations of a round are cleared by their own patches
+// while the next round uses the other of two arrays; the second one lies
+// where the node ids were, which are only needed to build the table.  Nothing
+// is written to memory before the last round: a barrier would wait for it.
+// Measured per chunk: 627 patches of 1M triangles 14.1 -> 11.0 us; 1,638
+// patches of 65,536 triangles (10% per step) 48 -> 31 us in the mean, the
+// first chunks of a step, whose more than 1,024 undecided patches took the
+// global rounds before, 168 -> 58 us.
+// Global locks keep their round-1 values (k_apply releases them all).
 constexpr int kTailBlock = 1024;
-constexpr uint32_t kTailSlotsLog = 14, kTailSlots = 1u << kTailSlotsLog;  // LDS hash slots (load <= 0.63)
+constexpr uint32_t kTailSlotsLog = 14, kTailSlots = 1u << kTailSlotsLog;
+constexpr uint32_t kTailCap = kTailSlots / kNNode;  // patches: the table never overflows
+constexpr uint32_t kTailPer = 2;                    // patches per thread
 constexpr uint32_t kTailEmpty = 0xFFFFFFFFu;
+static_assert(kTailCap <= kTailPer * kTailBlock, "every patch of the LDS rounds has a thread");
 
 __device__ __forceinline__ uint32_t tailHash(uint32_t n) { return (n * 0x9E3779B1u) >> (32 - kTailSlotsLog); }
 
-// Slot of node n, inserted if absent (the table never fills).
+// Slot of node n, inserted if absent (the table never overflows).
 __device__ __forceinline__ uint32_t tailInsert(uint32_t *keys, uint32_t n) {
   uint32_t h = tailHash(n);
   for (uint32_t probe = 0; probe < kTailSlots; ++probe) {
@@ -638,79 +680,135 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
                                                            uint32_t *__restrict__ skipped, uint32_t *__restrict__ stats,
                                                            uint32_t *listA, uint32_t *listB,
                                                            const uint32_t *__restrict__ numPending) {
-  __shared__ uint32_t s_key[kTailSlots];   // node id, kTailEmpty
-  __shared__ uint32_t s_min[kTailSlots];   // lowest reserving rank this round
-  __shared__ uint8_t s_taken[kTailSlots];  // taken by a winner
+  __shared__ __align__(16) uint32_t s_min[2][kTailSlots];  // lowest reserving rank, rounds alternate; [1] starts as the node ids
+  __shared__ __align__(16) uint32_t s_taken4[kTailSlots / 4];  // bytes: taken by a winner
+  __shared__ uint32_t s_open[3];                 // undecided patches after a round (rounds rotate)
   __shared__ uint32_t s_cnt;
+  uint8_t *s_taken = reinterpret_cast<uint8_t *>(s_taken4);
   uint32_t num = *numPending;
+  if (num == 0) return;
   const uint32_t maxRound = num + 2;
-  uint32_t round = 2;
-  if (num <= (uint32_t)kTailBlock) {
-    for (uint32_t i = threadIdx.x; i < kTailSlots; i += kTailBlock) s_key[i] = kTailEmpty;
-    __syncthreads();
-    const bool mine = threadIdx.x < num;
-    const uint32_t k = mine ? listA[threadIdx.x] : 0u;
-    uint32_t sl[kNNode];
-    for (int j = 0; j < kNNode; ++j) {
-      const uint32_t n = mine ? recs[k].node[j] : NONE;
-      sl[j] = n == NONE ? kTailEmpty : tailInsert(s_key, n);
+  if (num <= kTailCap) {
+    uint32_t k[kTailPer], node[kTailPer][kNNode], moved[kTailPer][2];
+    bool taken[kTailPer][kNNode];
+#pragma unroll
+    for (uint32_t q = 0; q < kTailPer; ++q) {
+      const uint32_t at = threadIdx.x + q * kTailBlock;
+      k[q] = at < num ? listA[at] : NONE;
     }
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < kTailSlots; i += kTailBlock) {
-      s_min[i] = kTailEmpty;
-      const uint32_t n = s_key[i];
-      s_taken[i] = n != kTailEmpty &&
-                   (__hip_atomic_load(locks + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) == 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kTailPer; ++q) {
+      const PatchRec *r = recs + (k[q] == NONE ? 0u : k[q]);
+#pragma unroll
+      for (int j = 0; j < kNNode; ++j) node[q][j] = k[q] == NONE ? NONE : r->node[j];
+      moved[q][0] = r->moved[0];
+      moved[q][1] = r->moved[1];
     }
-    bool open = mine;  // undecided
+    uint4 *min4 = reinterpret_cast<uint4 *>(&s_min[0][0]), *taken16 = reinterpret_cast<uint4 *>(s_taken4);
+    for (uint32_t i = threadIdx.x; i < 2 * kTailSlots / 4; i += kTailBlock)
+      min4[i] = make_uint4(kTailEmpty, kTailEmpty, kTailEmpty, kTailEmpty);
+    for (uint32_t i = threadIdx.x; i < kTailSlots / 16; i += kTailBlock) taken16[i] = make_uint4(0, 0, 0, 0);
+    if (threadIdx.x < 3) s_open[threadIdx.x] = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kTailPer; ++q)
+#pragma unroll
+      for (int j = 0; j < kNNode; ++j)
+        taken[q][j] = node[q][j] != NONE &&
+                      (__hip_atomic_load(locks + node[q][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) == 0;
     __syncthreads();
-    for (; num > 0 && round <= maxRound; ++round) {
-      if (open)  // reserve
-        for (int j = 0; j < kNNode; ++j)
-          if (sl[j] != kTailEmpty && !s_taken[sl[j]]) atomicMin(s_min + sl[j], k);
-      if (threadIdx.x == 0) s_cnt = 0;
-      __syncthreads();
-      if (open) {  // decide
-        bool holdAll = true, lost = false;
-        for (int j = 0; j < kNNode; ++j) {
-          if (sl[j] == kTailEmpty) continue;
-          if (s_taken[sl[j]]) lost = true;
-          if (s_min[sl[j]] != k) holdAll = false;
+#pragma unroll
+    for (uint32_t q = 0; q < kTailPer; ++q)
+#pragma unroll
+      for (int j = 0; j < kNNode; ++j)
+        if (node[q][j] != NONE) {  // node[][] holds table slots from here on
+          node[q][j] = tailInsert(s_min[1], node[q][j]);
+          if (taken[q][j]) s_taken[node[q][j]] = 1;
         }
-        PatchRec *r = recs + k;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < kTailPer; ++q)  // the node ids give way to the odd rounds' reservations
+#pragma unroll
+      for (int j = 0; j < kNNode; ++j)
+        if (node[q][j] != NONE) s_min[1][node[q][j]] = kTailEmpty;
+    uint32_t state[kTailPer];
+    bool reserved[kTailPer];  // in the round before
+#pragma unroll
+    for (uint32_t q = 0; q < kTailPer; ++q) {
+      state[q] = k[q] == NONE ? REC_NONE : REC_PENDING;
+      reserved[q] = false;
+    }
+    __syncthreads();
+    for (uint32_t round = 0; round <= maxRound; ++round) {
+      uint32_t *cur = s_min[round & 1], *old = s_min[(round & 1) ^ 1];
+      bool now[kTailPer];
+#pragma unroll
+      for (uint32_t q = 0; q < kTailPer; ++q) {
+        now[q] = false;
+        if (state[q] != REC_PENDING) continue;
+        bool lost = false;
+#pragma unroll
+        for (int j = 0; j < kNNode; ++j) lost |= node[q][j] != NONE && s_taken[node[q][j]] != 0;
         if (lost) {
-          r->ok = REC_LOST;
-          skipped[k] += 1;
-          atomicAdd(stats + ST_CONFLICT, 1u);
-          open = false;
-        } else if (holdAll) {
-          for (int j = 0; j < kNNode; ++j)
-            if (sl[j] != kTailEmpty) s_taken[sl[j]] = 1;
-          r->ok = REC_WON;
-          marks[r->moved[0]] = k;  // moved roots are patch nodes: one applied patch each
-          marks[r->moved[1]] = k;
-          open = false;
-        } else {
-          atomicAdd(&s_cnt, 1u);
+          state[q] = REC_LOST;
+          continue;
         }
+        now[q] = true;
+#pragma unroll
+        for (int j = 0; j < kNNode; ++j)
+          if (node[q][j] != NONE) atomicMin(cur + node[q][j], k[q]);
       }
+      if (threadIdx.x == 0) s_open[(round + 1) % 3] = 0;
       __syncthreads();
-      num = s_cnt;
-      for (uint32_t i = threadIdx.x; i < kTailSlots; i += kTailBlock) s_min[i] = kTailEmpty;
+      uint32_t open = 0;
+#pragma unroll
+      for (uint32_t q = 0; q < kTailPer; ++q) {
+        if (reserved[q]) {
+#pragma unroll
+          for (int j = 0; j < kNNode; ++j)
+            if (node[q][j] != NONE) old[node[q][j]] = kTailEmpty;
+        }
+        reserved[q] = now[q];
+        if (!now[q]) continue;
+        bool holdAll = true;
+#pragma unroll
+        for (int j = 0; j < kNNode; ++j) holdAll &= node[q][j] == NONE || cur[node[q][j]] == k[q];
+        if (!holdAll) {
+          ++open;
+          continue;
+        }
+        state[q] = REC_WON;
+#pragma unroll
+        for (int j = 0; j < kNNode; ++j)
+          if (node[q][j] != NONE) s_taken[node[q][j]] = 1;
+      }
+      if (open) atomicAdd(&s_open[round % 3], open);
       __syncthreads();
+      if (s_open[round % 3] == 0) break;  // workgroup-uniform
     }
-    if (open) {
-      recs[k].ok = REC_LOST;
-      skipped[k] += 1;
-      atomicAdd(stats + ST_CONFLICT, 1u);
-      atomicAdd(stats + ST_UNRESOLVED, 1u);
+    uint32_t conflicts = 0, unresolved = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kTailPer; ++q) {
+      if (state[q] == REC_NONE) continue;
+      PatchRec *r = recs + k[q];
+      if (state[q] == REC_WON) {
+        r->ok = REC_WON;
+        marks[moved[q][0]] = k[q];  // moved roots are patch nodes: one applied patch each
+        marks[moved[q][1]] = k[q];
+        continue;
+      }
+      unresolved += state[q] == REC_PENDING;
+      ++conflicts;
+      r->ok = REC_LOST;
+      skipped[k[q]] += 1;
     }
+    if (conflicts) atomicAdd(stats + ST_CONFLICT, conflicts);
+    if (unresolved) atomicAdd(stats + ST_UNRESOLVED, unresolved);
     return;
   }
   // more undecided patches than the LDS table takes: the rounds on the
   // global locks
   uint32_t *cur = listA, *nxt = listB;
-  for (; num > 0 && round <= maxRound; ++round) {
+  for (uint32_t round = 2; num > 0 && round <= maxRound; ++round) {
     for (uint32_t i = threadIdx.x; i < num; i += kTailBlock) reserve(recs + cur[i], cur[i], round, locks);
     if (threadIdx.x == 0) s_cnt = 0;
     __syncthreads();
@@ -735,28 +833,37 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
 }
 
 // Drops a winner whose insertion point lies below a node another winner moves.
-__global__ __launch_bounds__(256) void k_contain(PatchRec *__restrict__ recs, uint32_t K,
-                                                 const bvht_BVHNode *__restrict__ nodes, uint32_t root, uint32_t N,
-                                                 const uint32_t *__restrict__ marks, uint32_t *__restrict__ skipped,
-                                                 uint32_t *__restrict__ stats) {
-  const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-  if (k >= K) return;
-  PatchRec *r = recs + k;
-  if (r->ok != REC_WON) return;
+// Two lanes per patch, one for each insertion point; a level's mark and
+// parent link are loaded together, so a level costs one round trip (1M
+// triangles: 31.1 -> 12.4 us with the two walks one after the other and
+// two dependent loads per level before).
+constexpr uint32_t kContainBlock = 64;
+__global__ __launch_bounds__(kContainBlock) void k_contain(PatchRec *__restrict__ recs, uint32_t K,
+                                                           const bvht_BVHNode *__restrict__ nodes, uint32_t root,
+                                                           uint32_t N, const uint32_t *__restrict__ marks,
+                                                           uint32_t *__restrict__ skipped,
+                                                           uint32_t *__restrict__ stats) {
+  const uint32_t k = blockIdx.x * (kContainBlock / 2) + threadIdx.x / 2, w = threadIdx.x & 1;
+  const bool in = k < K;  // every lane stays for the shuffle
+  PatchRec *r = recs + (in ? k : 0);
+  const uint32_t ok = in ? r->ok : (uint32_t)REC_NONE;
+  uint32_t x = r->best[w];  // written for every patch that reserved; only read for winners
+  const bool won = ok == REC_WON;
   bool bad = false;
-  for (int w = 0; w < 2 && !bad; ++w) {
-    uint32_t x = r->best[w];
+  if (won) {
     for (uint32_t steps = 0; steps < N; ++steps) {
-      const uint32_t m = marks[x];
+      uint32_t m = marks[x], p = nodes[x].parent;
+      asm volatile("" : "+v"(m), "+v"(p));  // both loads go out before either is used
       if (m != NONE && m != k) {
         bad = true;
         break;
       }
       if (x == root) break;
-      x = nodes[x].parent;
+      x = p;
     }
   }
-  if (bad) {
+  const bool other = __shfl_xor((int)bad, 1, 64) != 0;
+  if (won && w == 0 && (bad || other)) {
     r->ok = REC_CONTAINED;
     skipped[k] += 1;
     atomicAdd(stats + ST_CONTAIN, 1u);
@@ -764,33 +871,36 @@ __global__ __launch_bounds__(256) void k_contain(PatchRec *__restrict__ recs, ui
 }
 
 // Winners write their topology; every patch releases its locks and marks.
-__global__ __launch_bounds__(256) void k_apply(PatchRec *__restrict__ recs, uint32_t K, bvht_BVHNode *__restrict__ nodes,
-                                               uint64_t *__restrict__ locks, uint32_t *__restrict__ marks,
-                                               uint32_t *__restrict__ fixStarts, uint32_t *__restrict__ numPending,
-                                               uint32_t *__restrict__ stats) {
-  const uint32_t k = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(kPatchBlock) void k_apply(PatchRec *__restrict__ recs, uint32_t K,
+                                                       bvht_BVHNode *__restrict__ nodes, uint64_t *__restrict__ locks,
+                                                       uint32_t *__restrict__ marks, uint32_t *__restrict__ fixStarts,
+                                                       uint32_t *__restrict__ numPending,
+                                                       uint32_t *__restrict__ stats) {
+  const uint32_t k = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes, j = threadIdx.x % kPatchLanes;
   if (k >= K) return;
-  if (k == 0) *numPending = 0;
+  if (k == 0 && j == 0) *numPending = 0;
   PatchRec *r = recs + k;
-  const uint32_t ok = r->ok;
+  const uint32_t ok = r->ok;  // read by all 16 lanes (of one wave) before lane 0 writes it below
+  const uint32_t jn = j < (uint32_t)kNNode ? j : 0u;
+  const uint32_t n = r->node[jn], parent = r->parent[jn], left = r->left[jn], right = r->right[jn],
+                 isLeft = r->isLeft[jn], fix = r->fix[j < 3 ? j : 0u], moved = r->moved[j & 1];
   const bool win = ok == REC_WON;
-  for (int i = 0; i < 3; ++i) fixStarts[3 * k + i] = win ? r->fix[i] : NONE;
+  if (j < 3) fixStarts[3 * k + j] = win ? fix : NONE;
   if (ok == REC_NONE) return;
-  for (int i = 0; i < kNNode; ++i) {
-    const uint32_t n = r->node[i];
-    if (n == NONE) continue;
+  if (j < (uint32_t)kNNode && n != NONE) {
     locks[n] = kLockFree;
     if (win) {  // MiniPatch::applyOne -- BVHPatch.hpp:72-80
-      nodes[n].parent = r->parent[i];
-      nodes[n].left = r->left[i];
-      nodes[n].right = r->right[i];
-      nodes[n].isLeft = (uint16_t)r->isLeft[i];
+      nodes[n].parent = parent;
+      nodes[n].left = left;
+      nodes[n].right = right;
+      nodes[n].isLeft = (uint16_t)isLeft;
     }
   }
-  marks[r->moved[0]] = NONE;
-  marks[r->moved[1]] = NONE;
-  r->ok = REC_NONE;
-  if (win) atomicAdd(stats + ST_APPLIED, 1u);
+  if (j >= 14) marks[moved] = NONE;
+  if (j == 0) {
+    r->ok = REC_NONE;
+    if (win) atomicAdd(stats + ST_APPLIED, 1u);
+  }
 }
 
 // kFixTree3_1 -- Bittner13CUDA.cu:407-423: count the arrivals per node.
@@ -1475,16 +1585,16 @@ void bn13_rmAndReinsChunk(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer
                                           in->recs, in->locks, in->stats, sinkOf(in),
                                           chunk == 0 ? in->sortScratch + in->plan.errOff : nullptr);
   if (!checkLaunch("k_search")) return;
-  k_commitFirst<<<divUp(K, 256), 256, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped, in->stats,
+  k_commitFirst<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped, in->stats,
                                                      in->pending[0], in->numPending);
   if (!checkLaunch("k_commitFirst")) return;
   k_resolveTail<<<1, kTailBlock, 0, stream()>>>(in->recs, in->locks, in->marks, in->skipped, in->stats, in->pending[0],
                                                 in->pending[1], in->numPending);
   if (!checkLaunch("k_resolveTail")) return;
-  k_contain<<<divUp(K, 256), 256, 0, stream()>>>(in->recs, K, bvh->nodes, in->root, in->N, in->marks, in->skipped,
+  k_contain<<<divUp(K, kContainBlock / 2), kContainBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->root, in->N, in->marks, in->skipped,
                                                  in->stats);
   if (!checkLaunch("k_contain")) return;
-  k_apply<<<divUp(K, 256), 256, 0, stream()>>>(in->recs, K, bvh->nodes, in->locks, in->marks, in->fixStarts,
+  k_apply<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->locks, in->marks, in->fixStarts,
                                                in->numPending, in->stats);
   if (!checkLaunch("k_apply")) return;
   const uint32_t num = 3 * K;
