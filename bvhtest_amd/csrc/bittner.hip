@@ -19,15 +19,16 @@
 //               the reference has no guard);
 //     k_apply   winners write their topology, all locks are released;
 //     k_refit   two-phase targeted refit from the 3 changed nodes of every
-//               winner (kFixTree3_1 / kFixTree3_2 protocol, agent-scope
-//               acquire/release atomics).  Boxes are exact min/max, so this
-//               equals the reference's full refit (kFixTree1).
+//               winner (the kFixTree3_1 / kFixTree3_2 result).  Boxes are
+//               exact min/max, so this equals the reference's full refit
+//               (kFixTree1).
 // The root never moves (reinsertion at the root is refused, :310).
 #include "mlp.hpp"
 #include "radix_sort.hpp"
 #include "refit.hpp"
 #include "wave.hpp"
 
+#include <algorithm>
 #include <cstring>
 #include <new>
 #include <vector>
@@ -97,6 +98,12 @@ __device__ __forceinline__ void globalBox(const bvht_BVHNode *nodes, uint32_t n,
   b[3] = __uint_as_float(a.w);
   b[4] = __uint_as_float(w.x);
   b[5] = __uint_as_float(w.y);
+}
+
+__device__ __forceinline__ void storeBox(bvht_BVHNode *nd, const float b[6], float sa) {
+  reinterpret_cast<float4 *>(nd)[0] = make_float4(b[0], b[1], b[2], b[3]);
+  reinterpret_cast<float2 *>(nd)[2] = make_float2(b[4], b[5]);
+  nd->surfaceArea = sa;
 }
 
 __device__ __forceinline__ float sa6(const float b[6]) { return surfaceArea(b[0], b[1], b[2], b[3], b[4], b[5]); }
@@ -903,78 +910,281 @@ __global__ __launch_bounds__(kPatchBlock) void k_apply(PatchRec *__restrict__ re
   }
 }
 
-// kFixTree3_1 -- Bittner13CUDA.cu:407-423: count the arrivals per node.
-__global__ __launch_bounds__(256) void k_refitCount(const uint32_t *__restrict__ starts, uint32_t num,
-                                                    const bvht_BVHNode *__restrict__ nodes, uint32_t N,
-                                                    uint32_t *__restrict__ cnt) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= num) return;
+// ---- targeted refit (kFixTree3, Bittner13CUDA.cu:407-467) ------------------
+//
+// Two launches over the start nodes.  k_refitCount marks the paths from the
+// starts to the root: a node's word holds how many of its children are on a
+// path (bits 0-1), whether it is a start (bit 2), whether it is one more than
+// once (bit 3) and, when both children are, the slot their walks meet in
+// (bits 4..31: the index of the start whose walk arrived second and ended
+// there, so no counter hands them out).  k_refitApply then walks up with the
+// box of the node below in registers:
+//   one child on a path   the other child's box does not change during the
+//                         refit: a plain load that goes out beside the
+//                         parent's links and word, one round trip per level;
+//   both on a path        each walk exchanges its box into the slot.  The
+//                         exchanged words carry the box and a tag, so one
+//                         round trip tells a walk whether it came second and
+//                         hands it the other's box; the first one ends.  The
+//                         words of two walks may interleave: the walk that
+//                         came second on word 0 goes on, and waits for the
+//                         words that it reached first (the other walk has
+//                         already issued them).
+// Nothing else passes between walks, so boxes and words are written with
+// plain stores.  Before, every level was an arrival count, coherent loads of
+// both children's boxes and coherent stores that were waited for, three round
+// trips past the L2: 1,881 starts in 1M triangles 59 -> 23 us, 100,000
+// leaves of them 57 -> 37 us.
+constexpr uint32_t kRefitChildren = 3u, kRefitStart = 4u, kRefitDup = 8u, kRefitSlotShift = 4u;
+constexpr uint32_t kRefitBlock = 256;
+
+__global__ __launch_bounds__(kRefitBlock) void k_refitCount(const uint32_t *__restrict__ starts, uint32_t num,
+                                                            uint32_t walks, const bvht_BVHNode *__restrict__ nodes, uint32_t N,
+                                                            uint32_t *__restrict__ cnt) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t i = (blockIdx.x * (kRefitBlock / 64) + threadIdx.x / 64) * walks + lane;
+  if (lane >= walks || i >= num) return;
   uint32_t node = starts[i];
   if (node >= N) return;
-  for (uint32_t steps = 0; steps < N; ++steps) {
-    const uint32_t p = loadRelaxedAgent(&nodes[node].parent);  // issued beside the count: one round trip per level
-    if (atomicAdd(cnt + node, 1u) != 0) return;
-    if (p == node) return;
+  uint32_t p = loadRelaxedAgent(&nodes[node].parent);  // issued beside the count: one round trip per level
+  uint32_t old = atomicOr(cnt + node, kRefitStart);
+  if (old & kRefitStart) atomicOr(cnt + node, kRefitDup);
+  for (uint32_t steps = 0; steps < N && old == 0; ++steps) {  // the first to touch a node walks on
+    if (p == node || p >= N) return;
     node = p;
+    p = loadRelaxedAgent(&nodes[node].parent);
+    old = atomicAdd(cnt + node, 1u);
+    if ((old & kRefitChildren) == 1) atomicOr(cnt + node, i << kRefitSlotShift);
   }
 }
 
-// kFixTree3_2 -- Bittner13CUDA.cu:425-467: the last arrival recomputes.
-// With leafCnt/subSA (the learned priority's subtree features) the same walk
-// keeps them exact: the nodes it recomputes are exactly those whose subtree
-// changed.
-__global__ __launch_bounds__(256) void k_refitApply(const uint32_t *__restrict__ starts, uint32_t num,
-                                                    bvht_BVHNode *__restrict__ nodes, uint32_t N,
-                                                    uint32_t *__restrict__ cnt, uint32_t *leafCnt, float *subSA) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= num) return;
-  uint32_t node = starts[i];
-  if (node >= N) return;
-  if (nodes[node].isLeafFlag != 0) {
-    // a leaf start (dynamic refit) is not recomputed; k_refitCount counted
-    // every occurrence of it and walked on once, so only the last
-    // occurrence walks on here (a list may name a leaf more than once)
-    if (__hip_atomic_fetch_sub(cnt + node, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 1) return;
-    const uint32_t p = nodes[node].parent;
-    if (p == node || p >= N) return;
-    node = p;
+// Words of a slot: three halfwords of payload below a 16-bit tag (0: empty,
+// 1: from the left child, 2: from the right).
+template <int WORDS>
+__device__ __forceinline__ void packSlot(const uint32_t (&v)[6 + 2 * (WORDS - 4) / 2], uint32_t tag,
+                                         uint64_t (&w)[WORDS]) {
+  constexpr int VALS = 6 + 2 * (WORDS - 4) / 2;
+#pragma unroll
+  for (int i = 0; i < WORDS; ++i) {
+    uint64_t x = (uint64_t)tag << 48;
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+      const int at = 3 * i + h;
+      if (at < 2 * VALS) x |= (uint64_t)((v[at / 2] >> (16 * (at & 1))) & 0xFFFFu) << (16 * h);
+    }
+    w[i] = x;
   }
-  for (uint32_t steps = 0; steps < N; ++steps) {
-    // The topology does not change during the refit, so its load goes out
-    // beside the count (the chain of last arrivals near the root is serial:
-    // each level costs the count, the child boxes and the stores).  Relaxed
-    // atomic loads keep the compiler from sinking them below the count.
-    const uint32_t p = loadRelaxedAgent(&nodes[node].parent), l = loadRelaxedAgent(&nodes[node].left),
-                   r = loadRelaxedAgent(&nodes[node].right);
-    const uint32_t left = __hip_atomic_fetch_sub(cnt + node, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (left != 1) return;
-    // Boxes and features written by this walk move between XCDs through
-    // device-coherent accesses: the loads below read past the L2 (issued
-    // after the count returned), the stores write through it and are waited
-    // for before the next count.  This replaces an acquire fence (an L2
-    // invalidation) and a release fence (an L2 write-back) per level.
-    bvht_AABB b = loadBoxAgent(nodes + l);
-    const bvht_AABB br = loadBoxAgent(nodes + r);
-    // the children's subtree features load with their boxes, ahead of the
-    // node's stores (which may alias them), not one round trip later
-    uint32_t cl = 0, cr = 0;
-    float sl = 0.0f, sr = 0.0f;
-    if (leafCnt) {
-      cl = loadRelaxedAgent(leafCnt + l);
-      cr = loadRelaxedAgent(leafCnt + r);
-      sl = loadRelaxedAgent(subSA + l);
-      sr = loadRelaxedAgent(subSA + r);
+}
+template <int WORDS>
+__device__ __forceinline__ void unpackSlot(const uint64_t (&w)[WORDS], uint32_t (&v)[6 + 2 * (WORDS - 4) / 2]) {
+  constexpr int VALS = 6 + 2 * (WORDS - 4) / 2;
+#pragma unroll
+  for (int k = 0; k < VALS; ++k) v[k] = 0;
+#pragma unroll
+  for (int at = 0; at < 2 * VALS; ++at)
+    v[at / 2] |= (uint32_t)((w[at / 3] >> (16 * (at % 3))) & 0xFFFFu) << (16 * (at & 1));
+}
+
+// With FEAT (the learned priority's subtree features) the walk also keeps
+// leaf counts and subtree areas exact: the nodes it recomputes are exactly
+// those whose subtree changed.
+//
+// A walk is bound by latency, so a level is one round trip for every lane of
+// the wave, whichever way its two children are: the next level's links, the
+// other child's box (unused where it comes from the slot) and the exchanges
+// go out together, and a node's own stores follow them (vector memory
+// operations retire in order, so stores ahead of the loads would be waited
+// for).  `walks` of a wave's lanes walk (the low ones): with few walks, fewer
+// lanes a wave means fewer scattered accesses an instruction.
+//
+// NEAR: neighbours in the list are neighbours in the tree (a list of leaves
+// in their order), and most walks meet inside their workgroup.  They do so
+// in LDS first: the one that comes first leaves its box under the node's id
+// and stops, the second takes it and goes on.  When every walk of the
+// workgroup has stopped, those whose box nobody took meet other workgroups'
+// walks in the slots.  Exchanging everything in the slots instead is bound
+// by the exchanges themselves (100,000 leaves of 1M: 52 us against 37).
+constexpr uint32_t kNearSlots = 2 * kRefitBlock;  // LDS table, at most half full
+template <bool FEAT, bool NEAR>
+__global__ __launch_bounds__(kRefitBlock) void k_refitApply(const uint32_t *__restrict__ starts, uint32_t num,
+                                                            uint32_t walks, bvht_BVHNode *__restrict__ nodes,
+                                                            uint32_t N, uint32_t *__restrict__ cnt, uint64_t *slots,
+                                                            uint32_t *__restrict__ leafCnt,
+                                                            float *__restrict__ subSA, uint32_t *__restrict__ stats) {
+  static_assert(!(FEAT && NEAR), "a near list keeps no features");
+  constexpr int WORDS = FEAT ? 6 : 4;
+  __shared__ unsigned long long s_key[NEAR ? kNearSlots : 1];  // node id << 32 | thread that left its box
+  __shared__ uint32_t s_box[6][NEAR ? kRefitBlock : 1];
+  __shared__ uint32_t s_taken[NEAR ? kRefitBlock : 1];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  if (NEAR) {
+    for (uint32_t k = tid; k < kNearSlots; k += kRefitBlock) s_key[k] = ~0ull;
+    s_taken[tid] = 0;
+    __syncthreads();
+  }
+  const uint32_t i = (blockIdx.x * (kRefitBlock / 64) + tid / 64) * walks + lane;
+  uint32_t child = lane < walks && i < num ? starts[i] : NONE;
+  bool go = child < N;
+  if (!go) child = 0;
+  NodeView nv = globalView(nodes, child);
+  uint32_t c = cnt[child];
+  // a walk from below recomputes the node (or has: its word is cleared)
+  go = go && c != 0 && (c & kRefitChildren) == 0;
+  // one occurrence of a start named more than once goes on
+  if (go && (c & kRefitDup)) go = atomicExch(cnt + child, 0u) != 0;
+  if (!NEAR && !go) return;
+  uint32_t node = nv.parent;
+  bool end = node == child || node >= N;
+  NodeView nvUp = globalView(nodes, end ? child : node);
+  uint32_t cUp = cnt[end ? child : node];
+  // the node below (`child`): its box and area
+  float b[6], sa, sub = 0.0f;
+  uint32_t leaves = 0;
+  if (nv.isLeaf == 0) {
+    float r[6];
+    globalBox(nodes, nv.left, b);
+    globalBox(nodes, nv.right, r);
+    merge6(b, r);
+    sa = sa6(b);
+    if (FEAT) {
+      leaves = leafCnt[nv.left] + leafCnt[nv.right];
+      sub = subSA[nv.left] + subSA[nv.right] + sa;
     }
-    mergeInto(b, br);
-    const float sa = surfaceArea(b);
-    storeBoxAgent(nodes + node, b, sa);
-    if (leafCnt) {
-      storeRelaxedAgent(leafCnt + node, cl + cr);
-      storeRelaxedAgent(subSA + node, sl + sr + sa);
+  } else {  // a leaf start (dynamic refit) is not recomputed: it keeps its values
+    globalBox(nodes, child, b);
+    sa = nodes[child].surfaceArea;
+    if (FEAT) {
+      leaves = leafCnt[child];
+      sub = subSA[child];
     }
-    waitVectorMemory();
-    if (p == node) return;
-    node = p;
+  }
+  // complete before the loop, whose waits then only count the loop's own loads
+  asm volatile("" : "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]), "+v"(b[4]), "+v"(b[5]), "+v"(sa), "+v"(leaves),
+                    "+v"(sub), "+v"(nvUp.parent), "+v"(nvUp.left), "+v"(nvUp.right), "+v"(cUp));
+#pragma unroll
+  for (int phase = NEAR ? 0 : 1; phase < 2; ++phase) {
+    bool wait = false;  // stopped with its box left in LDS
+    for (uint32_t steps = 0; go && steps <= N; ++steps) {
+      nv = nvUp;
+      c = cUp;
+      const bool left = nv.left == child;
+      const uint32_t sib = left ? nv.right : nv.left, p = nv.parent;
+      const bool top = p == node || p >= N;
+      const bool meet = !end && (c & kRefitChildren) != 1;
+      const uint32_t at = c >> kRefitSlotShift;
+      float s[6];
+      uint32_t sibLeaves = 0;
+      float sibSub = 0.0f;
+      if (!end) {
+        // the next level's links and word (both fixed until this walk arrives)
+        nvUp = globalView(nodes, top ? node : p);
+        cUp = cnt[top ? node : p];
+        globalBox(nodes, sib, s);
+        if (FEAT) {
+          sibLeaves = leafCnt[sib];
+          sibSub = subSA[sib];
+        }
+      }
+      uint64_t w[WORDS];
+      uint64_t *slot = slots + (size_t)at * WORDS;
+      const bool bad = meet && at >= num;  // not a tree (more than two children on a path)
+      if (phase == 1 && meet && !bad) {
+        uint32_t v[6 + 2 * (WORDS - 4) / 2];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) v[k] = __float_as_uint(b[k]);
+        if constexpr (FEAT) {
+          v[6] = leaves;
+          v[7] = __float_as_uint(sub);
+        }
+        packSlot<WORDS>(v, left ? 1u : 2u, w);
+#pragma unroll
+        for (int k = 0; k < WORDS; ++k)
+          w[k] = __hip_atomic_exchange(slot + k, w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      storeBox(nodes + child, b, sa);
+      if (FEAT) {
+        leafCnt[child] = leaves;
+        subSA[child] = sub;
+      }
+      cnt[child] = 0;
+      if (end || bad) break;
+      if (phase == 0 && meet) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+          __hip_atomic_store(&s_box[k][tid], __float_as_uint(b[k]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        memoryChanged();  // the box before its key (LDS operations of a wave stay in order)
+        uint32_t h = (node * 0x9E3779B1u) >> 16 & (kNearSlots - 1);
+        uint32_t from = NONE;
+        for (uint32_t probe = 0; probe < kNearSlots; ++probe) {
+          const unsigned long long old = atomicCAS(s_key + h, ~0ull, ((unsigned long long)node << 32) | tid);
+          if (old == ~0ull) break;
+          if ((uint32_t)(old >> 32) == node) {
+            from = (uint32_t)old;
+            break;
+          }
+          h = (h + 1) & (kNearSlots - 1);
+        }
+        if (from == NONE) {
+          wait = true;
+          break;
+        }
+        s_taken[from] = 1;
+        memoryChanged();
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+          s[k] = __uint_as_float(
+              __hip_atomic_load(&s_box[k][from], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+      }
+      if (phase == 1 && meet) {
+        if ((w[0] >> 48) == 0) break;  // first: the other walk goes on
+        const uint32_t other = left ? 2u : 1u;
+        for (uint32_t spins = 0;; ++spins) {
+          bool missing = false;
+#pragma unroll
+          for (int k = 1; k < WORDS; ++k) missing |= (w[k] >> 48) != other;
+          if (!missing) break;
+          if (spins > (1u << 22)) {  // never, unless memory is broken: counted, the box is then wrong
+            atomicAdd(stats + ST_UNRESOLVED, 1u);
+            break;
+          }
+#pragma unroll
+          for (int k = 1; k < WORDS; ++k)
+            if ((w[k] >> 48) != other)
+              w[k] = __hip_atomic_load(slot + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        uint32_t v[6 + 2 * (WORDS - 4) / 2];
+        unpackSlot<WORDS>(w, v);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) s[k] = __uint_as_float(v[k]);
+        if constexpr (FEAT) {
+          sibLeaves = v[6];
+          sibSub = __uint_as_float(v[7]);
+        }
+#pragma unroll
+        for (int k = 0; k < WORDS; ++k)
+          __hip_atomic_store(slot + k, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      // the left child's box merges the right one's
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        const float l = left ? b[k] : s[k], r = left ? s[k] : b[k];
+        b[k] = k < 3 ? mergeMin(l, r) : mergeMax(l, r);
+      }
+      sa = sa6(b);
+      if (FEAT) {
+        leaves += sibLeaves;
+        sub = sub + sibSub + sa;  // commutes: left + right + own
+      }
+      child = node;
+      node = p;
+      end = top;
+    }
+    if (phase == 0) {  // whose box nobody took goes on from the same node
+      __syncthreads();
+      go = wait && s_taken[tid] == 0;
+      nvUp = nv;
+      cUp = c;
+    }
   }
 }
 
@@ -1186,10 +1396,16 @@ struct Internal {
   SortPlan plan;
   uint32_t *sorted = nullptr;  // -> vals[result]
   PatchRec *recs = nullptr;
+  // the words that initData sets, one allocation: `noneWords` of all ones
+  // (locks, marks, fixStarts), then zeroes (the others)
+  uint32_t *state = nullptr;
+  size_t noneWords = 0, stateWords = 0;
   uint64_t *locks = nullptr;
   uint32_t *marks = nullptr, *cnt = nullptr, *refitCnt = nullptr;
   uint32_t *pending[2] = {nullptr, nullptr}, *numPending = nullptr;
   uint32_t *fixStarts = nullptr;
+  uint64_t *refitSlots = nullptr;  // where two refit walks meet (all zero between launches)
+  size_t refitSlotWords = 0;
   uint32_t *skipped = nullptr;
   uint32_t *stats = nullptr;
   uint32_t *selCounts = nullptr;
@@ -1206,6 +1422,28 @@ struct Internal {
   uint32_t *recCount = nullptr;
   uint32_t recMax = 0;
 };
+
+// Lays the per-node and per-patch words of `state` out; `words` receives
+// their number (before the allocation the pointers mean nothing yet).
+void carveState(Internal *in, size_t &words) {
+  size_t off = 0;
+  auto take = [&](size_t n) {
+    uint32_t *p = in->state ? in->state + off : nullptr;
+    off += (n + 3) & ~(size_t)3;  // 16-byte steps
+    return p;
+  };
+  in->locks = reinterpret_cast<uint64_t *>(take(2 * (size_t)in->N));
+  in->marks = take(in->N);
+  in->fixStarts = take(3 * (size_t)in->K);
+  in->noneWords = off;
+  in->refitSlots = reinterpret_cast<uint64_t *>(take(2 * in->refitSlotWords));
+  in->cnt = take(in->N);
+  in->refitCnt = take(in->N);
+  in->skipped = take(in->K);
+  in->stats = take(ST_WORDS);
+  in->numPending = take(1);
+  words = off;
+}
 
 bool features(Internal *in, const bvht_CUDAMemoryBVHPointer *bvh) {
   if (!in->feat) {
@@ -1226,9 +1464,35 @@ bool features(Internal *in, const bvht_CUDAMemoryBVHPointer *bvh) {
                          in->feat);
 }
 
-// Refit arguments that keep the subtree features (when they are in use).
-uint32_t *refitLeafCnt(const Internal *in) { return in->subValid ? in->leafCnt : nullptr; }
-float *refitSubSA(const Internal *in) { return in->subValid ? in->subSA : nullptr; }
+// Refit from `num` device start nodes.  near: a list of leaves in their order
+// (no features kept); otherwise a chunk's scattered starts, 8 walks a wave
+// (1,881 starts in 1M triangles: 23.2, 25.0, 26.3, 29.2 us with 8, 16, 32, 64),
+// with the subtree features kept when they are in use.  A list longer than
+// the slots is done in pieces: a node above starts of two pieces is
+// recomputed by each, last with both its children final.
+bool refitFrom(Internal *in, const bvht_CUDAMemoryBVHPointer *bvh, const uint32_t *starts, uint32_t num, bool near) {
+  const bool feat = !near && in->subValid;
+  const uint32_t walks = near ? 64 : 8;
+  const uint32_t most = (uint32_t)std::min<size_t>(in->refitSlotWords / (feat ? 6 : 4), 1u << (32 - kRefitSlotShift));
+  for (uint32_t at = 0; at < num;) {
+    const uint32_t n = std::min(most, num - at), blocks = divUp(n, walks * (kRefitBlock / 64));
+    k_refitCount<<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N, in->cnt);
+    if (!checkLaunch("k_refitCount")) return false;
+    if (near)
+      k_refitApply<false, true><<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N, in->cnt,
+                                                                      in->refitSlots, nullptr, nullptr, in->stats);
+    else if (feat)
+      k_refitApply<true, false><<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N, in->cnt,
+                                                                      in->refitSlots, in->leafCnt, in->subSA, in->stats);
+    else
+      k_refitApply<false, false><<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N,
+                                                                       in->cnt, in->refitSlots, nullptr, nullptr,
+                                                                       in->stats);
+    if (!checkLaunch("k_refitApply")) return false;
+    at += n;
+  }
+  return true;
+}
 
 RecordSink sinkOf(const Internal *in) {
   RecordSink r{nullptr, in->recFeat, in->recGain, in->recCount, in->recMax};
@@ -1305,6 +1569,9 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
   in->numInner = bvh->numNodes - numFaces;
   in->K = batchSize;
   in->plan = makeSortPlan(in->numInner, 4, 32);
+  // a chunk's 3 starts per patch in one piece, and lists of up to a quarter of the leaves
+  in->refitSlotWords = std::max<size_t>(6 * 3 * (size_t)batchSize, 4 * (size_t)divUp(numFaces, 4));
+  carveState(in, in->stateWords);
   const uint32_t selBlocks = divUp(in->N, kSelTile);
   m.numLeafNodes = in->numLeaves;
   m.numInnerNodes = in->numInner;
@@ -1316,18 +1583,14 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
             devAlloc(&in->keys[0], in->numInner, "bn13 keys") && devAlloc(&in->keys[1], in->numInner, "bn13 keys") &&
             devAlloc(&in->vals[0], in->numInner, "bn13 vals") && devAlloc(&in->vals[1], in->numInner, "bn13 vals") &&
             devMalloc(reinterpret_cast<void **>(&in->sortScratch), sortScratchBytes(in->plan), "bn13 sort") &&
-            devAlloc(&in->recs, batchSize, "bn13 patches") && devAlloc(&in->locks, in->N, "bn13 locks") &&
+            devAlloc(&in->recs, batchSize, "bn13 patches") && devAlloc(&in->state, in->stateWords, "bn13 state") &&
             devAlloc(&in->pending[0], batchSize, "bn13 pending") && devAlloc(&in->pending[1], batchSize, "bn13 pending") &&
-            devAlloc(&in->numPending, 1, "bn13 pending count") &&
-            devAlloc(&in->marks, in->N, "bn13 marks") && devAlloc(&in->cnt, in->N, "bn13 refit counters") &&
-            devAlloc(&in->refitCnt, in->N, "bn13 refit counters") &&
-            devAlloc(&in->fixStarts, 3 * (size_t)batchSize, "bn13 fix starts") &&
-            devAlloc(&in->skipped, batchSize, "bn13 skipped") && devAlloc(&in->stats, ST_WORDS, "bn13 stats") &&
             devAlloc(&in->selCounts, selBlocks, "bn13 select") && devAlloc(&in->partials, kSahBlocks, "bn13 SAH");
   if (!ok) {
     freeMemory(&m);
     return m;
   }
+  carveState(in, in->stateWords);
   m.result = true;
   return m;
 }
@@ -1345,16 +1608,9 @@ void freeMemory(bvht_GPUWorkingMemory *data) {
     devFree(in->vals[1]);
     devFree(in->sortScratch);
     devFree(in->recs);
-    devFree(in->locks);
+    devFree(in->state);
     devFree(in->pending[0]);
     devFree(in->pending[1]);
-    devFree(in->numPending);
-    devFree(in->marks);
-    devFree(in->cnt);
-    devFree(in->refitCnt);
-    devFree(in->fixStarts);
-    devFree(in->skipped);
-    devFree(in->stats);
     devFree(in->selCounts);
     devFree(in->partials);
     devFree(in->feat);
@@ -1411,14 +1667,8 @@ void initData(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bvh, uint3
     return;
   k_selWrite<<<selBlocks, kSelBlock, 0, stream()>>>(bvh->nodes, in->N, in->selCounts, in->inner, in->leaves);
   if (!checkLaunch("k_selWrite")) return;
-  fillU32(reinterpret_cast<uint32_t *>(in->locks), NONE, 2ull * in->N);  // kLockFree
-  fillU32(in->numPending, 0u, 1);
-  fillU32(in->marks, NONE, in->N);
-  fillU32(in->cnt, 0u, in->N);
-  fillU32(in->refitCnt, 0u, in->N);
-  fillU32(in->skipped, 0u, in->K);
-  fillU32(in->stats, 0u, ST_WORDS);
-  fillU32(in->fixStarts, NONE, 3ull * in->K);
+  fillU32(in->state, NONE, in->noneWords);  // locks: kLockFree
+  fillU32(in->state + in->noneWords, 0u, in->stateWords - in->noneWords);
   check(hipMemsetAsync(in->recs, 0, sizeof(PatchRec) * in->K, stream()), "initData patches");
   check(hipStreamSynchronize(stream()), "initData sync");
 }
@@ -1435,12 +1685,7 @@ void fixTree3(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bvh, uint3
   (void)blockSize;
   Internal *in = inOf(data);
   if (!in || !validBVH(bvh, "fixTree3")) return;
-  const uint32_t num = 3 * in->K;
-  k_refitCount<<<divUp(num, 256), 256, 0, stream()>>>(in->fixStarts, num, bvh->nodes, in->N, in->cnt);
-  if (!checkLaunch("k_refitCount")) return;
-  k_refitApply<<<divUp(num, 256), 256, 0, stream()>>>(in->fixStarts, num, bvh->nodes, in->N, in->cnt,
-                                                    refitLeafCnt(in), refitSubSA(in));
-  checkLaunch("k_refitApply");
+  refitFrom(in, bvh, in->fixStarts, 3 * in->K, false);
 }
 
 void selectDynamicLeafNodes(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bvh, uint32_t *out,
@@ -1488,11 +1733,8 @@ bool bvht_fixTreeFrom(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bv
     setError("bvht_fixTreeFrom: no start nodes");
     return false;
   }
-  k_refitCount<<<divUp(num, 256), 256, 0, stream()>>>(devStarts, num, bvh->nodes, in->N, in->cnt);
-  if (!checkLaunch("k_refitCount")) return false;
   in->subValid = false;  // leaf boxes may have changed (dynamic refit)
-  k_refitApply<<<divUp(num, 256), 256, 0, stream()>>>(devStarts, num, bvh->nodes, in->N, in->cnt, nullptr, nullptr);
-  return checkLaunch("k_refitApply");
+  return refitFrom(in, bvh, devStarts, num, true);
 }
 
 void bn13_selectNodes(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bvh, bvht_AlgoCFG cfg) {
@@ -1597,12 +1839,7 @@ void bn13_rmAndReinsChunk(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer
   k_apply<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->locks, in->marks, in->fixStarts,
                                                in->numPending, in->stats);
   if (!checkLaunch("k_apply")) return;
-  const uint32_t num = 3 * K;
-  k_refitCount<<<divUp(num, 256), 256, 0, stream()>>>(in->fixStarts, num, bvh->nodes, in->N, in->cnt);
-  if (!checkLaunch("k_refitCount")) return;
-  k_refitApply<<<divUp(num, 256), 256, 0, stream()>>>(in->fixStarts, num, bvh->nodes, in->N, in->cnt,
-                                                    refitLeafCnt(in), refitSubSA(in));
-  checkLaunch("k_refitApply");
+  refitFrom(in, bvh, in->fixStarts, 3 * K, false);
 }
 
 void bn13_doAlgorithmStep(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bvh, bvht_AlgoCFG cfg) {

@@ -430,8 +430,9 @@ uint32_t calcNumSkipped(bvht_GPUWorkingMemory *data);
  * [0] lock conflicts, [1] patches dropped (removal impossible or reinsertion
  * at the root), [2] patches dropped because their insertion point lies in a
  * subtree another patch moves, [3] search frontier overflows, [4] applied
- * patches, [5] patches the conflict resolution left undecided (0 unless the
- * device breaks memory ordering; they are dropped), [6] searches stopped at
+ * patches, [5] patches the conflict resolution left undecided, which are
+ * dropped, and waits that a refit gave up (0 unless the device breaks memory
+ * ordering), [6] searches stopped at
  * the step bound (0 for a tree; the patch is dropped), [7] steps whose
  * priority sort gave up a bounded wait (0 unless the device breaks memory
  * ordering; that step's order is then wrong).  Returns the number of words

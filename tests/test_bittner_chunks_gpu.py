@@ -1,4 +1,7 @@
 """Chunk kernels of the optimizer at the sizes where their paths change."""
+import ctypes
+
+import numpy as np
 import pytest
 
 from test_bittner_gpu import replay_check
@@ -13,3 +16,41 @@ def test_conflict_rounds_equal_replay(bvh, orc, percent):
     v, f = bvh.scene_heightfield(48, 40, 51, 0.2)
     print(f"K={int(percent / 100 * (2 * len(f) - 1))}", flush=True)
     replay_check(bvh, orc, v, f, 2, 1, percent, search=1)
+
+
+# Refits from lists of leaves: one walk, a workgroup's edge (256), more than the
+# meeting places of one launch (a quarter of the leaves), all leaves, all of
+# them twice over and some inner nodes among them.
+@pytest.mark.parametrize("count", [1, 2, 63, 255, 256, 257, 2000, 2001, "all", "twice"])
+def test_refit_from_leaf_lists(bvh, orc, count):
+    v, f = bvh.scene_spheres_soup(8, 4000, 61)
+    mesh = bvh.DeviceMesh(v, f)
+    tree = bvh.lbvh_build(mesh)
+    opt = bvh.Bittner13GPU(maxNumStepps=1, numChunks=4, batchPercent=0.5)
+    opt.run(tree, len(f))
+    nodes = tree.download()
+    rng = np.random.default_rng(5)
+    leaves = np.nonzero(nodes["isLeafFlag"] != 0)[0].astype(np.uint32)
+    inner = np.nonzero(nodes["isLeafFlag"] == 0)[0].astype(np.uint32)
+    moved = leaves if count in ("all", "twice") else np.sort(rng.choice(leaves, count, replace=False))
+    starts = moved
+    if count == "twice":
+        starts = rng.permutation(np.concatenate([moved, moved, rng.choice(inner, 500)]))
+    print(f"{len(starts)} starts over {len(leaves)} leaves", flush=True)
+    v2 = v + rng.uniform(-0.05, 0.05, v.shape).astype(np.float32)
+    L = bvh.lib()
+    mem, raw = opt.mem, mesh.raw
+    d_moved = bvh.DeviceBuffer(moved.nbytes).upload(moved)
+    d_starts = bvh.DeviceBuffer(starts.nbytes).upload(starts)
+    assert L.runMemcpy(raw.vert, v2.ctypes.data_as(ctypes.c_void_p), v2.nbytes, 1)
+    L.refitDynamicTris(ctypes.byref(tree.ptr), raw, d_moved.ptr, len(moved), 64)
+    assert L.bvht_fixTreeFrom(ctypes.byref(mem), ctypes.byref(tree.ptr), d_starts.ptr, len(starts))
+    L.doCudaDevSync()
+    assert bvh.last_error() == ""
+    want = orc.fix_tree1(orc.refit_leaf_tris(nodes, v2, f, moved))
+    assert tree.download().tobytes() == want.tobytes()
+    assert opt.stats()["unresolved"] == 0
+    # the words are clear again: the next refit from one leaf changes nothing
+    assert L.bvht_fixTreeFrom(ctypes.byref(mem), ctypes.byref(tree.ptr), d_starts.ptr, 1)
+    L.doCudaDevSync()
+    assert tree.download().tobytes() == want.tobytes()
