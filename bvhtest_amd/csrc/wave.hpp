@@ -146,6 +146,22 @@ __device__ __forceinline__ uint32_t blockExclusiveScan(uint32_t v, uint32_t *s_t
   return prefix + inc - v;
 }
 
+// Minimum over the wave of a value without NaN, the same in every lane (all
+// 64 active).  Data moves between lanes inside the vector ALU (DPP): one
+// instruction per step and no LDS round trip.  Lanes without a source keep
+// their value; each step waits the two states that DPP needs after a write.
+__device__ __forceinline__ float waveMinUniform(float x) {
+  asm volatile("s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"  // lane 15 of a row: the row's
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+      "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"  // lane 63: every row's
+      "s_nop 1"
+      : "+v"(x));
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+
 __device__ __forceinline__ float waveMin(float x) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
