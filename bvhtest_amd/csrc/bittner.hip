@@ -1507,7 +1507,8 @@ bool features(Internal *in, const bvht_CUDAMemoryBVHPointer *bvh) {
       return false;
   }
   if (!in->subValid) {
-    if (!computeSubtree(bvh->nodes, in->N, in->leaves, in->numLeaves, in->leafCnt, in->subSA, in->refitCnt))
+    if (!computeSubtree(bvh->nodes, in->N, in->leaves, in->numLeaves, in->leafCnt, in->subSA, in->refitCnt, in->anc[0],
+                        in->anc[1]))
       return false;
     in->subValid = true;
   }

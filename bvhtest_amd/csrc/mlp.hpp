@@ -39,9 +39,10 @@ struct PriorityModel {
 };
 
 // Leaf count and subtree surface-area sum of every node (bottom-up from the
-// leaves; `arrive` holds N zeros on entry and on exit).
+// leaves; `arrive` holds N zeros on entry and on exit; list[numLeaves] and
+// listCount are scratch).
 bool computeSubtree(const bvht_BVHNode *nodes, uint32_t N, const uint32_t *leaves, uint32_t numLeaves,
-                    uint32_t *leafCnt, float *subSA, uint32_t *arrive);
+                    uint32_t *leafCnt, float *subSA, uint32_t *arrive, uint32_t *list, uint32_t *listCount);
 // Depth of every node, exact below 2^kDepthRounds (larger depths come out
 // as at least that), by pointer jumping over double buffers anc[2][N],
 // dep[2][N]; returns the buffer index holding the result (-1 on error).
