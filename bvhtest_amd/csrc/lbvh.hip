@@ -18,6 +18,7 @@
 // read to build it and no global atomic is needed for the refit.
 #include "lbvh.hpp"
 #include "lbvh_kernels.hpp"
+#include "lbvh_small.hpp"
 #include "msd_sort.hpp"
 #include "radix_sort.hpp"
 #include "split_sort.hpp"
@@ -163,13 +164,6 @@ __global__ __launch_bounds__(kBoxBlock) void k_sceneBox(const bvht_vec3 *__restr
 // Neither pass ends in a last-block reduction (one global atomic per block
 // on one counter, then a serial tail): each block writes its partial box,
 // and every block of the next kernel reduces all partials itself.
-__device__ __forceinline__ void shiftedBox(float mn[3], float mx[3]) {
-  for (int a = 0; a < 3; ++a) {  // -+FLT_EPSILON, then the origin (LBVH_CUDA.cu:104-106)
-    mn[a] = mergeMin(0.0f, mn[a] - kFltEpsilon);
-    mx[a] = mergeMax(0.0f, mx[a] + kFltEpsilon);
-  }
-}
-
 // Block reduction of per-thread boxes; thread 0 writes partials[blockIdx.x].
 __device__ void writeBoxPartial(const float mn[3], const float mx[3], float *__restrict__ partials) {
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -216,12 +210,6 @@ __device__ void readBoxPartials(const float *__restrict__ partials, uint32_t cou
   }
   __syncthreads();
   for (int a = 0; a < 6; ++a) box[a] = s_box[a];
-}
-
-// LBVH_calcMortonCodes host part (LBVH_CUDA.cu:171-180), f32, IEEE division.
-__device__ __forceinline__ void mortonMapping(const float box[6], bvht_vec3 &off, bvht_vec3 &sc) {
-  off = {0.0f - box[0], 0.0f - box[1], 0.0f - box[2]};
-  sc = {__fdiv_rn(1.0f, box[3] + off.x), __fdiv_rn(1.0f, box[4] + off.y), __fdiv_rn(1.0f, box[5] + off.z)};
 }
 
 // Box of all vertices.  The vertex array is read as 16-byte words (float4
@@ -747,6 +735,15 @@ bool buildAll(bvht_LBVH_WorkingMemory *mem, const bvht_MeshRaw *mesh, bvht_CUDAM
   Timing &tm = timing();
   tm.start();
   tm.record("begin");
+  if (!in->useMsd && mesh->numFaces <= kSmallSortMax) {
+    void *keys = mem->opts.topology == 1 ? mem->keys[0] : nullptr;
+    if (!smallSort(*mesh, (int)mem->opts.mortonBits, (BuildParams *)mem->params, keys, mem->values[0])) return false;
+    tm.record("k_smallSort");
+    in->resultBuf = 0;
+    mem->sortedValues = mem->values[0];
+    mem->sortedKeys = keys;
+    return runTree(mem, mesh, bvh);
+  }
   // the vertex box (one streaming pass) when the keys come from k_morton,
   // which checks it; the MSD key pass takes the triangles' box
   const bool vertexBox = !in->useMsd;

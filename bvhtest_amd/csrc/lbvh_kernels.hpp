@@ -17,6 +17,20 @@ struct SegDesc {
   uint32_t vertBase;  // first vertex of the mesh
 };
 
+// The box of min / max over vertices as the reference reduces triangle boxes.
+__device__ __forceinline__ void shiftedBox(float mn[3], float mx[3]) {
+  for (int a = 0; a < 3; ++a) {  // -+FLT_EPSILON, then the origin (LBVH_CUDA.cu:104-106)
+    mn[a] = mergeMin(0.0f, mn[a] - kFltEpsilon);
+    mx[a] = mergeMax(0.0f, mx[a] + kFltEpsilon);
+  }
+}
+
+// LBVH_calcMortonCodes host part (LBVH_CUDA.cu:171-180), f32, IEEE division.
+__device__ __forceinline__ void mortonMapping(const float box[6], bvht_vec3 &off, bvht_vec3 &sc) {
+  off = {0.0f - box[0], 0.0f - box[1], 0.0f - box[2]};
+  sc = {__fdiv_rn(1.0f, box[3] + off.x), __fdiv_rn(1.0f, box[4] + off.y), __fdiv_rn(1.0f, box[5] + off.z)};
+}
+
 // The three 16-byte words of a 48-byte node.
 struct NodeWords {
   uint4 w[3];
