@@ -13,7 +13,6 @@ constexpr uint32_t kCountMask = (1u << 30) - 1;
 // bit 15 and bit 31 set when published.
 constexpr uint32_t kHalfFlags = 0x80008000u, kHalfCount = 0x7FFFu;
 constexpr uint32_t kWideStatusWords = kSortRadix / 2;  // per tile
-static_assert(kWideTile <= kHalfCount, "a tile's count of one digit fits 15 bits");
 constexpr uint32_t kLookWindow = 8;  // look-back statuses loaded per round trip
 
 // Histogram of all passes: LDS counters per block, then one global atomic
@@ -211,10 +210,11 @@ __global__ __launch_bounds__(kSortBlock, 3) void k_onesweep(const K *__restrict_
     if (out[k] < n) valsOut[out[k]] = s_v[tid + k * kSortBlock];
 }
 
-// Wide tiles: workgroups of 1024 threads x 17 keys (17,408 keys per tile),
-// used when the tiles of a pass fit the CUs in one round (244 tiles at 4.24M
-// keys: a dispatch ramp of 244 workgroups instead of 753).  Ranking and
-// scatter are those of k_onesweep (16 waves, 256 digit owners).
+// Wide tiles: workgroups of BLOCK threads x ITEMS keys, used when the tiles of
+// a pass fit the CUs in one round (1024 x 17 keys: 244 tiles at 4.24M keys, a
+// dispatch ramp of 244 workgroups instead of 753; smaller ones below that, so
+// that the tiles still spread over the chip: see makeSortPlan).  Ranking and
+// scatter are those of k_onesweep (a wave per 64 threads, 256 digit owners).
 //  - Global accesses are buffer loads and stores with 32-bit byte offsets
 //    (the wide path only runs below 2^23 keys): one address register per
 //    access instead of a 64-bit pointer per item, which keeps the kernel
@@ -226,37 +226,37 @@ __global__ __launch_bounds__(kSortBlock, 3) void k_onesweep(const K *__restrict_
 //    first pass: values are the input index, made when they are staged) or
 //    kValsNone (a keys-only sort).
 //  - The tile's global offsets are the sums of every earlier tile's
-//    published per-digit counts, loaded by all 1024 threads at once instead
+//    published per-digit counts, loaded by all threads at once instead
 //    of a chained look-back.  The counts are published two digits to a word
 //    (15 bits each), so a 16-byte load brings eight digits and, with 8 loads
-//    in flight per thread, one round trip covers 256 predecessors.
-//    Tile ids come from `counter`, so every tile a workgroup waits for has
-//    started; the wait for a count is bounded and raises the error flag.
+//    in flight per thread, one round trip covers 64 to 256 predecessors.
+//  - The tile is the workgroup's id.  Workgroups start in id order on each
+//    XCD and a CU holds one of any tile size, so the lowest tile that has not
+//    started yet only waits for tiles that have, and they do not wait for it;
+//    the wait for a count is bounded all the same and raises the error flag.
+//    (Tile ids from an atomic counter: 1.5 to 3.4 us at the start of a pass.)
 enum { kValsLoaded = 0, kValsIdentity = 1, kValsNone = 2 };
-template <typename K, int VALS>
-__global__ __launch_bounds__(kWideBlock, 1) void k_onesweepWide(const K *__restrict__ keysIn,
-                                                             const uint32_t *__restrict__ valsIn,
-                                                             K *__restrict__ keysOut, uint32_t *__restrict__ valsOut,
-                                                             uint32_t n, uint32_t shift,
-                                                             const uint32_t *__restrict__ hist,
-                                                             uint32_t *status,
-                                                             uint32_t *counter, uint32_t *err) {
-  constexpr int WAVES = kWideBlock / 64;
-  constexpr int ITEMS = kWideItems;
-  constexpr uint32_t TILE = kWideTile;
+template <typename K, int VALS, int BLOCK, int ITEMS>
+__global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__ keysIn,
+                                                           const uint32_t *__restrict__ valsIn,
+                                                           K *__restrict__ keysOut, uint32_t *__restrict__ valsOut,
+                                                           uint32_t n, uint32_t shift,
+                                                           const uint32_t *__restrict__ hist, uint32_t *status,
+                                                           uint32_t *err) {
+  constexpr int WAVES = BLOCK / 64;
+  constexpr uint32_t TILE = BLOCK * ITEMS;
+  static_assert(BLOCK >= kSortRadix && TILE <= kHalfCount, "a thread per digit; a tile's count of one digit fits 15 bits");
   constexpr bool WIDE = sizeof(K) == 8;
   __shared__ uint32_t s_wave[WAVES][kSortRadix];  // per-wave digit counters, then prefix partials
   __shared__ uint32_t s_bstart[kSortRadix];
   __shared__ uint32_t s_gstart[kSortRadix];
   __shared__ uint32_t s_scan[WAVES];
-  __shared__ uint32_t s_tile;
   __shared__ K s_buf[TILE];  // the staged keys, then the values in the same words
 
   const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  if (tid == 0) s_tile = atomicAdd(counter, 1u);
-  for (uint32_t i = tid; i < (uint32_t)WAVES * kSortRadix; i += kWideBlock) (&s_wave[0][0])[i] = 0;
+  for (uint32_t i = tid; i < (uint32_t)WAVES * kSortRadix; i += BLOCK) (&s_wave[0][0])[i] = 0;
   __syncthreads();
-  const uint32_t tile = s_tile;
+  const uint32_t tile = blockIdx.x;
   const uint32_t first = tile * TILE + wave * 64 * ITEMS + lane;  // item i is key first + 64 i
   const uint32_t histDigit = tid < kSortRadix ? hist[tid] : 0u;  // issued now, used after the ranking
 
@@ -300,14 +300,14 @@ __global__ __launch_bounds__(kWideBlock, 1) void k_onesweepWide(const K *__restr
       s_wave[w][tid] = total;
       total += c;
     }
-    // two digits per word: 15-bit counts (a tile holds at most kWideTile
-    // keys), each half flagged when published
+    // two digits per word: 15-bit counts (at most 17,408
+    // keys in a tile), each half flagged when published
     const uint32_t odd = __shfl_xor(total, 1, 64);  // waves 0..3, all lanes
     if ((tid & 1u) == 0)
       storeRelaxedAgent(status + (size_t)tile * kWideStatusWords + tid / 2, kHalfFlags | total | (odd << 16));
   }
-  const uint32_t hbase = blockExclusiveScan<kWideBlock>(histDigit, s_scan);
-  const uint32_t bstart = blockExclusiveScan<kWideBlock>(total, s_scan);
+  const uint32_t hbase = blockExclusiveScan<BLOCK>(histDigit, s_scan);
+  const uint32_t bstart = blockExclusiveScan<BLOCK>(total, s_scan);
   if (tid < kSortRadix) s_bstart[tid] = bstart;
   __syncthreads();
 
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(kWideBlock, 1) void k_onesweepWide(const K *__restr
   // loads, 8 in flight (one round trip for up to 256 predecessors); the 32
   // partial sums of a digit are then added in two steps.
   {
-    constexpr uint32_t OCTS = kSortRadix / 8, QG = kWideBlock / OCTS, QB = 8;
+    constexpr uint32_t OCTS = kSortRadix / 8, QG = BLOCK / OCTS, QB = 8;
     static_assert(QG == 2 * WAVES, "two look-back groups per row of s_wave");
     const uint32_t q = tid % OCTS, g = tid / OCTS;
     const BufferRsrc st = bufferRsrc(status, tile * kWideStatusWords * 4u);  // the earlier tiles' words
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(kWideBlock, 1) void k_onesweepWide(const K *__restr
   uint32_t out[ITEMS];
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
-    const uint32_t j = tid + k * kWideBlock;
+    const uint32_t j = tid + k * BLOCK;
     out[k] = n;
     if (j < tileCount) {
       const K kk = s_buf[j];
@@ -430,7 +430,39 @@ __global__ __launch_bounds__(kWideBlock, 1) void k_onesweepWide(const K *__restr
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k)
-    if (out[k] < n) bufferStore(s_v[tid + k * kWideBlock], vout, out[k] * 4u);
+    if (out[k] < n) bufferStore(s_v[tid + k * BLOCK], vout, out[k] * 4u);
+}
+
+// Keys per tile of the wide sizes: BLOCK x ITEMS of launchWide's cases.
+constexpr int kWideSizes = 7;
+constexpr uint32_t kWideTiles[kWideSizes + 1] = {0, 256 * 2, 256 * 4, 512 * 4, 1024 * 4, 1024 * 8, 1024 * 12, kWideTile};
+
+struct WidePass {
+  const void *keysIn;
+  const uint32_t *valsIn;
+  void *keysOut;
+  uint32_t *valsOut;
+  uint32_t n, shift;
+  const uint32_t *hist;
+  uint32_t *status, *err;
+};
+template <typename K, int VALS, int BLOCK, int ITEMS>
+void launchWideSize(const SortPlan &p, const WidePass &w) {
+  k_onesweepWide<K, VALS, BLOCK, ITEMS><<<p.numTiles, BLOCK, 0, stream()>>>(
+      static_cast<const K *>(w.keysIn), w.valsIn, static_cast<K *>(w.keysOut), w.valsOut, w.n, w.shift, w.hist,
+      w.status, w.err);
+}
+template <typename K, int VALS>
+void launchWide(const SortPlan &p, const WidePass &w) {
+  switch (p.wide) {
+    case 1: launchWideSize<K, VALS, 256, 2>(p, w); break;
+    case 2: launchWideSize<K, VALS, 256, 4>(p, w); break;
+    case 3: launchWideSize<K, VALS, 512, 4>(p, w); break;
+    case 4: launchWideSize<K, VALS, 1024, 4>(p, w); break;
+    case 5: launchWideSize<K, VALS, 1024, 8>(p, w); break;
+    case 6: launchWideSize<K, VALS, 1024, 12>(p, w); break;
+    default: launchWideSize<K, VALS, kWideBlock, kWideItems>(p, w); break;
+  }
 }
 
 }  // namespace
@@ -441,15 +473,24 @@ SortPlan makeSortPlan(uint32_t n, int keyBytes, int keyBits) {
   p.keyBytes = keyBytes;
   p.keyBits = keyBits;
   p.passes = (keyBits + kSortRadixBits - 1) / kSortRadixBits;
-  // wide tiles when they fit the CUs in one round of workgroups (their
-  // 32-bit byte offsets need n * 8 < 2^31: true for any device below 30,000 CUs)
-  const uint32_t wideTiles = n == 0 ? 0 : divUp(n, kWideTile);
-  p.wide = n > 0 && wideTiles <= (uint32_t)numCUs() && (uint64_t)n * 8 < (1ull << 31);
-  p.tile = p.wide ? kWideTile : kSortBlock * (keyBytes == 8 ? kSortItems64 : kSortItems32);
+  // Wide tiles when they fit the CUs in one round of workgroups (their
+  // 32-bit byte offsets need n * 8 < 2^31: true for any device below 30,000
+  // CUs).  A pass takes as long as one tile, so the smallest tile that does is
+  // taken; of the smallest two, which read the counts of 64 predecessors per
+  // round trip, only half as many.  Whole builds with 30-bit keys, this tile
+  // against the largest one for every size: 65,536 triangles (1,024 keys per
+  // tile) 62 against 97 us, 199,220 (2,048) 69 against 105 (1,024: 75),
+  // 909,000 (4,096) 101 against 132 (8,192: 110), 1.88M (8,192) 146 against
+  // 168, 2.79M (12,288) 191 against 203.
+  p.wide = 0;
+  if (n > 0 && (uint64_t)n * 8 < (1ull << 31))
+    for (int w = 1; w <= kWideSizes && !p.wide; ++w)
+      if (divUp(n, kWideTiles[w]) <= (uint32_t)numCUs() / (w < 3 ? 2 : 1)) p.wide = w;
+  p.tile = p.wide ? kWideTiles[p.wide] : kSortBlock * (keyBytes == 8 ? kSortItems64 : kSortItems32);
   p.numTiles = n == 0 ? 0 : divUp(n, p.tile);
   p.histWords = (size_t)p.passes * kSortRadix;
   p.counterWords = 16;  // a tile counter per pass (at most 8), then the error word
-  p.statusWords = (size_t)p.passes * p.numTiles * kSortRadix;
+  p.statusWords = (size_t)p.passes * p.numTiles * (p.wide ? kWideStatusWords : (uint32_t)kSortRadix);
   p.histOff = 0;
   p.counterOff = p.histOff + p.histWords;
   p.statusOff = p.counterOff + p.counterWords;
@@ -488,26 +529,22 @@ int sortRun(const SortPlan &p, void *keys[2], uint32_t *vals[2], bool identityVa
     const uint32_t *hist = scratch + p.histOff + (size_t)pass * kSortRadix;
     uint32_t *counter = scratch + p.counterOff + pass;
     uint32_t *err = scratch + p.errOff;  // one word for every pass
-    uint32_t *status = scratch + p.statusOff + (size_t)pass * p.numTiles * kSortRadix;
+    uint32_t *status = scratch + p.statusOff + pass * (p.statusWords / p.passes);
     const uint32_t *vin = (keysOnly || (pass == firstPass && identityValues)) ? nullptr : vals[cur];
     bool last = pass == p.passes - 1;
     void *kout = (last && !keepKeys) ? nullptr : keys[cur ^ 1];
     uint32_t shift = pass * kSortRadixBits;
+    const WidePass w = {keys[cur], vin, kout, keysOnly ? nullptr : vals[cur ^ 1], p.n, shift, hist, status, err};
     if (keysOnly)
-      k_onesweepWide<uint64_t, kValsNone><<<p.numTiles, kWideBlock, 0, stream()>>>(
-          (const uint64_t *)keys[cur], nullptr, (uint64_t *)kout, nullptr, p.n, shift, hist, status, counter, err);
+      launchWide<uint64_t, kValsNone>(p, w);
     else if (p.wide && p.keyBytes == 8 && !vin)
-      k_onesweepWide<uint64_t, kValsIdentity><<<p.numTiles, kWideBlock, 0, stream()>>>(
-          (const uint64_t *)keys[cur], vin, (uint64_t *)kout, vals[cur ^ 1], p.n, shift, hist, status, counter, err);
+      launchWide<uint64_t, kValsIdentity>(p, w);
     else if (p.wide && p.keyBytes == 8)
-      k_onesweepWide<uint64_t, kValsLoaded><<<p.numTiles, kWideBlock, 0, stream()>>>(
-          (const uint64_t *)keys[cur], vin, (uint64_t *)kout, vals[cur ^ 1], p.n, shift, hist, status, counter, err);
+      launchWide<uint64_t, kValsLoaded>(p, w);
     else if (p.wide && !vin)
-      k_onesweepWide<uint32_t, kValsIdentity><<<p.numTiles, kWideBlock, 0, stream()>>>(
-          (const uint32_t *)keys[cur], vin, (uint32_t *)kout, vals[cur ^ 1], p.n, shift, hist, status, counter, err);
+      launchWide<uint32_t, kValsIdentity>(p, w);
     else if (p.wide)
-      k_onesweepWide<uint32_t, kValsLoaded><<<p.numTiles, kWideBlock, 0, stream()>>>(
-          (const uint32_t *)keys[cur], vin, (uint32_t *)kout, vals[cur ^ 1], p.n, shift, hist, status, counter, err);
+      launchWide<uint32_t, kValsLoaded>(p, w);
     else if (p.keyBytes == 8)
       k_onesweep<uint64_t, kSortItems64><<<p.numTiles, kSortBlock, 0, stream()>>>(
           (const uint64_t *)keys[cur], vin, (uint64_t *)kout, vals[cur ^ 1], p.n, shift, hist, status, counter, err);

@@ -20,7 +20,7 @@ constexpr int kSortRadix = 1 << kSortRadixBits;
 constexpr int kSortBlock = 256;
 constexpr int kSortItems32 = 20;  // keys per thread, 32-bit keys
 constexpr int kSortItems64 = 22;  // keys per thread, 64-bit keys: 753 tiles at 4.24M keys, one wave of workgroups
-// Wide tiles (k_onesweepWide): 1024 threads x 17 keys, 244 tiles at 4.24M keys.
+// Largest wide tiles (k_onesweepWide): 1024 threads x 17 keys, 244 tiles at 4.24M keys.
 constexpr int kWideBlock = 1024;
 constexpr int kWideItems = 17;
 constexpr uint32_t kWideTile = kWideBlock * kWideItems;
@@ -32,7 +32,7 @@ struct SortPlan {
   int passes = 0;
   uint32_t tile = 0;
   uint32_t numTiles = 0;
-  bool wide = false;  // k_onesweepWide (tiles of kWideTile keys)
+  int wide = 0;  // k_onesweepWide's tile size (1 smallest .. 7: kWideTile keys), 0: k_onesweep
   // u32 word offsets into the scratch buffer
   size_t histWords = 0, counterWords = 0, statusWords = 0;
   size_t histOff = 0, counterOff = 0, statusOff = 0, totalWords = 0;
