@@ -4,21 +4,31 @@
 // Traversal visits nodes in the reference's order (Afra & Szirmay-Kalos
 // 2014, the bit-trail algorithm of kTraceRay): at an inner node both children
 // are tested against the current nearest hit, the nearer hit child is entered
-// first and the other is remembered by a set trail bit; a remembered child is
-// entered later without a second box test.  Two changes make it fast without
-// changing that order:
-//   * each inner node's two child boxes, ids and leaf triangles are packed
-//     into one 64-byte record (k_packPairs), each triangle into (v0, e1, e2)
-//     (k_packTris, the same f32 subtractions the test makes), so a visit is
-//     one 64-byte load instead of three 48-byte node loads;
-//   * the remembered children are cached in a 16-entry per-lane LDS stack, so
-//     backtracking pops instead of walking parent links.  The trail stays the
-//     authority: when the cache has dropped an entry (deeper than 16 pending
-//     children), the walk falls back to the parent links.
+// first and the other one later, without a second box test.  What makes it
+// fast without changing that order:
+//   * every node becomes one 64-byte record (k_packNodes): an inner node holds
+//     its two children's boxes and references, a leaf its triangle as
+//     (v0, e1, e2) (the same f32 subtractions the test makes), in leaf order,
+//     so a visit is one record whichever kind it is;
+//   * a reference is one word (node id, top bit: leaf), and the children still
+//     to be entered are kept in a 24-entry per-lane LDS stack of them.  A ray
+//     that needs a 25th starts over with the reference's 128-bit trail and its
+//     parent links (slowWalk), so the common walk carries neither;
+//   * the walk is bound by vector issue and by the L1's accesses (74% and 65
+//     to 83% busy on primary rays at 1080p over 4.2M triangles), so a step
+//     visits an inner node and, if that leads to one, the leaf: a ray's last
+//     box test and its triangle test take one step of the wave.  A lane's own
+//     sequence of visits does not change.
+// Measured against separate pair and triangle records, a 16-entry ring and a
+// trail in every walk, one visit a step (1080p, 4.2M triangles; 512x512, 65k):
+// primary rays 3.65 -> 3.27 ms and 278 -> 240 us, secondary rays 4.05 -> 4.00 ms
+// and 681 -> 600 us.  Either kind in a step: 3.67 ms; the kind that more lanes
+// wait for: 3.87 ms.  16, 20, 24, 32, 48 entries: 4.26 (rays that start over),
+// 3.31, 3.27, 3.52, 4.10 ms (the LDS limits the waves).
 // Arithmetic is f32 with no FMA contraction and IEEE division, so the visit
 // order, hit triangle and distance are a pure function of the inputs (the
-// oracle reproduces them exactly).  The 128-bit trail limits trees to depth
-// 128, as in the reference.
+// oracle reproduces them exactly).  The 128-bit mask limits trees to depth
+// 128, as the reference's trail does.
 //
 // Rays are generated in f64 from a camera basis computed in f64 on the host
 // (the exact inverse of lookAtRH), then rounded once to f32.
@@ -90,234 +100,296 @@ struct TraceOut {
   uint16_t intCount;
 };
 
-// One inner node's children: boxes (min.xyz, max.xyz each), node ids and
-// leaf info (kInnerChild, the first face of a one-triangle leaf, or
-// kLookupLeaf for a leaf holding several triangles).
-struct PackedPair {
-  float4 a;  // l.min.x l.min.y l.min.z l.max.x
-  float4 b;  // l.max.y l.max.z r.min.x r.min.y
-  float4 c;  // r.min.z r.max.x r.max.y r.max.z
-  uint4 d;   // l r lInfo rInfo
+// One node, 64 bytes.  Inner: a b c hold the left child's box, then the
+// right's (min.xyz max.xyz each), d.x and d.y the children's references.
+// Leaf: a = v0 and the first face, b = e1 = v1 - v0 and the face count,
+// c = e2 = v2 - v0 (of that face).
+struct NodeRec {
+  float4 a, b, c;
+  uint4 d;
 };
-struct PackedTri {
-  float4 v0, e1, e2;  // e1 = v1 - v0, e2 = v2 - v0 (w unused)
-};
-constexpr uint32_t kInnerChild = 0xFFFFFFFFu, kLookupLeaf = 0xFFFFFFFEu, kEmptyLeaf = 0xFFFFFFFDu;
-constexpr int kStackCap = 16;  // cached remembered children per lane (power of two)
-constexpr uint32_t kTraceWavesPerCU = 20;  // 160 KiB of LDS / 8 KiB of stack cache per wave
-constexpr uint32_t kRefillAt = 16;         // idle lanes that make a k_traceRaysDyn wave fetch rays
+static_assert(sizeof(NodeRec) == 64, "one record per visit");
+constexpr uint32_t kLeafRef = 0x80000000u;  // the other bits: node id
+constexpr int kStackCap = 24;  // pending children per lane: 6 KiB of LDS a wave, 26 waves on a CU
+// k_traceRaysDyn waves on a CU.  16, 20, 24, 26: 4.11, 3.99, 4.14, 4.13 ms at
+// 1080p over 4.2M triangles, 685, 600, 608, 602 us at 512x512 over 65k (beyond
+// 20 the waves displace each other's records from the L1).
+constexpr uint32_t kTraceWavesPerCU = 20;
+constexpr uint32_t kRefillAt = 16;  // idle lanes that make a k_traceRaysDyn wave fetch rays
 
-__device__ __forceinline__ uint32_t leafInfo(const bvht_BVHNode &n) {
-  if (n.isLeafFlag == 0) return kInnerChild;
-  return n.right == 1 ? n.left : kLookupLeaf;
-}
-
-// Packs every inner node below `bound`; a child index at or past `bound`
-// becomes an empty leaf and raises *bad (the traversal then never reads past
-// the arrays).
-__global__ __launch_bounds__(256) void k_packPairs(const bvht_BVHNode *__restrict__ nodes, uint32_t bound,
-                                                   PackedPair *__restrict__ pairs, uint32_t *__restrict__ bad) {
+// Packs every node below `bound`; a child index at or past `bound` becomes
+// an empty leaf (a reference past the records) and raises *bad (the traversal
+// then never reads past the arrays).
+__global__ __launch_bounds__(256) void k_packNodes(const bvht_BVHNode *__restrict__ nodes, uint32_t bound,
+                                                   const bvht_Triangle *__restrict__ faces,
+                                                   const bvht_vec3 *__restrict__ vert, uint32_t numFaces,
+                                                   NodeRec *__restrict__ recs, uint32_t *__restrict__ bad) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i >= bound) return;
-  const bvht_BVHNode n = nodes[i];
-  if (n.isLeafFlag != 0) return;
-  uint32_t l = n.left, r = n.right, li = kEmptyLeaf, ri = kEmptyLeaf;
-  bvht_AABB lb = {{{0.f, 0.f, 0.f}, {-1.f, -1.f, -1.f}}}, rb = lb;
-  if (l < bound) {
-    const bvht_BVHNode c = nodes[l];
-    lb = c.bbox;
-    li = leafInfo(c);
+  const uint4 *w = reinterpret_cast<const uint4 *>(nodes + i);
+  const uint32_t left = w[1].w;
+  const uint2 rf = *reinterpret_cast<const uint2 *>(w + 2);  // right, flags
+  NodeRec p;
+  p.d = make_uint4(0, 0, 0, 0);
+  if ((rf.y & 0xFFFFu) != 0) {
+    bvht_vec3 v0 = {0.f, 0.f, 0.f}, e1 = v0, e2 = v0;
+    if (left < numFaces) {
+      const bvht_Triangle t = faces[left];
+      v0 = vert[t.v1];
+      e1 = vsub(vert[t.v2], v0);
+      e2 = vsub(vert[t.v3], v0);
+    }
+    p.a = make_float4(v0.x, v0.y, v0.z, __uint_as_float(left));
+    p.b = make_float4(e1.x, e1.y, e1.z, __uint_as_float(rf.x));
+    p.c = make_float4(e2.x, e2.y, e2.z, 0.f);
   } else {
-    *bad = 1;
-    l = i;
+    uint32_t child[2] = {left, rf.x};
+    bvht_AABB box[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (child[k] < bound) {
+        box[k] = nodes[child[k]].bbox;
+        if (nodes[child[k]].isLeafFlag != 0) child[k] |= kLeafRef;
+      } else {
+        *bad = 1;
+        box[k] = {{{0.f, 0.f, 0.f}, {-1.f, -1.f, -1.f}}};
+        child[k] = 0xFFFFFFFFu;
+      }
+    }
+    p.a = make_float4(box[0].minMax[0].x, box[0].minMax[0].y, box[0].minMax[0].z, box[0].minMax[1].x);
+    p.b = make_float4(box[0].minMax[1].y, box[0].minMax[1].z, box[1].minMax[0].x, box[1].minMax[0].y);
+    p.c = make_float4(box[1].minMax[0].z, box[1].minMax[1].x, box[1].minMax[1].y, box[1].minMax[1].z);
+    p.d.x = child[0];
+    p.d.y = child[1];
   }
-  if (r < bound) {
-    const bvht_BVHNode c = nodes[r];
-    rb = c.bbox;
-    ri = leafInfo(c);
-  } else {
-    *bad = 1;
-    r = i;
-  }
-  PackedPair p;
-  p.a = make_float4(lb.minMax[0].x, lb.minMax[0].y, lb.minMax[0].z, lb.minMax[1].x);
-  p.b = make_float4(lb.minMax[1].y, lb.minMax[1].z, rb.minMax[0].x, rb.minMax[0].y);
-  p.c = make_float4(rb.minMax[0].z, rb.minMax[1].x, rb.minMax[1].y, rb.minMax[1].z);
-  p.d = make_uint4(l, r, li, ri);
-  pairs[i] = p;
+  recs[i] = p;
 }
 
-__global__ __launch_bounds__(256) void k_packTris(const bvht_Triangle *__restrict__ faces,
-                                                  const bvht_vec3 *__restrict__ vert, uint32_t nf,
-                                                  PackedTri *__restrict__ tris) {
-  const uint32_t f = blockIdx.x * 256 + threadIdx.x;
-  if (f >= nf) return;
-  const bvht_Triangle t = faces[f];
-  const bvht_vec3 v0 = vert[t.v1], v1 = vert[t.v2], v2 = vert[t.v3];
-  const bvht_vec3 e1 = vsub(v1, v0), e2 = vsub(v2, v0);
-  tris[f] = PackedTri{make_float4(v0.x, v0.y, v0.z, 0.f), make_float4(e1.x, e1.y, e1.z, 0.f),
-                      make_float4(e2.x, e2.y, e2.z, 0.f)};
+// A ray in registers; sx, sy, sz are its sign flags.
+struct WalkRay {
+  bvht_vec3 pos, dir, inv;
+  bool sx, sy, sz;
+};
+__device__ __forceinline__ WalkRay walkRay(const bvht_Ray &r) {
+  return WalkRay{r.pos, r.dir, r.invDir, r.sign[0] != 0, r.sign[1] != 0, r.sign[2] != 0};
 }
 
-// intersectRayAABB -- CUDAKernels.cu:66-85, on a packed box.
+// intersectRayAABB -- CUDAKernels.cu:66-85, on a packed box, against
+// (0.01, t1).  The reference starts from x and takes y and z where they
+// compare greater (near) or smaller (far): a NaN there is ignored, as max and
+// min do, and a NaN in x makes the box missed, which the ordered compare adds.
 __device__ __forceinline__ bool hitBox6(float mnx, float mny, float mnz, float mxx, float mxy, float mxz,
-                                        const bvht_Ray &r, float t0, float t1, float &tmin) {
-  float tmax, tymin, tymax, tzmin, tzmax;
-  tmin = ((r.sign[0] ? mxx : mnx) - r.pos.x) * r.invDir.x;
-  tmax = ((r.sign[0] ? mnx : mxx) - r.pos.x) * r.invDir.x;
-  tymin = ((r.sign[1] ? mxy : mny) - r.pos.y) * r.invDir.y;
-  tymax = ((r.sign[1] ? mny : mxy) - r.pos.y) * r.invDir.y;
-  tzmin = ((r.sign[2] ? mxz : mnz) - r.pos.z) * r.invDir.z;
-  tzmax = ((r.sign[2] ? mnz : mxz) - r.pos.z) * r.invDir.z;
-  if (tymin > tmin) tmin = tymin;
-  if (tzmin > tmin) tmin = tzmin;
-  if (tymax < tmax) tmax = tymax;
-  if (tzmax < tmax) tmax = tzmax;
-  return (tmin < tmax) && (tmin < t1) && (tmax > t0);
+                                        const WalkRay &r, float t1, float &tmin) {
+  const float nx = ((r.sx ? mxx : mnx) - r.pos.x) * r.inv.x, fx = ((r.sx ? mnx : mxx) - r.pos.x) * r.inv.x;
+  const float ny = ((r.sy ? mxy : mny) - r.pos.y) * r.inv.y, fy = ((r.sy ? mny : mxy) - r.pos.y) * r.inv.y;
+  const float nz = ((r.sz ? mxz : mnz) - r.pos.z) * r.inv.z, fz = ((r.sz ? mnz : mxz) - r.pos.z) * r.inv.z;
+  tmin = fmaxf(fmaxf(nx, ny), nz);
+  const float tmax = fminf(fminf(fx, fy), fz);
+  return !__builtin_isunordered(nx, fx) & (tmin < fminf(tmax, t1)) & (tmax > 0.01f);
 }
 
 // intersectRayTriangle2 -- CUDAKernels.cu:88-112, one-sided (the
-// cudaFaceCulling default, meson_options.txt:1), with the edges precomputed
-// by k_packTris.  IEEE 1/det replaces __fdividef.
-__device__ __forceinline__ bool hitTriPacked(const bvht_Ray &r, const PackedTri &t, float &dist) {
-  const bvht_vec3 v0 = {t.v0.x, t.v0.y, t.v0.z}, e1 = {t.e1.x, t.e1.y, t.e1.z}, e2 = {t.e2.x, t.e2.y, t.e2.z};
+// cudaFaceCulling default, meson_options.txt:1), on v0 and the two edges.
+// IEEE 1/det replaces __fdividef; only hits divide.
+__device__ __forceinline__ bool hitTri(const WalkRay &r, bvht_vec3 v0, bvht_vec3 e1, bvht_vec3 e2, float &dist) {
   const bvht_vec3 p = vcross(r.dir, e2);
   const float det = vdot(e1, p);
   const bvht_vec3 tv = vsub(r.pos, v0);
   const bvht_vec3 q = vcross(tv, e1);
-  const float invDet = __fdiv_rn(1.0f, det);
   const float u = vdot(tv, p);
   const float v = vdot(r.dir, q);
-  dist = vdot(e2, q) * invDet;
-  return (det > 0.0f) && ((u >= 0.0f && u <= det) && (v >= 0.0f && (u + v) <= det));
-}
-
-struct TraceCtx {
-  const PackedPair *pairs;
-  const PackedTri *tris;
-  const bvht_BVHNode *nodes;  // parent links (fallback) and multi-triangle leaves
-  uint32_t bound;             // node count the packing covered
-  uint32_t numFaces;
-};
-
-// kTraceRay traversal loop -- CUDAKernels.cu:146-204, over packed nodes,
-// as a state machine: travInit sets up a walk, each travStep visits one
-// node (an inner node's two child boxes, or a leaf's triangles) and moves
-// to the next.  MODE 0: reference triangle test.  MODE 1: hits need
-// t > tMin and are not the triangle `skip` (secondary rays leaving a
-// surface).  `stk` is this lane's column of a [kStackCap][64] LDS array.
-struct TravState {
-  uint64_t lo, hi;  // bit trail: a 1 marks a level whose second child is still pending
-  uint32_t node, info, top, cached, steps;
-  float nearest;
-  TraceOut o;
-};
-
-// Returns false when there is nothing to walk (the root lies outside the tree).
-__device__ __forceinline__ bool travInit(TravState &s, const TraceCtx &cx, uint32_t root) {
-  s.o = {kNoHit, HUGE_VALF, 0};
-  s.nearest = HUGE_VALF;
-  s.lo = s.hi = 0;
-  s.top = s.cached = s.steps = 0;
-  if (root >= cx.bound) return false;
-  s.node = root;
-  s.info = leafInfo(cx.nodes[root]);
+  if (!((det > 0.0f) & (u >= 0.0f) & (u <= det) & (v >= 0.0f) & (u + v <= det))) return false;
+  dist = vdot(e2, q) * __fdiv_rn(1.0f, det);
   return true;
 }
 
-// One visit; returns true when the walk has ended.
-template <int MODE>
-__device__ __forceinline__ bool travStep(TravState &s, const bvht_Ray &ray, const TraceCtx &cx, float tMin,
-                                         uint32_t skip, uint2 *stk) {
-  float dist;
-  if (s.info == kInnerChild) {
-    s.o.intCount++;
-    const PackedPair pp = cx.pairs[s.node];
-    float minL, minR;
-    const bool hl = hitBox6(pp.a.x, pp.a.y, pp.a.z, pp.a.w, pp.b.x, pp.b.y, ray, 0.01f, s.nearest + 0.01f, minL);
-    const bool hr = hitBox6(pp.b.z, pp.b.w, pp.c.x, pp.c.y, pp.c.z, pp.c.w, ray, 0.01f, s.nearest + 0.01f, minR);
-    if (hl || hr) {
-      s.hi = (s.hi << 1) | (s.lo >> 63);
-      s.lo <<= 1;
-      if (hl && hr) {
-        s.lo |= 1;
-        const bool leftFirst = minL < minR;
-        stk[s.top * 64] = leftFirst ? make_uint2(pp.d.y, pp.d.w) : make_uint2(pp.d.x, pp.d.z);
-        s.top = (s.top + 1) & (kStackCap - 1);
-        s.cached = s.cached < kStackCap ? s.cached + 1 : kStackCap;
-        s.node = leftFirst ? pp.d.x : pp.d.y;
-        s.info = leftFirst ? pp.d.z : pp.d.w;
-      } else {
-        s.node = hl ? pp.d.x : pp.d.y;
-        s.info = hl ? pp.d.z : pp.d.w;
-      }
-      return false;
-    }
-  } else if (s.info != kEmptyLeaf) {
-    uint32_t first = s.info, count = 1;
-    if (s.info == kLookupLeaf) {
-      first = cx.nodes[s.node].left;
-      count = cx.nodes[s.node].right;
-    }
-    for (uint32_t k = 0; k < count; ++k) {
-      const uint32_t t = first + k;
-      if (t >= cx.numFaces) break;
-      bool h = hitTriPacked(ray, cx.tris[t], dist);
-      if (MODE == 1) h = h && dist > tMin && t != skip;
-      if (h && dist < s.nearest) {
-        s.nearest = dist;
-        s.o.tri = t;
-      }
-    }
-  }
-  // backtrack to the deepest remembered child
-  if (s.lo == 0 && s.hi == 0) return true;
-  uint32_t tz;
-  if (s.lo != 0) {
-    tz = (uint32_t)__builtin_ctzll(s.lo);
-    if (tz) {
-      s.lo = (s.lo >> tz) | (s.hi << (64 - tz));
-      s.hi >>= tz;
-    }
-  } else {
-    tz = 64 + (uint32_t)__builtin_ctzll(s.hi);
-    s.lo = s.hi >> (tz - 64);
-    s.hi = 0;
-  }
-  s.lo ^= 1;
-  if (s.cached > 0) {
-    s.top = (s.top - 1) & (kStackCap - 1);
-    --s.cached;
-    const uint2 e = stk[s.top * 64];
-    s.node = e.x;
-    s.info = e.y;
-  } else {  // the entry fell out of the cache: walk the parent links
-    uint32_t node = s.node;
-    for (uint32_t k = 0; k < tz && node < cx.bound; ++k) node = cx.nodes[node].parent;
-    if (node >= cx.bound) return true;
-    const uint32_t p = cx.nodes[node].parent;
-    if (p >= cx.bound) return true;
-    node = cx.nodes[node].isLeft == 0 ? cx.nodes[p].left : cx.nodes[p].right;
-    if (node >= cx.bound) return true;
-    s.node = node;
-    s.info = leafInfo(cx.nodes[node]);
-  }
-  return false;
+struct TraceCtx {
+  const NodeRec *recs;
+  const bvht_BVHNode *nodes;  // parent links (dropped children)
+  const bvht_Triangle *faces;
+  const bvht_vec3 *vert;
+  uint32_t bound;  // node count the packing covered
+  uint32_t numFaces;
+};
+
+// One ray's walk (kTraceRay's loop, CUDAKernels.cu:146-204) between two visits.
+struct Walk {
+  uint32_t ref;    // the node to visit
+  uint32_t sp;     // pending children on the stack; kStackCap + 1: one too many, see slowWalk
+  uint32_t count;  // inner nodes visited
+  uint32_t tri;
+  float nearest, t1;  // t1 = nearest + 0.01: boxes beyond are not entered
+};
+
+__device__ __forceinline__ void walkReset(Walk &s, uint32_t rootRef) {
+  s.ref = rootRef;
+  s.sp = s.count = 0;
+  s.tri = kNoHit;
+  s.nearest = s.t1 = HUGE_VALF;
+}
+__device__ __forceinline__ uint32_t rootRef(const TraceCtx &cx, uint32_t root) {
+  return root | (cx.nodes[root].isLeafFlag != 0 ? kLeafRef : 0u);
 }
 
-// A valid tree is walked in at most ~4 visits per node; the step bound only
-// ends the walk on a malformed (cyclic) tree.
-constexpr uint32_t kMaxSteps = 1u << 26;
+// Goes to the next pending child; false: the walk has ended.
+__device__ __forceinline__ bool walkPop(Walk &s, const uint32_t *stk) {
+  if (s.sp == 0) return false;
+  --s.sp;
+  s.ref = stk[s.sp * 64];
+  return true;
+}
 
-template <int MODE>
-__device__ TraceOut traversePacked(const bvht_Ray &ray, const TraceCtx &cx, uint32_t root, float tMin, uint32_t skip,
-                                   uint2 *stk) {
-  TravState s;
-  if (travInit(s, cx, root))
-    while (!travStep<MODE>(s, ray, cx, tMin, skip, stk) && ++s.steps < kMaxSteps) {
+// The two children of an inner node: which one is entered now and which one
+// waits (kNoChild: none).
+constexpr uint32_t kNoChild = 0xFFFFFFFEu;
+__device__ __forceinline__ void innerChildren(const NodeRec *r, const WalkRay &ray, float t1, uint32_t &now,
+                                              uint32_t &later) {
+  const float4 a = r->a, b = r->b, c = r->c;
+  const uint2 d = *reinterpret_cast<const uint2 *>(&r->d);
+  float minL, minR;
+  const bool hl = hitBox6(a.x, a.y, a.z, a.w, b.x, b.y, ray, t1, minL);
+  const bool hr = hitBox6(b.z, b.w, c.x, c.y, c.z, c.w, ray, t1, minR);
+  const bool both = hl & hr, left = hl & (!hr | (minL < minR));
+  now = (hl | hr) ? (left ? d.x : d.y) : kNoChild;
+  later = both ? (left ? d.y : d.x) : kNoChild;
+}
+
+// Visits an inner node; false: the walk has ended or gone past the stack.
+// `stk` is this lane's column of a [kStackCap][64] LDS array.
+__device__ __forceinline__ bool visitInner(Walk &s, const WalkRay &ray, const TraceCtx &cx, uint32_t *stk) {
+  uint32_t now, later;
+  innerChildren(cx.recs + s.ref, ray, s.t1, now, later);
+  s.count++;
+  if (later != kNoChild) {
+    if (s.sp >= (uint32_t)kStackCap) {
+      s.sp = kStackCap + 1;
+      return false;
     }
-  s.o.t = s.nearest;
-  return s.o;
+    stk[s.sp * 64] = later;
+    ++s.sp;
+  }
+  if (now == kNoChild) return walkPop(s, stk);
+  s.ref = now;
+  return true;
+}
+
+// Visits a leaf.  MODE 0: reference triangle test.  MODE 1: hits need
+// t > tMin and are not the triangle `skip` (secondary rays leaving a surface).
+template <int MODE>
+__device__ __forceinline__ void leafHit(Walk &s, uint32_t tri, float dist, float tMin, uint32_t skip) {
+  if (MODE == 1 && !(dist > tMin && tri != skip)) return;
+  if (dist < s.nearest) {
+    s.nearest = dist;
+    s.t1 = dist + 0.01f;
+    s.tri = tri;
+  }
+}
+template <int MODE>
+__device__ __forceinline__ void leafTest(Walk &s, const WalkRay &ray, const TraceCtx &cx, float tMin, uint32_t skip) {
+  const uint32_t node = s.ref & ~kLeafRef;
+  if (node < cx.bound) {
+    const NodeRec *r = cx.recs + node;
+    const float4 a = r->a, b = r->b, c = r->c;
+    const uint32_t first = __float_as_uint(a.w), count = __float_as_uint(b.w);
+    float dist;
+    if (count == 0 || first >= cx.numFaces) return;
+    if (hitTri(ray, {a.x, a.y, a.z}, {b.x, b.y, b.z}, {c.x, c.y, c.z}, dist))
+      leafHit<MODE>(s, first, dist, tMin, skip);
+    for (uint32_t k = 1; k < count; ++k) {  // leaves of several triangles
+      const uint32_t t = first + k;
+      if (t >= cx.numFaces) break;
+      const bvht_Triangle f = cx.faces[t];
+      const bvht_vec3 v0 = cx.vert[f.v1];
+      if (hitTri(ray, v0, vsub(cx.vert[f.v2], v0), vsub(cx.vert[f.v3], v0), dist))
+        leafHit<MODE>(s, t, dist, tMin, skip);
+    }
+  }
+}
+template <int MODE>
+__device__ __forceinline__ bool visitLeaf(Walk &s, const WalkRay &ray, const TraceCtx &cx, float tMin, uint32_t skip,
+                                          const uint32_t *stk) {
+  leafTest<MODE>(s, ray, cx, tMin, skip);
+  return walkPop(s, stk);
+}
+
+// One step of a wave's walks.  `active` lanes have a node to visit.
+template <int MODE>
+__device__ __forceinline__ void walkStep(bool &active, Walk &s, const WalkRay &ray, const TraceCtx &cx,
+                                         float tMin, uint32_t skip, uint32_t *stk) {
+  if (active && (s.ref & kLeafRef) == 0) active = visitInner(s, ray, cx, stk);
+  if (active && (s.ref & kLeafRef) != 0) active = visitLeaf<MODE>(s, ray, cx, tMin, skip, stk);
+}
+
+// A valid tree is walked in at most ~4 visits per node; this bound on the
+// inner visits (looked at now and then) only ends walks of a malformed
+// (cyclic) tree, whose every cycle passes inner nodes.
+constexpr uint32_t kMaxSteps = 1u << 26, kCheckSteps = 1u << 20;
+
+// The walk of a ray that had more than kStackCap children pending, from the
+// start: the reference's 128-bit trail (a 1 marks a level whose second child
+// is still pending) and its parent links instead of a stack.  Same visits.
+template <int MODE>
+__device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx &cx, uint32_t top, float tMin, uint32_t skip) {
+  Walk s;
+  walkReset(s, top);
+  uint64_t lo = 0, hi = 0;
+  while (s.count < kMaxSteps) {
+    const bool leaf = (s.ref & kLeafRef) != 0;
+    if (leaf) {
+      leafTest<MODE>(s, ray, cx, tMin, skip);
+    } else {
+      uint32_t now, later;
+      innerChildren(cx.recs + s.ref, ray, s.t1, now, later);
+      s.count++;
+      if (now != kNoChild) {
+        hi = (hi << 1) | (lo >> 63);
+        lo = (lo << 1) | (later != kNoChild ? 1u : 0u);
+        s.ref = now;
+        continue;
+      }
+    }
+    if ((lo | hi) == 0) break;
+    uint32_t up;  // levels to the deepest node whose second child is pending
+    if (lo != 0) {
+      up = (uint32_t)__builtin_ctzll(lo);
+      if (up) {
+        lo = (lo >> up) | (hi << (64 - up));
+        hi >>= up;
+      }
+    } else {
+      up = 64 + (uint32_t)__builtin_ctzll(hi);
+      lo = hi >> (up - 64);
+      hi = 0;
+    }
+    lo ^= 1;
+    uint32_t node = s.ref & ~kLeafRef;
+    for (uint32_t k = 0; k < up && node < cx.bound; ++k) node = cx.nodes[node].parent;
+    if (node >= cx.bound) break;
+    const uint32_t p = cx.nodes[node].parent;
+    if (p >= cx.bound) break;
+    node = cx.nodes[node].isLeft == 0 ? cx.nodes[p].left : cx.nodes[p].right;
+    if (node >= cx.bound) break;
+    s.ref = rootRef(cx, node);
+  }
+  return TraceOut{s.tri, s.nearest, (uint16_t)s.count};
+}
+
+// Walks one ray per lane to its end (every lane of the wave calls).
+template <int MODE>
+__device__ __forceinline__ TraceOut walkAll(bool active, const bvht_Ray &r, const TraceCtx &cx, uint32_t root,
+                                            float tMin, uint32_t skip, uint32_t *stk) {
+  const WalkRay ray = walkRay(r);
+  const uint32_t top = root < cx.bound ? rootRef(cx, root) : 0u;
+  Walk s;
+  walkReset(s, top);
+  active = active && root < cx.bound;
+  for (uint32_t it = 1;; ++it) {
+    if (__ballot(active) == 0) break;
+    walkStep<MODE>(active, s, ray, cx, tMin, skip, stk);
+    if ((it & (kCheckSteps - 1)) == 0 && s.count >= kMaxSteps) active = false;
+  }
+  if (s.sp > (uint32_t)kStackCap) return slowWalk<MODE>(ray, cx, top, tMin, skip);
+  return TraceOut{s.tri, s.nearest, (uint16_t)s.count};
 }
 
 // Shading of CUDAKernels.cu:208-218.
@@ -338,19 +410,24 @@ __device__ __forceinline__ bvht_CUDAPixel shade(const TraceOut &o, const bvht_Ra
   return px;
 }
 
+// Pixel of lane l in an 8x8 tile: 2x2 blocks of lanes are 2x2 blocks of
+// pixels, so the four lanes whose accesses the L1 merges first are neighbours
+// both ways.
+__device__ __forceinline__ uint32_t tileX(uint32_t l) { return (l & 1) | ((l >> 1) & 2) | ((l >> 2) & 4); }
+__device__ __forceinline__ uint32_t tileY(uint32_t l) { return tileX(l >> 1); }
+
 // Image path: 8x8 pixel tiles per wave (kTraceRay launch shape, CUDAKernels.cu:409-416).
-__global__ __launch_bounds__(64) void k_traceImage(const bvht_Ray *__restrict__ rays, bvht_CUDAPixel *__restrict__ img,
-                                                   TraceCtx cx, uint32_t root, const bvht_vec3 *__restrict__ vert,
-                                                   const bvht_Triangle *__restrict__ faces, bvht_vec3 light, uint32_t w,
-                                                   uint32_t h) {
-  __shared__ uint2 s_stk[kStackCap * 64];
-  const uint32_t x = blockIdx.x * 8 + (threadIdx.x & 7);
-  const uint32_t y = blockIdx.y * 8 + (threadIdx.x >> 3);
-  if (x >= w || y >= h) return;
-  const size_t i = (size_t)y * w + x;
+__global__ __launch_bounds__(64) void k_traceImage(const bvht_Ray *__restrict__ rays,
+                                                      bvht_CUDAPixel *__restrict__ img, TraceCtx cx, uint32_t root,
+                                                      bvht_vec3 light, uint32_t w, uint32_t h) {
+  __shared__ uint32_t s_stk[kStackCap * 64];
+  const uint32_t x = blockIdx.x * 8 + tileX(threadIdx.x);
+  const uint32_t y = blockIdx.y * 8 + tileY(threadIdx.x);
+  const bool in = x < w && y < h;
+  const size_t i = in ? (size_t)y * w + x : 0;
   const bvht_Ray ray = rays[i];
-  const TraceOut o = traversePacked<0>(ray, cx, root, 0.0f, kNoHit, s_stk + threadIdx.x);
-  img[i] = shade(o, ray, vert, faces, light);
+  const TraceOut o = walkAll<0>(in, ray, cx, root, 0.0f, kNoHit, s_stk + threadIdx.x);
+  if (in) img[i] = shade(o, ray, cx.vert, cx.faces, light);
 }
 
 // Ray bundles (kTraceRayBundle, CUDAKernels.cu:240-383): the 64 rays of an
@@ -363,29 +440,28 @@ __global__ __launch_bounds__(64) void k_traceImage(const bvht_Ray *__restrict__ 
 // the same distance the first one met may differ from the per-ray order.
 __global__ __launch_bounds__(64) void k_traceImageBundle(const bvht_Ray *__restrict__ rays,
                                                          bvht_CUDAPixel *__restrict__ img, TraceCtx cx, uint32_t root,
-                                                         const bvht_vec3 *__restrict__ vert,
-                                                         const bvht_Triangle *__restrict__ faces, bvht_vec3 light,
-                                                         uint32_t w, uint32_t h) {
-  __shared__ uint2 s_stk[128];  // pending children: at most one per trail bit
+                                                         bvht_vec3 light, uint32_t w, uint32_t h) {
+  __shared__ uint32_t s_stk[128];  // pending children: at most one per trail bit
   const uint32_t x = blockIdx.x * 8 + (threadIdx.x & 7);
   const uint32_t y = blockIdx.y * 8 + (threadIdx.x >> 3);
   const bool valid = x < w && y < h;
-  bvht_Ray ray;
-  if (valid) ray = rays[(size_t)y * w + x];
+  const bvht_Ray ray = rays[valid ? (size_t)y * w + x : 0];
+  const WalkRay wr = walkRay(ray);
   TraceOut o = {kNoHit, HUGE_VALF, 0};
   if (root < cx.bound) {
     uint64_t lo = 0, hi = 0;  // wave-uniform from here on
-    uint32_t node = root, info = leafInfo(cx.nodes[root]), sp = 0;
+    uint32_t ref = rootRef(cx, root), sp = 0;
     float nearest = HUGE_VALF, dist;
     for (uint32_t steps = 0; steps < (1u << 26); ++steps) {
-      if (info == kInnerChild) {
+      const uint32_t node = ref & ~kLeafRef;
+      if ((ref & kLeafRef) == 0) {
         o.intCount++;
-        const PackedPair pp = cx.pairs[node];
+        const NodeRec pp = cx.recs[node];
         float minL = 0.0f, minR = 0.0f;
         const bool hl =
-            valid && hitBox6(pp.a.x, pp.a.y, pp.a.z, pp.a.w, pp.b.x, pp.b.y, ray, 0.01f, nearest + 0.01f, minL);
+            valid && hitBox6(pp.a.x, pp.a.y, pp.a.z, pp.a.w, pp.b.x, pp.b.y, wr, nearest + 0.01f, minL);
         const bool hr =
-            valid && hitBox6(pp.b.z, pp.b.w, pp.c.x, pp.c.y, pp.c.z, pp.c.w, ray, 0.01f, nearest + 0.01f, minR);
+            valid && hitBox6(pp.b.z, pp.b.w, pp.c.x, pp.c.y, pp.c.z, pp.c.w, wr, nearest + 0.01f, minR);
         const bool anyL = __ballot(hl) != 0, anyR = __ballot(hr) != 0;
         if (anyL || anyR) {
           hi = (hi << 1) | (lo >> 63);
@@ -395,26 +471,28 @@ __global__ __launch_bounds__(64) void k_traceImageBundle(const bvht_Ray *__restr
             const bool wantL = hl && (minL < minR || !hr), wantR = hr && (minR < minL || !hl);
             const int vote = __popcll(__ballot(wantL)) - __popcll(__ballot(wantR));
             const bool leftFirst = vote > 0;
-            if (sp < 128) s_stk[sp] = leftFirst ? make_uint2(pp.d.y, pp.d.w) : make_uint2(pp.d.x, pp.d.z);
+            if (sp < 128) s_stk[sp] = leftFirst ? pp.d.y : pp.d.x;
             ++sp;
-            node = leftFirst ? pp.d.x : pp.d.y;
-            info = leftFirst ? pp.d.z : pp.d.w;
+            ref = leftFirst ? pp.d.x : pp.d.y;
           } else {
-            node = anyL ? pp.d.x : pp.d.y;
-            info = anyL ? pp.d.z : pp.d.w;
+            ref = anyL ? pp.d.x : pp.d.y;
           }
           continue;
         }
-      } else if (info != kEmptyLeaf) {
-        uint32_t first = info, count = 1;
-        if (info == kLookupLeaf) {
-          first = cx.nodes[node].left;
-          count = cx.nodes[node].right;
-        }
+      } else if (node < cx.bound) {
+        const NodeRec pt = cx.recs[node];
+        const uint32_t first = __float_as_uint(pt.a.w), count = __float_as_uint(pt.b.w);
         for (uint32_t k = 0; k < count; ++k) {
           const uint32_t t = first + k;
           if (t >= cx.numFaces) break;
-          if (valid && hitTriPacked(ray, cx.tris[t], dist) && dist < nearest) {
+          bvht_vec3 v0 = {pt.a.x, pt.a.y, pt.a.z}, e1 = {pt.b.x, pt.b.y, pt.b.z}, e2 = {pt.c.x, pt.c.y, pt.c.z};
+          if (k > 0) {
+            const bvht_Triangle f = cx.faces[t];
+            v0 = cx.vert[f.v1];
+            e1 = vsub(cx.vert[f.v2], v0);
+            e2 = vsub(cx.vert[f.v3], v0);
+          }
+          if (valid && hitTri(wr, v0, e1, e2, dist) && dist < nearest) {
             nearest = dist;
             o.tri = t;
           }
@@ -434,24 +512,22 @@ __global__ __launch_bounds__(64) void k_traceImageBundle(const bvht_Ray *__restr
       }
       lo ^= 1;
       if (sp == 0 || sp > 128) break;  // a trail deeper than 128 levels (unsupported, as in the reference)
-      const uint2 e = s_stk[--sp];
-      node = e.x;
-      info = e.y;
+      ref = s_stk[--sp];
     }
     o.t = nearest;
   }
-  if (valid) img[(size_t)y * w + x] = shade(o, ray, vert, faces, light);
+  if (valid) img[(size_t)y * w + x] = shade(o, ray, cx.vert, cx.faces, light);
 }
 
 template <int MODE>
 __global__ __launch_bounds__(64) void k_traceRays(const bvht_Ray *__restrict__ rays, uint32_t num, TraceCtx cx,
-                                                  uint32_t root, const bvht_vec3 *__restrict__ vert,
-                                                  const bvht_Triangle *__restrict__ faces, bvht_vec3 light, float tMin,
-                                                  const uint32_t *__restrict__ skip, bvht_Hit *__restrict__ hits,
-                                                  bvht_CUDAPixel *__restrict__ img, const uint32_t *__restrict__ order,
-                                                  uint32_t imgW) {
-  __shared__ uint2 s_stk[kStackCap * 64];
+                                                     uint32_t root, bvht_vec3 light, float tMin,
+                                                     const uint32_t *__restrict__ skip, bvht_Hit *__restrict__ hits,
+                                                     bvht_CUDAPixel *__restrict__ img,
+                                                     const uint32_t *__restrict__ order, uint32_t imgW) {
+  __shared__ uint32_t s_stk[kStackCap * 64];
   uint32_t i;
+  bool in;
   if (imgW) {  // the rays of an imgW-wide image, row-major: one 8x8 pixel tile per wave
     const uint32_t tilesX = (imgW + 7) / 8;
     // workgroups go to the 8 XCDs round-robin: runs of 4 consecutive tiles
@@ -461,20 +537,21 @@ __global__ __launch_bounds__(64) void k_traceRays(const bvht_Ray *__restrict__ r
     // 5.0 against 3.8 ms at 1080p); the last partial group keeps its order
     const uint32_t b = blockIdx.x, g0 = b / 32 * 32;
     const uint32_t t = g0 + 32 <= gridDim.x ? g0 + (b % 8) * 4 + (b / 8) % 4 : b;
-    const uint32_t x = (t % tilesX) * 8 + (threadIdx.x & 7), y = (t / tilesX) * 8 + (threadIdx.x >> 3);
-    if (x >= imgW || (uint64_t)y * imgW + x >= num) return;
+    const uint32_t x = (t % tilesX) * 8 + tileX(threadIdx.x), y = (t / tilesX) * 8 + tileY(threadIdx.x);
+    in = x < imgW && (uint64_t)y * imgW + x < num;
     i = y * imgW + x;
   } else {
     const uint32_t slot = blockIdx.x * 64 + threadIdx.x;
-    if (slot >= num) return;
-    i = order ? order[slot] : slot;
+    in = slot < num;
+    i = order && in ? order[slot] : slot;
   }
+  if (!in) i = 0;
   const bvht_Ray ray = rays[i];
-  TraceOut o = {kNoHit, HUGE_VALF, 0};
-  if (!(ray.dir.x == 0.0f && ray.dir.y == 0.0f && ray.dir.z == 0.0f))
-    o = traversePacked<MODE>(ray, cx, root, tMin, skip ? skip[i] : kNoHit, s_stk + threadIdx.x);
+  const bool still = ray.dir.x == 0.0f && ray.dir.y == 0.0f && ray.dir.z == 0.0f;
+  const TraceOut o = walkAll<MODE>(in && !still, ray, cx, root, tMin, skip ? skip[i] : kNoHit, s_stk + threadIdx.x);
+  if (!in) return;
   if (hits) hits[i] = bvht_Hit{o.tri, o.t};
-  if (img) img[i] = shade(o, ray, vert, faces, light);
+  if (img) img[i] = shade(o, ray, cx.vert, cx.faces, light);
 }
 
 // Rays of one call traced by resident waves that refill their idle lanes
@@ -485,50 +562,62 @@ __global__ __launch_bounds__(64) void k_traceRays(const bvht_Ray *__restrict__ r
 // has passed `num` and its lanes are idle.
 template <int MODE>
 __global__ __launch_bounds__(64) void k_traceRaysDyn(const bvht_Ray *__restrict__ rays, uint32_t num, TraceCtx cx,
-                                                     uint32_t root, const bvht_vec3 *__restrict__ vert,
-                                                     const bvht_Triangle *__restrict__ faces, bvht_vec3 light,
-                                                     float tMin, const uint32_t *__restrict__ skip,
-                                                     bvht_Hit *__restrict__ hits, bvht_CUDAPixel *__restrict__ img,
-                                                     const uint32_t *__restrict__ order, uint32_t *__restrict__ next) {
-  __shared__ uint2 s_stk[kStackCap * 64];
-  uint2 *stk = s_stk + threadIdx.x;
+                                                        uint32_t root, bvht_vec3 light, float tMin,
+                                                        const uint32_t *__restrict__ skip, bvht_Hit *__restrict__ hits,
+                                                        bvht_CUDAPixel *__restrict__ img,
+                                                        const uint32_t *__restrict__ order,
+                                                        uint32_t *__restrict__ next) {
+  __shared__ uint32_t s_stk[kStackCap * 64];
+  uint32_t *stk = s_stk + threadIdx.x;
   const uint64_t lt = __lanemask_lt();
+  const uint32_t top = rootRef(cx, root);  // the caller has checked the root
   bool active = false, drained = false;
   uint32_t i = 0, skipTri = kNoHit;
-  bvht_Ray ray;
-  TravState s;
-  while (true) {
-    const uint64_t idle = __ballot(!active);
-    const uint32_t nIdle = (uint32_t)__popcll(idle);
-    if (!drained && (nIdle >= kRefillAt || nIdle == 64)) {  // wave-uniform
+  WalkRay ray = {};
+  Walk s;
+  walkReset(s, 0);
+  for (uint32_t it = 1;; ++it) {
+    uint64_t act = __ballot(active);
+    const uint32_t nIdle = 64 - (uint32_t)__popcll(act);
+    if (!drained && (nIdle >= kRefillAt)) {  // wave-uniform
       uint32_t base = 0;
       if (threadIdx.x == 0) base = atomicAdd(next, nIdle);
       base = __shfl(base, 0, 64);
       if (base + nIdle >= num) drained = true;
       if (!active) {
-        const uint32_t slot = base + (uint32_t)__popcll(idle & lt);
+        const uint32_t slot = base + (uint32_t)__popcll(~act & lt);
         if (slot < num) {
           i = order ? order[slot] : slot;
-          ray = rays[i];
+          const bvht_Ray r = rays[i];
+          ray = walkRay(r);
           skipTri = skip ? skip[i] : kNoHit;
-          active = !(ray.dir.x == 0.0f && ray.dir.y == 0.0f && ray.dir.z == 0.0f) && travInit(s, cx, root);
+          walkReset(s, top);
+          active = !(r.dir.x == 0.0f && r.dir.y == 0.0f && r.dir.z == 0.0f);
           if (!active) {  // nothing to walk: a miss
-            const TraceOut o = {kNoHit, HUGE_VALF, 0};
-            if (hits) hits[i] = bvht_Hit{o.tri, o.t};
-            if (img) img[i] = shade(o, ray, vert, faces, light);
+            if (hits) hits[i] = bvht_Hit{kNoHit, HUGE_VALF};
+            if (img) img[i] = bvht_CUDAPixel{0, 0, 0};
           }
         }
       }
+      act = __ballot(active);
     }
-    if (__ballot(active) == 0) {
+    if (act == 0) {
       if (drained) break;
       continue;
     }
-    if (active && (travStep<MODE>(s, ray, cx, tMin, skipTri, stk) || ++s.steps >= kMaxSteps)) {
-      s.o.t = s.nearest;
-      if (hits) hits[i] = bvht_Hit{s.o.tri, s.o.t};
-      if (img) img[i] = shade(s.o, ray, vert, faces, light);
-      active = false;
+    const bool was = active;
+    walkStep<MODE>(active, s, ray, cx, tMin, skipTri, stk);
+    if ((it & (kCheckSteps - 1)) == 0 && s.count >= kMaxSteps) active = false;
+    if (was && !active) {
+      TraceOut o = {s.tri, s.nearest, (uint16_t)s.count};
+      if (s.sp > (uint32_t)kStackCap) o = slowWalk<MODE>(ray, cx, top, tMin, skipTri);
+      if (hits) hits[i] = bvht_Hit{o.tri, o.t};
+      if (img) {
+        bvht_Ray r = {};
+        r.pos = ray.pos;
+        r.dir = ray.dir;
+        img[i] = shade(o, r, cx.vert, cx.faces, light);
+      }
     }
   }
 }
@@ -659,13 +748,11 @@ __global__ __launch_bounds__(256) void k_rayKeys(const bvht_Ray *__restrict__ ra
   }
 }
 
-// Packed copies of the tree and mesh, rebuilt by every trace call (the tree
-// may have changed since the last one); the buffers only grow.
+// Packed copy of the tree and its triangles, rebuilt by every trace call (the
+// tree may have changed since the last one); the buffer only grows.
 struct TraceCache {
-  PackedPair *pairs = nullptr;
-  size_t pairCap = 0;
-  PackedTri *tris = nullptr;
-  size_t triCap = 0;
+  NodeRec *recs = nullptr;
+  size_t recCap = 0;
   uint32_t *bad = nullptr;
   uint32_t *next = nullptr;  // ray counter of k_traceRaysDyn
   // the ray buffer generateRays last filled, as a w x h image
@@ -690,32 +777,24 @@ bool prepareTrace(const bvht_BVHNode *nodes, const bvht_MeshRaw &mesh, TraceCtx 
     return false;
   }
   const uint64_t bound = 2ull * mesh.numFaces - 1;
-  if (bound >= kEmptyLeaf) {
-    setError("%s: %u faces exceed the 32-bit node range", what, mesh.numFaces);
+  if (bound >= kLeafRef) {
+    setError("%s: %u faces exceed the 31-bit node range", what, mesh.numFaces);
     return false;
   }
   TraceCache &c = traceCache();
-  if (c.pairCap < bound) {
-    devFree(c.pairs);
-    c.pairs = nullptr;
-    c.pairCap = 0;
-    if (!devAlloc(&c.pairs, bound, "trace node pairs")) return false;
-    c.pairCap = bound;
-  }
-  if (c.triCap < mesh.numFaces) {
-    devFree(c.tris);
-    c.tris = nullptr;
-    c.triCap = 0;
-    if (!devAlloc(&c.tris, mesh.numFaces, "trace triangles")) return false;
-    c.triCap = mesh.numFaces;
+  if (c.recCap < bound) {
+    devFree(c.recs);
+    c.recs = nullptr;
+    c.recCap = 0;
+    if (!devAlloc(&c.recs, bound, "trace node records")) return false;
+    c.recCap = bound;
   }
   if (!c.bad && !devAlloc(&c.bad, 1, "trace flag")) return false;
   if (!fillU32(c.bad, 0u, 1)) return false;
-  k_packPairs<<<divUp(bound, 256), 256, 0, stream()>>>(nodes, (uint32_t)bound, c.pairs, c.bad);
-  if (!checkLaunch("k_packPairs")) return false;
-  k_packTris<<<divUp(mesh.numFaces, 256), 256, 0, stream()>>>(mesh.faces, mesh.vert, mesh.numFaces, c.tris);
-  if (!checkLaunch("k_packTris")) return false;
-  cx = TraceCtx{c.pairs, c.tris, nodes, (uint32_t)bound, mesh.numFaces};
+  k_packNodes<<<divUp(bound, 256), 256, 0, stream()>>>(nodes, (uint32_t)bound, mesh.faces, mesh.vert, mesh.numFaces,
+                                                       c.recs, c.bad);
+  if (!checkLaunch("k_packNodes")) return false;
+  cx = TraceCtx{c.recs, nodes, mesh.faces, mesh.vert, (uint32_t)bound, mesh.numFaces};
   return true;
 }
 
@@ -815,9 +894,9 @@ void tracerImage(bvht_Ray *rays, bvht_CUDAPixel *img, bvht_BVHNode *nodes, uint3
   if (!prepareTrace(nodes, mesh, cx, "tracerImage")) return;
   dim3 grid(divUp(w, 8), divUp(h, 8));
   if (bundle)
-    k_traceImageBundle<<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, mesh.vert, mesh.faces, light, w, h);
+    k_traceImageBundle<<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
   else
-    k_traceImage<<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, mesh.vert, mesh.faces, light, w, h);
+    k_traceImage<<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
   checkLaunch(bundle ? "k_traceImageBundle" : "k_traceImage");
 }
 
@@ -859,7 +938,7 @@ bool bvht_traceRays(const bvht_Ray *rays, uint32_t num, bvht_BVHNode *nodes, uin
     const TraceCache &c = traceCache();
     const bool image = rays == c.imgRays && (uint64_t)num == (uint64_t)c.imgW * c.imgH;
     const uint32_t blocks = image ? divUp(c.imgW, 8) * divUp(c.imgH, 8) : divUp(num, 64);
-    k_traceRays<0><<<blocks, 64, 0, stream()>>>(rays, num, cx, rootNode, mesh.vert, mesh.faces, light, tMin, skipTri,
+    k_traceRays<0><<<blocks, 64, 0, stream()>>>(rays, num, cx, rootNode, light, tMin, skipTri,
                                                 hits, img, order, image ? c.imgW : 0u);
     return checkLaunch("k_traceRays");
   }
@@ -867,9 +946,9 @@ bool bvht_traceRays(const bvht_Ray *rays, uint32_t num, bvht_BVHNode *nodes, uin
   TraceCache &c = traceCache();
   if (!c.next && !devAlloc(&c.next, 1, "trace ray counter")) return false;
   if (!fillU32(c.next, 0u, 1)) return false;
-  // resident waves only: kTraceWavesPerCU of them fill a CU (LDS-bound)
+  // resident waves only
   const uint32_t waves = std::min<uint32_t>(divUp(num, 64), (uint32_t)numCUs() * kTraceWavesPerCU);
-  k_traceRaysDyn<1><<<waves, 64, 0, stream()>>>(rays, num, cx, rootNode, mesh.vert, mesh.faces, light, tMin, skipTri,
+  k_traceRaysDyn<1><<<waves, 64, 0, stream()>>>(rays, num, cx, rootNode, light, tMin, skipTri,
                                                 hits, img, order, c.next);
   return checkLaunch("k_traceRaysDyn");
 }
