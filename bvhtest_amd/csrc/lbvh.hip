@@ -780,8 +780,8 @@ static bool treeLevelsT(bvht_BVHNode *nodes, const uint32_t *sorted, const bvht_
     const uint64_t U = (((uint64_t)n) + (1ull << unitLog) - 1) >> unitLog;
     const uint32_t blocks = (uint32_t)((U + (1u << TLOG) - 1) >> TLOG);
     if (first)
-      k_buildLevel0<TLOG, false, false><<<blocks, kBuildBlock, 0, stream()>>>(nodes, sorted, faces, vert, nullptr, sd,
-                                                                              nullptr, nullptr);
+      k_buildLevel0<TLOG, false, false><<<blocks, level0Block(TLOG), 0, stream()>>>(nodes, sorted, faces, vert, nullptr,
+                                                                                   sd, nullptr, nullptr);
     else
       k_buildLevelUp<TLOG, false><<<blocks, kBuildBlock, 0, stream()>>>(nodes, sd, nullptr, nullptr, unitLog);
     if (!checkLaunch(first ? "k_buildLevel0" : "k_buildLevelUp")) return false;
@@ -813,11 +813,11 @@ static bool treeLevelsBatchT(bvht_BVHNode *nodes, const uint32_t *sorted, const 
   for (int L = 0; L < levels; ++L) {
     if (counts[L] == 0) continue;
     if (L == 0 && rec)
-      k_buildLevel0<TLOG, true, true><<<counts[L], kBuildBlock, 0, stream()>>>(nodes, sorted, faces, vert, rec, none,
-                                                                                 segs, tiles[L]);
+      k_buildLevel0<TLOG, true, true><<<counts[L], level0Block(TLOG), 0, stream()>>>(nodes, sorted, faces, vert, rec,
+                                                                                    none, segs, tiles[L]);
     else if (L == 0)
-      k_buildLevel0<TLOG, true, false><<<counts[L], kBuildBlock, 0, stream()>>>(nodes, sorted, faces, vert, nullptr,
-                                                                                  none, segs, tiles[L]);
+      k_buildLevel0<TLOG, true, false><<<counts[L], level0Block(TLOG), 0, stream()>>>(nodes, sorted, faces, vert,
+                                                                                     nullptr, none, segs, tiles[L]);
     else
       k_buildLevelUp<TLOG, true><<<counts[L], kBuildBlock, 0, stream()>>>(nodes, none, segs, tiles[L],
                                                                             (uint32_t)(L * TLOG));

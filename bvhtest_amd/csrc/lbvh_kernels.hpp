@@ -4,6 +4,8 @@
 #include "radix_sort.hpp"
 #include "wave.hpp"
 
+#include <type_traits>
+
 namespace bvht {
 
 constexpr int kBuildBlock = 256;
@@ -45,12 +47,18 @@ __device__ __forceinline__ NodeWords packNode(const bvht_AABB &b, uint32_t paren
   return o;
 }
 
+// Orders a wave's own LDS words: what its lanes stored before, they read after.
+__device__ __forceinline__ void stagedFence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // The 64 lanes of a wave write the nodes dst[0..63] (lane l's node, if
 // `write`) through an LDS staging buffer of 64 nodes, so that every store
 // instruction covers 1 KB of consecutive bytes instead of 16 bytes every 48
 // (three instructions per node, each touching 24 lines in part).  All
-// threads of the workgroup call it (barriers: lanes read other lanes'
-// words, and the next call reuses the buffer).
+// lanes of the wave call it; `stage` and `stageOk` are the wave's own, so no
+// other wave waits.
 __device__ __forceinline__ void storeNodesStaged(uint4 *stage, uint8_t *stageOk, bvht_BVHNode *dst, const NodeWords &nw,
                                                  bool write) {
   const uint32_t lane = threadIdx.x & 63;
@@ -58,14 +66,14 @@ __device__ __forceinline__ void storeNodesStaged(uint4 *stage, uint8_t *stageOk,
   stage[3 * lane + 1] = nw.w[1];
   stage[3 * lane + 2] = nw.w[2];
   stageOk[lane] = write ? 1 : 0;
-  __syncthreads();
+  stagedFence();
   uint4 *d = reinterpret_cast<uint4 *>(dst);
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     const uint32_t c = lane + 64 * q;
     if (stageOk[c / 3]) d[c] = stage[c];
   }
-  __syncthreads();
+  stagedFence();
 }
 
 // Writes one full 48-byte node with three 16-byte stores.
@@ -119,26 +127,46 @@ __device__ __forceinline__ void nodeAtIndex(uint32_t p, uint32_t N1, uint32_t &l
   }
 }
 
-// One butterfly step of the in-wave box reduction: b holds the box of the
-// aligned block of `half` leaves around the lane's leaf k and becomes that
-// of the block of 2 * half.  The lower half always comes first in the
-// merge, as a node merges its left child with its right; an upper half
-// starting at or past cnt (no leaves) leaves the box unchanged.
-__device__ __forceinline__ void boxStep(float b[6], uint32_t k, uint32_t half, uint32_t cnt) {
-  float o[6];
-#pragma unroll
-  for (int c = 0; c < 6; ++c) o[c] = __shfl_xor(b[c], (int)half);
-  if (((k & ~(2 * half - 1)) | half) >= cnt) return;
-  const bool upper = (k & half) != 0;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const float lo = upper ? o[c] : b[c], hi = upper ? b[c] : o[c];
-    b[c] = mergeMin(lo, hi);
+// The values of the lower and the upper half of the lane's aligned block of
+// 2 * HALF lanes, where all lanes of a half hold the same.
+template <int HALF>
+__device__ __forceinline__ void halves(float x, float &lo, float &hi) {
+  const int v = __float_as_int(x);
+  int l, h;
+  if constexpr (HALF == 1) {
+    l = __builtin_amdgcn_update_dpp(v, v, 0xA0, 0xF, 0xF, false);  // quad_perm [0, 0, 2, 2]
+    h = __builtin_amdgcn_update_dpp(v, v, 0xF5, 0xF, 0xF, false);  // quad_perm [1, 1, 3, 3]
+  } else if constexpr (HALF == 2) {
+    l = __builtin_amdgcn_update_dpp(v, v, 0x44, 0xF, 0xF, false);  // quad_perm [0, 1, 0, 1]
+    h = __builtin_amdgcn_update_dpp(v, v, 0xEE, 0xF, 0xF, false);  // quad_perm [2, 3, 2, 3]
+  } else if constexpr (HALF == 4 || HALF == 8) {  // the other half's lanes of each row of 16, shifted
+    l = __builtin_amdgcn_update_dpp(v, v, 0x110 + HALF, 0xF, HALF == 4 ? 0xA : 0xC, false);
+    h = __builtin_amdgcn_update_dpp(v, v, 0x100 + HALF, 0xF, HALF == 4 ? 0x5 : 0x3, false);
+  } else {  // odd rows of the first operand change places with even rows of the second; then halves
+    static_assert(HALF == 16 || HALF == 32, "in a wave");
+    const auto r = HALF == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
+                              : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    l = (int)r[0];
+    h = (int)r[1];
   }
+  lo = __int_as_float(l);
+  hi = __int_as_float(h);
+}
+
+// One step of the in-wave box reduction: b holds the box of the aligned block
+// of HALF leaves around the lane's leaf k (the same in all of its lanes) and
+// becomes that of the block of 2 * HALF.  The lower half comes first in the
+// merge, as a node merges its left child with its right; an upper half
+// starting at or past cnt (no leaves) leaves the lower half's box.
+template <int HALF>
+__device__ __forceinline__ void boxStep(float b[6], uint32_t k, uint32_t cnt) {
+  const bool one = ((k & ~(2u * HALF - 1)) | HALF) >= cnt;
 #pragma unroll
-  for (int c = 3; c < 6; ++c) {
-    const float lo = upper ? o[c] : b[c], hi = upper ? b[c] : o[c];
-    b[c] = mergeMax(lo, hi);
+  for (int c = 0; c < 6; ++c) {
+    float lo, hi;
+    halves<HALF>(b[c], lo, hi);
+    const float m = c < 3 ? mergeMin(lo, hi) : mergeMax(lo, hi);
+    b[c] = one ? lo : m;
   }
 }
 
@@ -170,26 +198,30 @@ __device__ __forceinline__ void storeInner(bvht_BVHNode *nodes, uint32_t l, uint
 // inner node written by the lane of position p is the one whose index is p,
 // so a wave's inner nodes are as contiguous as its leaves (an index of a
 // node in the tile lies in the tile).  Boxes of aligned blocks of up to 64
-// positions come from butterfly shuffles inside the wave; the few larger
+// positions come from lane exchanges inside the wave; the few larger
 // blocks of the tile are reduced in LDS from the 64-position blocks.
-// Six workgroups per CU (at most 80 VGPRs) measure faster than four (the
-// compiler's 105 VGPRs without the bound) and than eight (64 VGPRs, with
-// spills).
+// One position per thread (two in tiles of 2,048): a thread's chain is one
+// leaf's, and only the blocks larger than a wave meet at a workgroup barrier.
+// Large builds are bound by memory (4.2M triangles: 137 us whether the boxes
+// come from shuffles through LDS and the stores wait for the workgroup, or as
+// here); small ones by that chain.  Whole builds: 1M triangles 144 -> 142.6 us;
+// in 1,024-position tiles a batch of 64 meshes (700k triangles) 135 -> 128 us
+// and one of 512 (38.4M) 2.63 -> 2.57 ms; 256 threads with four positions each
+// 134 us and 2.80 ms.
 // REC: the leaf boxes are read from `rec` (three float2 per triangle, by
 // global face index, written by the key pass) instead of being made from a
 // face and three vertices: one gather per leaf instead of four.
+constexpr int level0Block(int tlog) { return tlog < 10 ? 1 << tlog : 1024; }
 template <int TLOG, bool BATCH, bool REC>
-__global__ __launch_bounds__(kBuildBlock, 6) void k_buildLevel0(bvht_BVHNode *__restrict__ nodesAll,
-                                                             const uint32_t *__restrict__ sorted,
-                                                             const bvht_Triangle *__restrict__ faces,
-                                                             const bvht_vec3 *__restrict__ vertAll,
-                                                             const float2 *__restrict__ rec, SegDesc single,
-                                                             const SegDesc *__restrict__ segs,
-                                                             const uint2 *__restrict__ tiles) {
+__global__ __launch_bounds__(level0Block(TLOG), (1 << TLOG) > 1024 ? 4 : 8) void k_buildLevel0(
+    bvht_BVHNode *__restrict__ nodesAll, const uint32_t *__restrict__ sorted, const bvht_Triangle *__restrict__ faces,
+    const bvht_vec3 *__restrict__ vertAll, const float2 *__restrict__ rec, SegDesc single,
+    const SegDesc *__restrict__ segs, const uint2 *__restrict__ tiles) {
+  constexpr int BLOCK = level0Block(TLOG);
   constexpr uint32_t T = 1u << TLOG;
-  constexpr int R = T / kBuildBlock;
+  constexpr int R = T / BLOCK;
   constexpr uint32_t NB = T / 64;  // 64-position blocks of a tile
-  static_assert(T % kBuildBlock == 0 && TLOG > 6, "tile holds whole workgroups of 64-position blocks");
+  static_assert(T % BLOCK == 0 && TLOG > 6, "tile holds whole workgroups of 64-position blocks");
   // block boxes of levels 6..TLOG; level j starts at 2 NB - (2 NB >> (j - 6))
   __shared__ float s_box[2 * NB][6];
   SegDesc sd;
@@ -219,7 +251,7 @@ __global__ __launch_bounds__(kBuildBlock, 6) void k_buildLevel0(bvht_BVHNode *__
   uint32_t f[R];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    const uint32_t k = threadIdx.x + i * kBuildBlock;
+    const uint32_t k = threadIdx.x + i * BLOCK;
     f[i] = k < cnt ? sorted[sd.faceBase + u0 + k] - sd.faceBase : 0u;
     if (f[i] >= n) f[i] = 0;  // never read outside the mesh, even from a corrupt permutation
   }
@@ -249,47 +281,39 @@ __global__ __launch_bounds__(kBuildBlock, 6) void k_buildLevel0(bvht_BVHNode *__
   // leaves first: the gathered vertices are dead before the reductions start.
   // A wave's 64 leaves (positions k - lane .. k - lane + 63) are written
   // through the LDS staging buffer.
-  __shared__ uint4 s_stage[kBuildBlock / 64][64 * 3];
-  __shared__ uint8_t s_stageOk[kBuildBlock / 64][64];
+  __shared__ uint4 s_stage[BLOCK / 64][64 * 3];
+  __shared__ uint8_t s_stageOk[BLOCK / 64][64];
   uint4 *stage = s_stage[threadIdx.x >> 6];
   uint8_t *stageOk = s_stageOk[threadIdx.x >> 6];
   const uint32_t lane = threadIdx.x & 63;
-  float leaf[R][6];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    const uint32_t k = threadIdx.x + i * kBuildBlock, p = u0 + k;
+    const uint32_t k = threadIdx.x + i * BLOCK, p = u0 + k;
     const bvht_AABB lb = lbs[i];
     uint32_t parent = 0, isLeft = 0;
     if (k < cnt) parentOf(p, p, N1, parent, isLeft);
     // kGenLeafNodes (LBVH_CUDA.cu:273-292): left = face, right = 1, level = UINT8_MAX
     storeNodesStaged(stage, stageOk, nodes + N1 + (p - lane), packNode(lb, parent, f[i], 1u, 1u, isLeft, 255u, surfaceArea(lb)),
                      k < cnt);
-    leaf[i][0] = lb.minMax[0].x;
-    leaf[i][1] = lb.minMax[0].y;
-    leaf[i][2] = lb.minMax[0].z;
-    leaf[i][3] = lb.minMax[1].x;
-    leaf[i][4] = lb.minMax[1].y;
-    leaf[i][5] = lb.minMax[1].z;
-  }
-#pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const uint32_t k = threadIdx.x + i * kBuildBlock, p = u0 + k;
+    float b[6] = {lb.minMax[0].x, lb.minMax[0].y, lb.minMax[0].z, lb.minMax[1].x, lb.minMax[1].y, lb.minMax[1].z};
     // the inner node with index p, if it lies in the tile
     uint32_t l = 0, r = 0, jn = 0;
     if (k < cnt && p < N1) {
       nodeAtIndex(p, N1, l, r);
       if (l >= u0 && r < u0 + cnt) jn = 32 - __builtin_clz(l ^ r);
     }
-    float *b = leaf[i];
-    float pick[6];
+    float pick[6] = {};
+    auto step = [&](auto half, uint32_t j) {
+      boxStep<decltype(half)::value>(b, k, cnt);
 #pragma unroll
-    for (uint32_t j = 1; j <= 6; ++j) {
-      boxStep(b, k, 1u << (j - 1), cnt);
-      if (jn == j) {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) pick[c] = b[c];
-      }
-    }
+      for (int c = 0; c < 6; ++c) pick[c] = jn == j ? b[c] : pick[c];
+    };
+    step(std::integral_constant<int, 1>(), 1);
+    step(std::integral_constant<int, 2>(), 2);
+    step(std::integral_constant<int, 4>(), 3);
+    step(std::integral_constant<int, 8>(), 4);
+    step(std::integral_constant<int, 16>(), 5);
+    step(std::integral_constant<int, 32>(), 6);
     if ((k & 63) == 0) {
 #pragma unroll
       for (int c = 0; c < 6; ++c) s_box[k >> 6][c] = b[c];
@@ -321,7 +345,7 @@ __global__ __launch_bounds__(kBuildBlock, 6) void k_buildLevel0(bvht_BVHNode *__
   // inner nodes of blocks larger than a wave's 64 positions (a few per tile)
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    const uint32_t k = threadIdx.x + i * kBuildBlock, p = u0 + k;
+    const uint32_t k = threadIdx.x + i * BLOCK, p = u0 + k;
     if (k >= cnt || p >= N1) continue;
     uint32_t l, r;
     nodeAtIndex(p, N1, l, r);
