@@ -15,20 +15,23 @@
 //                sort pass and the box of the referenced vertices;
 //   k_segFix     per chunk: the two mesh boxes compared; a mesh whose
 //                boxes differ gets its keys and histograms recomputed;
-//   k_segPrefix  per (mesh, pass): exclusive scan of the histogram;
+//   k_segPrefix  per (mesh, pass): exclusive scan of the histogram (the wide
+//                passes scan it themselves);
 //   k_segOnesweep one segmented onesweep pass: sort tiles never cross a
 //                mesh, the look-back stops at the mesh's first tile, and
 //                digit offsets start at the mesh's prefix; u32 keys, 8- or
 //                10-bit digits (4 or 3 passes, chosen by the autotuner);
-//   k_segOnesweepWide the 8-bit pass over tiles of 1024 threads x 11 keys,
-//                look-back in rounds of 16 predecessors of the mesh;
+//   k_segOnesweepWide the 8-bit pass over tiles of 1024 threads x 1 to 11
+//                keys, look-back in rounds of 16 predecessors of the mesh;
 //   k_buildLevel0 / k_buildLevelUp the tile hierarchy per mesh (tiles
 //                never cross meshes).
 #include "lbvh_kernels.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 namespace bvht {
@@ -115,18 +118,21 @@ __global__ __launch_bounds__(kBuildBlock) void k_segVertBox(const bvht_vec3 *__r
 
 constexpr int kSegItems = 15;                               // keys per thread of a sort tile
 constexpr uint32_t kSegTile = kSortBlock * kSegItems;       // pairs per sort tile
-constexpr int kSegWideItems = 11;                           // keys per thread of a wide sort tile
-constexpr uint32_t kSegWideTile = kWideBlock * kSegWideItems;
+// Keys per thread of a wide sort tile, smallest first (1,024 threads).
+constexpr int kSegWideItems[] = {1, 2, 4, 7, 11};
+constexpr int kSegWideSizes = 5;
 // triangles per key-pass workgroup: 2^11, two trips of four per thread (512
 // meshes of 38.4M triangles in all: 2^15 left most of the GPU idle in the
-// last round of workgroups, 2.48 ms per build against 2.34)
-constexpr int kChunkLog = 11;
+// last round of workgroups, 2.48 ms per build against 2.34; 2^10: 2.58
+// against 2.57), or 2^10, one trip, while those are at most four workgroups
+// per CU (64 meshes, 700k triangles: 107.8 us against 109.8; 2^9: 113)
+constexpr int kChunkLog = 11, kChunkLogSmall = 10;
 constexpr int kSegMaxHist = 3 * 1024;                       // passes x radix, both digit widths
 constexpr uint32_t kSegFlagAgg = 1u << 30, kSegFlagInc = 2u << 30, kSegCountMask = (1u << 30) - 1;
 
 __host__ __device__ constexpr int segPasses(int radixBits) { return (30 + radixBits - 1) / radixBits; }
 
-// Morton keys of one chunk (up to 2^kChunkLog triangles of one mesh) and
+// Morton keys of one chunk (up to 2^chunkLog triangles of one mesh) and
 // the mesh's histograms of every pass (LDS, then one atomic per non-empty
 // bin).  Four triangles per thread per trip, loads issued before use.  The
 // triangle's leaf box (the tile build's, from the same vertices) goes to
@@ -143,7 +149,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_segMorton(const bvht_vec3 *__re
                                                            const SegDesc *__restrict__ segs,
                                                            const uint2 *__restrict__ chunks, uint32_t *boxOrd,
                                                            uint32_t *__restrict__ keys, float2 *__restrict__ rec,
-                                                           uint32_t *__restrict__ segHist) {
+                                                           uint32_t *__restrict__ segHist, int chunkLog) {
   constexpr int R = 1 << RB, P = segPasses(RB);
   static_assert(P * R <= kSegMaxHist, "histogram fits the LDS array");
   __shared__ uint32_t s_hist[P * R];
@@ -163,7 +169,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_segMorton(const bvht_vec3 *__re
   float rmn[3] = {HUGE_VALF, HUGE_VALF, HUGE_VALF}, rmx[3] = {-HUGE_VALF, -HUGE_VALF, -HUGE_VALF};
   const bvht_vec3 *vert = vertAll + sd.vertBase;
   const bvht_Triangle *fc = faces + sd.faceBase;
-  const uint32_t p0 = c.y << kChunkLog, p1 = min(p0 + (1u << kChunkLog), sd.n);
+  const uint32_t p0 = c.y << chunkLog, p1 = min(p0 + (1u << chunkLog), sd.n);
   constexpr int U = 4;
   __shared__ float2 s_rec[kBuildBlock / 64][64 * 3];
   float2 *wrec = s_rec[threadIdx.x >> 6];
@@ -236,7 +242,8 @@ __global__ __launch_bounds__(kBuildBlock) void k_segFix(const bvht_vec3 *__restr
                                                         const SegDesc *__restrict__ segs,
                                                         const uint2 *__restrict__ chunks,
                                                         const uint32_t *__restrict__ boxOrd,
-                                                        uint32_t *__restrict__ keys, uint32_t *__restrict__ segHist) {
+                                                        uint32_t *__restrict__ keys, uint32_t *__restrict__ segHist,
+                                                        int chunkLog) {
   constexpr int R = 1 << RB, P = segPasses(RB);
   const uint2 c = chunks[blockIdx.x];
   float vb[6], tb[6];
@@ -252,7 +259,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_segFix(const bvht_vec3 *__restr
   const bvht_vec3 off = {0.0f - tb[0], 0.0f - tb[1], 0.0f - tb[2]};
   const bvht_vec3 sc = {__fdiv_rn(1.0f, tb[3] + off.x), __fdiv_rn(1.0f, tb[4] + off.y), __fdiv_rn(1.0f, tb[5] + off.z)};
   const bvht_vec3 *vert = vertAll + sd.vertBase;
-  const uint32_t p0 = c.y << kChunkLog, p1 = min(p0 + (1u << kChunkLog), sd.n);
+  const uint32_t p0 = c.y << chunkLog, p1 = min(p0 + (1u << chunkLog), sd.n);
   for (uint32_t q = p0 + threadIdx.x; q < p1; q += kBuildBlock) {
     const bvht_Triangle t = faces[sd.faceBase + q];
     const uint32_t key = morton30(centroid(vert[t.v1], vert[t.v2], vert[t.v3]), off, sc);
@@ -432,8 +439,8 @@ __global__ __launch_bounds__(kSortBlock) void k_segOnesweep(const uint32_t *__re
 }
 
 // One pass of the segmented onesweep with 8-bit digits over wide tiles
-// (kSegWideTile keys; two workgroups per CU: 8 waves per SIMD, at most 64
-// VGPRs, 63 KB of LDS each), for batches whose key array
+// (1,024 x ITEMS keys; two workgroups per CU: 8 waves per SIMD, at most 64
+// VGPRs and 63 KB of LDS each), for batches whose key array
 // stays below 2^31 bytes (buffer accesses with 32-bit offsets; a load past
 // the end reads 0).  Same order as k_segOnesweep: stable by (mesh, digit).
 // Look-back in rounds of 16 predecessors of the same mesh: thread (g, q)
@@ -443,17 +450,20 @@ __global__ __launch_bounds__(kSortBlock) void k_segOnesweep(const uint32_t *__re
 // the nearest inclusive one.  No tile waits for another's look-back, so the
 // walk is one round unless a digit's nearest inclusive count lies more than
 // 16 tiles back; a mesh's first tile publishes an inclusive count at once.
+// The digits' starts in the mesh (`hist`: its counts) are scanned beside the
+// tile's own: a launch less for every build (4.7 us of 110 for 64 meshes).
+template <int ITEMS>
 __global__ __launch_bounds__(kWideBlock, 8) void k_segOnesweepWide(
     const uint32_t *__restrict__ keysIn, const uint32_t *__restrict__ valsIn, uint32_t *__restrict__ keysOut,
     uint32_t *__restrict__ valsOut, const uint2 *__restrict__ tileTab, const SegDesc *__restrict__ segs,
-    uint32_t total, uint32_t shift, const uint32_t *__restrict__ prefix, int passes, uint32_t *status,
+    uint32_t total, uint32_t shift, const uint32_t *__restrict__ hist, int passes, uint32_t *status,
     uint32_t *counter, uint32_t *err) {
-  constexpr int WAVES = kWideBlock / 64, ITEMS = kSegWideItems, R = kSortRadix;
-  constexpr uint32_t TILE = kSegWideTile, QUADS = R / 4, NONE = 0x80000000u;
+  constexpr int WAVES = kWideBlock / 64, R = kSortRadix;
+  constexpr uint32_t TILE = kWideBlock * ITEMS, QUADS = R / 4, NONE = 0x80000000u;
   static_assert(kWideBlock / QUADS == WAVES, "one look-back group per wave");
   __shared__ uint32_t s_wave[WAVES][R];  // per-wave digit counters, then look-back words
   __shared__ uint32_t s_bstart[R], s_gstart[R];
-  __shared__ uint32_t s_scan[WAVES];
+  __shared__ uint32_t s_scan[2][R / 64];
   __shared__ uint32_t s_tile;
   __shared__ uint32_t s_buf[TILE];  // the staged keys, then the values
 
@@ -466,7 +476,7 @@ __global__ __launch_bounds__(kWideBlock, 8) void k_segOnesweepWide(
   const SegDesc sd = segs[tt.x];
   const uint32_t lt = tt.y, segStart = sd.faceBase, segN = sd.n;
   const uint32_t first = lt * TILE + wave * 64 * ITEMS + lane;  // mesh-local index of item 0
-  const uint32_t meshPrefix = tid < R ? prefix[(size_t)tt.x * passes * R + tid] : 0u;  // issued now, used last
+  const uint32_t meshCount = tid < R ? hist[(size_t)tt.x * passes * R + tid] : 0u;  // issued now, used below
   const BufferRsrc keys = bufferRsrc(keysIn, total * 4u);
   uint32_t kw[ITEMS], rank[ITEMS];
 #pragma unroll
@@ -500,8 +510,26 @@ __global__ __launch_bounds__(kWideBlock, 8) void k_segOnesweepWide(
     }
     storeRelaxedAgent(status + (size_t)g * R + tid, (lt == 0 ? kSegFlagInc : kSegFlagAgg) | count);
   }
-  const uint32_t bstart = blockExclusiveScan<kWideBlock>(count, s_scan);
-  if (tid < R) s_bstart[tid] = bstart;
+  // exclusive scans over the digits: of the tile's counts and of the mesh's
+  uint32_t meshPrefix = 0, bstart = 0;
+  if (tid < R) {
+    bstart = waveInclusiveScan(count);
+    meshPrefix = waveInclusiveScan(meshCount);
+    if (lane == 63) {
+      s_scan[0][wave] = bstart;
+      s_scan[1][wave] = meshPrefix;
+    }
+  }
+  __syncthreads();
+  if (tid < R) {
+    bstart -= count;
+    meshPrefix -= meshCount;
+    for (uint32_t w = 0; w < wave; ++w) {
+      bstart += s_scan[0][w];
+      meshPrefix += s_scan[1][w];
+    }
+    s_bstart[tid] = bstart;
+  }
   __syncthreads();
 
   // keys to their tile positions (digits and item indices recomputed)
@@ -627,12 +655,14 @@ struct BatchInternal {
   int radixBits = 8;
   uint2 *chunks = nullptr;     // (mesh, chunk) of the Morton pass
   uint32_t numChunks = 0;
+  int chunkLog = kChunkLog;
   uint4 *vchunks = nullptr;    // (mesh, first vertex, count) of the vertex box pass
   uint32_t numVChunks = 0;
   uint2 *sortTiles = nullptr;  // (mesh, tile) of the sort passes
   uint32_t numSortTiles = 0;
   uint2 *wideTiles = nullptr;  // (mesh, tile) of the wide 8-bit passes
   uint32_t numWideTiles = 0;
+  int wideItems = 0;  // keys per thread of those tiles
   // sort scratch: [0, 16) pass counters + error word, then the mesh
   // histograms / prefixes (M x passes x radix), then the look-back status
   // (passes x sort tiles x radix); all of it is zeroed before every build
@@ -644,6 +674,31 @@ struct BatchInternal {
   const void *capVert = nullptr, *capFaces = nullptr, *capNodes = nullptr;
 };
 
+// Keys per thread of the wide tiles: the fewest for which the tiles fill no
+// more than a workgroup per CU, or are hardly more than with the largest size
+// (meshes smaller than a tile): a pass is then one workgroup's latency.  One
+// key a thread only for half as many tiles and meshes of at most 16 (one round
+// of look-back).  Whole batches with 1 / 2 / 4 / 7 / 11 keys a thread, us:
+// 64 meshes of up to 800 triangles (18k in all) 46 / 48 / 51 / 57 / 65, one of
+// 65,000 72 / 68 / 68 / 74 / 84, 4 of up to 400,000 (814k) 177 / 141 / 123 /
+// 125 / 130, 32 of up to 400,000 (1.4M) 210 / 170 / 147 / 137 / 145, 512 of up
+// to 500,000 (38.4M) 5,110 / 3,560 / 2,880 / 2,640 / 2,560.
+int segWideItems(const uint32_t *faceCounts, uint32_t numMeshes) {
+  auto tiles = [&](int items) {
+    uint64_t t = 0;
+    for (uint32_t i = 0; i < numMeshes; ++i) t += divUp(faceCounts[i], kWideBlock * items);
+    return t;
+  };
+  const int largest = kSegWideItems[kSegWideSizes - 1];
+  const uint64_t CUs = (uint64_t)numCUs(), alike = tiles(largest) * 5 / 4;
+  const uint32_t most = *std::max_element(faceCounts, faceCounts + numMeshes);
+  for (int items : kSegWideItems) {
+    if (items == 1 && most > 16u * kWideBlock) continue;
+    if (tiles(items) <= std::max(items == 1 ? CUs / 2 : CUs, alike)) return items;
+  }
+  return largest;
+}
+
 // Wide 8-bit passes apply while the key array stays below 2^31 bytes.
 bool useWideSegSort(const BatchInternal *in) { return in->radixBits == 8 && in->totalFaces < (1u << 29); }
 
@@ -652,16 +707,28 @@ bool segSort(BatchInternal *in, int &result) {
   constexpr int R = 1 << RB, P = segPasses(RB);
   uint32_t *counters = in->sortScratch, *hist = in->sortScratch + 16;
   uint32_t *status = hist + (size_t)in->M * P * R;
-  k_segPrefix<RB><<<in->M * P, kSortBlock, 0, stream()>>>(hist);
-  if (!checkLaunch("k_segPrefix")) return false;
+  const bool wide = RB == 8 && useWideSegSort(in);  // the wide passes scan the counts themselves
+  if (!wide) {
+    k_segPrefix<RB><<<in->M * P, kSortBlock, 0, stream()>>>(hist);
+    if (!checkLaunch("k_segPrefix")) return false;
+  }
   int cur = 0;
   for (int pass = 0; pass < P; ++pass) {
     const bool last = pass == P - 1;
-    if (RB == 8 && useWideSegSort(in)) {
-      k_segOnesweepWide<<<in->numWideTiles, kWideBlock, 0, stream()>>>(
-          in->keys[cur], pass == 0 ? nullptr : in->vals[cur], last ? nullptr : in->keys[cur ^ 1], in->vals[cur ^ 1],
-          in->wideTiles, in->segs, in->totalFaces, (uint32_t)(pass * RB), hist + (size_t)pass * R, P,
-          status + (size_t)pass * in->numWideTiles * R, counters + pass, counters + 15);
+    if (wide) {
+      auto launch = [&](auto items) {
+        k_segOnesweepWide<decltype(items)::value><<<in->numWideTiles, kWideBlock, 0, stream()>>>(
+            in->keys[cur], pass == 0 ? nullptr : in->vals[cur], last ? nullptr : in->keys[cur ^ 1], in->vals[cur ^ 1],
+            in->wideTiles, in->segs, in->totalFaces, (uint32_t)(pass * RB), hist + (size_t)pass * R, P,
+            status + (size_t)pass * in->numWideTiles * R, counters + pass, counters + 15);
+      };
+      switch (in->wideItems) {
+        case 1: launch(std::integral_constant<int, 1>()); break;
+        case 2: launch(std::integral_constant<int, 2>()); break;
+        case 4: launch(std::integral_constant<int, 4>()); break;
+        case 7: launch(std::integral_constant<int, 7>()); break;
+        default: launch(std::integral_constant<int, 11>()); break;
+      }
       if (!checkLaunch("k_segOnesweepWide")) return false;
       cur ^= 1;
       continue;
@@ -693,17 +760,17 @@ bool batchStagesT(BatchInternal *in, const bvht_vec3 *vert, const bvht_Triangle 
   int r = 0;
   if (in->radixBits == 10) {
     k_segMorton<10><<<in->numChunks, kBuildBlock, 0, stream()>>>(vert, faces, in->segs, in->chunks, in->boxOrd,
-                                                                 in->keys[0], in->rec, in->sortScratch + 16);
+                                                                 in->keys[0], in->rec, in->sortScratch + 16, in->chunkLog);
     if (!checkLaunch("k_segMorton")) return false;
     k_segFix<10><<<in->numChunks, kBuildBlock, 0, stream()>>>(vert, faces, in->segs, in->chunks, in->boxOrd,
-                                                              in->keys[0], in->sortScratch + 16);
+                                                              in->keys[0], in->sortScratch + 16, in->chunkLog);
     if (!checkLaunch("k_segFix") || !segSort<10>(in, r)) return false;
   } else {
     k_segMorton<8><<<in->numChunks, kBuildBlock, 0, stream()>>>(vert, faces, in->segs, in->chunks, in->boxOrd,
-                                                                in->keys[0], in->rec, in->sortScratch + 16);
+                                                                in->keys[0], in->rec, in->sortScratch + 16, in->chunkLog);
     if (!checkLaunch("k_segMorton")) return false;
     k_segFix<8><<<in->numChunks, kBuildBlock, 0, stream()>>>(vert, faces, in->segs, in->chunks, in->boxOrd,
-                                                             in->keys[0], in->sortScratch + 16);
+                                                             in->keys[0], in->sortScratch + 16, in->chunkLog);
     if (!checkLaunch("k_segFix") || !segSort<8>(in, r)) return false;
   }
   return launchTreeLevelsBatch(TLOG, nodes, in->vals[r], faces, vert, in->rec, in->segs, in->tiles.data(),
@@ -824,6 +891,7 @@ bvht_LBVH_BatchWorkingMemory bvht_LBVH_allocateBatch(uint32_t numMeshes, const u
     bvht_LBVH_freeBatch(&m);
     return m;
   }
+  in->wideItems = segWideItems(faceCounts, numMeshes);
   // Morton chunks and sort tiles: per mesh, never crossing one
   std::vector<uint2> chunks, sortTiles, wideTiles;
   std::vector<uint4> vchunks;
@@ -832,11 +900,14 @@ bvht_LBVH_BatchWorkingMemory bvht_LBVH_allocateBatch(uint32_t numMeshes, const u
     for (uint32_t c = 0; (uint64_t)c * kVertChunk < nv; ++c)
       vchunks.push_back(make_uint4(i, vb + c * kVertChunk, std::min(kVertChunk, nv - c * kVertChunk), 0u));
   }
+  uint64_t small = 0;
+  for (uint32_t i = 0; i < numMeshes; ++i) small += divUp(faceCounts[i], 1u << kChunkLogSmall);
+  in->chunkLog = small <= 4ull * numCUs() ? kChunkLogSmall : kChunkLog;
   for (uint32_t i = 0; i < numMeshes; ++i) {
     const uint32_t n = faceCounts[i];
-    for (uint32_t c = 0; (uint64_t)c << kChunkLog < n; ++c) chunks.push_back(make_uint2(i, c));
+    for (uint32_t c = 0; (uint64_t)c << in->chunkLog < n; ++c) chunks.push_back(make_uint2(i, c));
     for (uint32_t t = 0; (uint64_t)t * kSegTile < n; ++t) sortTiles.push_back(make_uint2(i, t));
-    for (uint32_t t = 0; (uint64_t)t * kSegWideTile < n; ++t) wideTiles.push_back(make_uint2(i, t));
+    for (uint32_t t = 0; (uint64_t)t * kWideBlock * in->wideItems < n; ++t) wideTiles.push_back(make_uint2(i, t));
   }
   in->numChunks = (uint32_t)chunks.size();
   in->numVChunks = (uint32_t)vchunks.size();
@@ -844,7 +915,7 @@ bvht_LBVH_BatchWorkingMemory bvht_LBVH_allocateBatch(uint32_t numMeshes, const u
   in->numWideTiles = (uint32_t)wideTiles.size();
   // scratch for the larger of the two digit widths (10 bits: 3 passes x 1024)
   in->histWords = (size_t)numMeshes * kSegMaxHist;
-  in->statusWords = (size_t)3 * in->numSortTiles * 1024;
+  in->statusWords = std::max((size_t)3 * in->numSortTiles * 1024, (size_t)4 * in->numWideTiles * kSortRadix);
   static_assert(segPasses(8) * 256 <= kSegMaxHist && segPasses(10) * 1024 <= kSegMaxHist, "histogram rows");
   if (!devAlloc(&in->chunks, chunks.size(), "batch chunks") ||
       !check(hipMemcpy(in->chunks, chunks.data(), sizeof(uint2) * chunks.size(), hipMemcpyHostToDevice), "batch chunks") ||
