@@ -658,39 +658,48 @@ __device__ uint32_t decide(PatchRec *r, uint32_t k, uint32_t round, uint64_t *lo
 // k_apply 11.1 -> 4.8 us.
 constexpr uint32_t kPatchLanes = 16, kPatchBlock = 256, kPatchesPerBlock = kPatchBlock / kPatchLanes;
 
+// An undecided patch after round 1, as k_resolveTail reads it: its nodes, its
+// rank and the roots it moves, one word per lane.
+constexpr uint32_t kOpenWords = kPatchLanes, kOpenRank = 12, kOpenMoved = 13;
+static_assert(kNNode <= (int)kOpenRank, "a patch's nodes lie below its rank");
+
 // Round 1 over every patch (the reservations were made by k_search).
 __global__ __launch_bounds__(kPatchBlock) void k_commitFirst(PatchRec *__restrict__ recs, uint32_t K, uint64_t *locks,
                                                              uint32_t *__restrict__ marks,
                                                              uint32_t *__restrict__ skipped,
                                                              uint32_t *__restrict__ stats,
-                                                             uint32_t *__restrict__ pending,
+                                                             uint32_t *__restrict__ open,
                                                              uint32_t *__restrict__ numPending) {
   const uint32_t k = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes, j = threadIdx.x % kPatchLanes;
   const bool in = k < K;  // every lane stays for the ballots
   PatchRec *r = recs + (in ? k : 0);
   const uint32_t ok = in ? r->ok : (uint32_t)REC_NONE;
   const uint32_t n = in && j < (uint32_t)kNNode ? r->node[j] : NONE;
-  const uint32_t moved = in && j < 2 ? r->moved[j] : NONE;
-  const bool open = ok == REC_PENDING, use = open && n != NONE;
+  const bool mover = j == kOpenMoved || j == kOpenMoved + 1;
+  const uint32_t moved = in && mover ? r->moved[j - kOpenMoved] : NONE;
+  const bool undecided = ok == REC_PENDING, use = undecided && n != NONE;
   const uint64_t mine = lockKey(1, k);
   const uint64_t v = use ? __hip_atomic_load(locks + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : mine;
   const uint32_t group = threadIdx.x & 63u & ~(kPatchLanes - 1);
   const bool lost = ((__ballot((v >> 32) == 0) >> group) & 0xFFFFu) != 0;  // node of an applied patch
   const bool holdAll = ((__ballot(v != mine) >> group) & 0xFFFFu) == 0;
-  if (!open) return;
+  if (!undecided) return;
   if (!lost && holdAll) {
     if (use)
       atomicMin(reinterpret_cast<unsigned long long *>(locks + n), (unsigned long long)lockKey(kRoundWin, k));
-    if (j < 2) marks[moved] = k;  // moved roots are patch nodes: one applied patch each
+    if (mover) marks[moved] = k;  // moved roots are patch nodes: one applied patch each
     if (j == 0) r->ok = REC_WON;
-  } else if (j == 0) {
-    if (lost) {
+  } else if (lost) {
+    if (j == 0) {
       r->ok = REC_LOST;
       skipped[k] += 1;
       atomicAdd(stats + ST_CONFLICT, 1u);
-    } else {
-      pending[atomicAdd(numPending, 1u)] = k;
     }
+  } else {
+    uint32_t slot = 0;
+    if (j == 0) slot = atomicAdd(numPending, 1u);
+    slot = __shfl(slot, 0, kPatchLanes);
+    open[slot * kOpenWords + j] = j == kOpenRank ? k : mover ? moved : n;
   }
 }
 
@@ -703,17 +712,21 @@ __global__ __launch_bounds__(kPatchBlock) void k_commitFirst(PatchRec *__restric
 // patches go into an LDS hash table holding, per node, whether a winner took
 // it (round 1's from its global lock, read once) and the lowest rank
 // reserving it this round, and each thread keeps its patches' table slots in
-// registers.  A round is two barriers: a patch with a taken node loses, the
+// registers.  The table is built by 16 lanes a patch, from the entries that
+// k_commitFirst left (a line each): a node a lane, every load and every first
+// probe of a thread in flight together (one thread a patch, node by node from
+// its record: 22.0 against 13.3 us before the first round with 772 patches,
+// 7.2 against 4.7 with 50).  A round is two barriers: a patch with a taken node loses, the
 // others reserve their nodes; a patch that holds them all wins and takes
 // them.  (A losing patch no longer reserves, which decides its neighbours no
 // later.)  The reservations of a round are cleared by their own patches
-// while the next round uses the other of two arrays; the second one lies
-// where the node ids were, which are only needed to build the table.  Nothing
+// while the next round uses the other of two arrays; the two lie where the
+// slots and the node ids were while the table was built.  Nothing
 // is written to memory before the last round: a barrier would wait for it.
-// Measured per chunk: 627 patches of 1M triangles 14.1 -> 11.0 us; 1,638
-// patches of 65,536 triangles (10% per step) 48 -> 31 us in the mean, the
+// Measured per chunk: 627 patches of 1M triangles 14.1 -> 10.4 us; 1,638
+// patches of 65,536 triangles (10% per step) 48 -> 24 us in the mean; the
 // first chunks of a step, whose more than 1,024 undecided patches took the
-// global rounds before, 168 -> 58 us.
+// global rounds before, 168 -> 47 us.
 // Global locks keep their round-1 values (k_apply releases them all).
 constexpr int kTailBlock = 1024;
 constexpr uint32_t kTailSlotsLog = 14, kTailSlots = 1u << kTailSlotsLog;
@@ -724,72 +737,106 @@ static_assert(kTailCap <= kTailPer * kTailBlock, "every patch of the LDS rounds 
 
 __device__ __forceinline__ uint32_t tailHash(uint32_t n) { return (n * 0x9E3779B1u) >> (32 - kTailSlotsLog); }
 
-// Slot of node n, inserted if absent (the table never overflows).
-__device__ __forceinline__ uint32_t tailInsert(uint32_t *keys, uint32_t n) {
-  uint32_t h = tailHash(n);
-  for (uint32_t probe = 0; probe < kTailSlots; ++probe) {
+// Slot of node n, inserted if absent, after a first probe at h found another
+// node (the table never overflows).
+__device__ __forceinline__ uint32_t tailInsert(uint32_t *keys, uint32_t n, uint32_t h) {
+  for (uint32_t probe = 1; probe < kTailSlots; ++probe) {
+    h = (h + 1) & (kTailSlots - 1);
     const uint32_t prev = atomicCAS(keys + h, kTailEmpty, n);
     if (prev == kTailEmpty || prev == n) return h;
-    h = (h + 1) & (kTailSlots - 1);
   }
-  return kTailEmpty;  // unreachable
+  return 0;  // unreachable
 }
+
+constexpr uint32_t kTailGroups = kTailBlock / kPatchLanes;                          // patches loaded at a time
+constexpr uint32_t kTailTrips = (kTailCap + kTailGroups - 1) / kTailGroups;
 
 __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict__ recs, uint64_t *locks,
                                                            uint32_t *__restrict__ marks,
                                                            uint32_t *__restrict__ skipped, uint32_t *__restrict__ stats,
-                                                           uint32_t *listA, uint32_t *listB,
-                                                           const uint32_t *__restrict__ numPending) {
-  __shared__ __align__(16) uint32_t s_min[2][kTailSlots];  // lowest reserving rank, rounds alternate; [1] starts as the node ids
+                                                           const uint32_t *__restrict__ open, uint32_t *listA,
+                                                           uint32_t *listB, const uint32_t *__restrict__ numPending) {
+  // lowest reserving rank per slot, rounds alternate; at first [1] holds the
+  // node ids and [0] the patches' slots (16 bits each)
+  __shared__ __align__(16) uint32_t s_min[2][kTailSlots];
   __shared__ __align__(16) uint32_t s_taken4[kTailSlots / 4];  // bytes: taken by a winner
   __shared__ uint32_t s_open[3];                 // undecided patches after a round (rounds rotate)
   __shared__ uint32_t s_cnt;
   uint8_t *s_taken = reinterpret_cast<uint8_t *>(s_taken4);
+  uint16_t *s_slot = reinterpret_cast<uint16_t *>(&s_min[0][0]);
+  static_assert(kTailSlots <= 65535 && kTailCap * kNNode * 2 <= sizeof(s_min[0]), "the slots fit s_min[0]");
   uint32_t num = *numPending;
   if (num == 0) return;
   const uint32_t maxRound = num + 2;
   if (num <= kTailCap) {
-    uint32_t k[kTailPer], node[kTailPer][kNNode], moved[kTailPer][2];
-    bool taken[kTailPer][kNNode];
+    // 16 lanes per patch: a lane loads one node of each of up to kTailTrips
+    // patches and its lock, all in flight together, and inserts it
+    const uint32_t j = threadIdx.x % kPatchLanes, first = threadIdx.x / kPatchLanes;
+    uint32_t n[kTailTrips], prev[kTailTrips], takenMask = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kTailTrips; ++i) {
+      n[i] = NONE;
+      if (i * kTailGroups < num && i * kTailGroups + first < num && j < (uint32_t)kNNode)
+        n[i] = open[(i * kTailGroups + first) * kOpenWords + j];
+    }
+    uint4 rank[kTailPer];  // the patches of the rounds: rank and moved roots
 #pragma unroll
     for (uint32_t q = 0; q < kTailPer; ++q) {
       const uint32_t at = threadIdx.x + q * kTailBlock;
-      k[q] = at < num ? listA[at] : NONE;
+      rank[q] = make_uint4(NONE, NONE, NONE, NONE);
+      if (at < num) rank[q] = *reinterpret_cast<const uint4 *>(open + at * kOpenWords + kOpenRank);
     }
-#pragma unroll
-    for (uint32_t q = 0; q < kTailPer; ++q) {
-      const PatchRec *r = recs + (k[q] == NONE ? 0u : k[q]);
-#pragma unroll
-      for (int j = 0; j < kNNode; ++j) node[q][j] = k[q] == NONE ? NONE : r->node[j];
-      moved[q][0] = r->moved[0];
-      moved[q][1] = r->moved[1];
-    }
-    uint4 *min4 = reinterpret_cast<uint4 *>(&s_min[0][0]), *taken16 = reinterpret_cast<uint4 *>(s_taken4);
-    for (uint32_t i = threadIdx.x; i < 2 * kTailSlots / 4; i += kTailBlock)
-      min4[i] = make_uint4(kTailEmpty, kTailEmpty, kTailEmpty, kTailEmpty);
+    uint4 *ids4 = reinterpret_cast<uint4 *>(&s_min[1][0]), *taken16 = reinterpret_cast<uint4 *>(s_taken4);
+    for (uint32_t i = threadIdx.x; i < kTailSlots / 4; i += kTailBlock)
+      ids4[i] = make_uint4(kTailEmpty, kTailEmpty, kTailEmpty, kTailEmpty);
     for (uint32_t i = threadIdx.x; i < kTailSlots / 16; i += kTailBlock) taken16[i] = make_uint4(0, 0, 0, 0);
     if (threadIdx.x < 3) s_open[threadIdx.x] = 0;
 #pragma unroll
-    for (uint32_t q = 0; q < kTailPer; ++q)
+    for (uint32_t i = 0; i < kTailTrips; ++i) {  // a lock's upper half: 0 once a winner of round 1 holds it
+      prev[i] = 1;
+      if (i * kTailGroups < num && n[i] != NONE)
+        prev[i] = loadRelaxedAgent(reinterpret_cast<const uint32_t *>(locks + n[i]) + 1);
+    }
 #pragma unroll
-      for (int j = 0; j < kNNode; ++j)
-        taken[q][j] = node[q][j] != NONE &&
-                      (__hip_atomic_load(locks + node[q][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) == 0;
+    for (uint32_t i = 0; i < kTailTrips; ++i) takenMask |= prev[i] == 0 ? 1u << i : 0u;
+    static_assert(kTailTrips <= 32, "a bit per trip");
     __syncthreads();
 #pragma unroll
-    for (uint32_t q = 0; q < kTailPer; ++q)
+    for (uint32_t i = 0; i < kTailTrips; ++i)  // the first probes go out together
+      if (i * kTailGroups < num && n[i] != NONE) prev[i] = atomicCAS(&s_min[1][tailHash(n[i])], kTailEmpty, n[i]);
 #pragma unroll
-      for (int j = 0; j < kNNode; ++j)
-        if (node[q][j] != NONE) {  // node[][] holds table slots from here on
-          node[q][j] = tailInsert(s_min[1], node[q][j]);
-          if (taken[q][j]) s_taken[node[q][j]] = 1;
-        }
+    for (uint32_t i = 0; i < kTailTrips; ++i) {
+      if (i * kTailGroups >= num) continue;
+      uint32_t h = 0xFFFFu;
+      if (n[i] != NONE) {
+        h = tailHash(n[i]);
+        if (prev[i] != kTailEmpty && prev[i] != n[i]) h = tailInsert(&s_min[1][0], n[i], h);
+        if (takenMask >> i & 1) s_taken[h] = 1;
+      }
+      n[i] = h;
+      const uint32_t at = i * kTailGroups + first;
+      if (at < num && j < (uint32_t)kNNode) s_slot[at * kNNode + j] = (uint16_t)h;
+    }
     __syncthreads();
+    uint32_t k[kTailPer], node[kTailPer][kNNode];  // slots
 #pragma unroll
-    for (uint32_t q = 0; q < kTailPer; ++q)  // the node ids give way to the odd rounds' reservations
+    for (uint32_t q = 0; q < kTailPer; ++q) {
+      const uint32_t at = threadIdx.x + q * kTailBlock;
+      k[q] = rank[q].x;
 #pragma unroll
-      for (int j = 0; j < kNNode; ++j)
-        if (node[q][j] != NONE) s_min[1][node[q][j]] = kTailEmpty;
+      for (int c = 0; c < kNNode; ++c) {
+        const uint32_t h = at < num ? s_slot[at * kNNode + c] : 0xFFFFu;
+        node[q][c] = h == 0xFFFFu ? NONE : h;
+      }
+    }
+    __syncthreads();
+    // the ids and the slots give way to reservations
+#pragma unroll
+    for (uint32_t i = 0; i < kTailTrips; ++i)
+      if (i * kTailGroups < num && n[i] != 0xFFFFu) s_min[1][n[i]] = kTailEmpty;
+    uint4 *min4 = reinterpret_cast<uint4 *>(&s_min[0][0]);
+    for (uint32_t i = threadIdx.x; i < kTailSlots / 4; i += kTailBlock)
+      min4[i] = make_uint4(kTailEmpty, kTailEmpty, kTailEmpty, kTailEmpty);
     uint32_t state[kTailPer];
     bool reserved[kTailPer];  // in the round before
 #pragma unroll
@@ -852,8 +899,8 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
       PatchRec *r = recs + k[q];
       if (state[q] == REC_WON) {
         r->ok = REC_WON;
-        marks[moved[q][0]] = k[q];  // moved roots are patch nodes: one applied patch each
-        marks[moved[q][1]] = k[q];
+        marks[rank[q].y] = k[q];  // moved roots are patch nodes: one applied patch each
+        marks[rank[q].z] = k[q];
         continue;
       }
       unresolved += state[q] == REC_PENDING;
@@ -867,6 +914,8 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
   }
   // more undecided patches than the LDS table takes: the rounds on the
   // global locks
+  for (uint32_t i = threadIdx.x; i < num; i += kTailBlock) listA[i] = open[i * kOpenWords + kOpenRank];
+  __syncthreads();
   uint32_t *cur = listA, *nxt = listB;
   for (uint32_t round = 2; num > 0 && round <= maxRound; ++round) {
     for (uint32_t i = threadIdx.x; i < num; i += kTailBlock) reserve(recs + cur[i], cur[i], round, locks);
@@ -1638,7 +1687,7 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
             devAlloc(&in->vals[0], in->numInner, "bn13 vals") && devAlloc(&in->vals[1], in->numInner, "bn13 vals") &&
             devMalloc(reinterpret_cast<void **>(&in->sortScratch), sortScratchBytes(in->plan), "bn13 sort") &&
             devAlloc(&in->recs, batchSize, "bn13 patches") && devAlloc(&in->state, in->stateWords, "bn13 state") &&
-            devAlloc(&in->pending[0], batchSize, "bn13 pending") && devAlloc(&in->pending[1], batchSize, "bn13 pending") &&
+            devAlloc(&in->pending[0], (1 + kOpenWords) * (size_t)batchSize, "bn13 pending") && devAlloc(&in->pending[1], batchSize, "bn13 pending") &&
             devAlloc(&in->selCounts, selBlocks, "bn13 select") && devAlloc(&in->partials, kSahBlocks, "bn13 SAH");
   if (!ok) {
     freeMemory(&m);
@@ -1885,7 +1934,8 @@ void bn13_rmAndReinsChunk(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer
                                                      in->pending[0], in->numPending);
   if (!checkLaunch("k_commitFirst")) return;
   k_resolveTail<<<1, kTailBlock, 0, stream()>>>(in->recs, in->locks, in->marks, in->skipped, in->stats, in->pending[0],
-                                                in->pending[1], in->numPending);
+                                                in->pending[0] + kOpenWords * (size_t)in->K, in->pending[1],
+                                                in->numPending);
   if (!checkLaunch("k_resolveTail")) return;
   k_contain<<<divUp(K, kContainBlock / 2), kContainBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->root, in->N, in->marks, in->skipped,
                                                  in->stats);
