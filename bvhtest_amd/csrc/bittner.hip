@@ -14,10 +14,11 @@
 //     k_commitFirst / k_resolveTail  deterministic reservations: exactly the
 //               patches a rank-ordered first-come locking applies (the
 //               reference's kCheckConflicts, timing-dependent there);
+//               (beside them, the paths above the insertion points are walked);
 //     k_contain a winner whose insertion point lies in a subtree another
 //               winner moves is dropped (two such patches would form a cycle;
-//               the reference has no guard);
-//     k_apply   winners write their topology, all locks are released;
+//               the reference has no guard); the others write their topology,
+//               all locks are released;
 //     k_refit   two-phase targeted refit from the 3 changed nodes of every
 //               winner (the kFixTree3_1 / kFixTree3_2 result).  Boxes are
 //               exact min/max, so this equals the reference's full refit
@@ -53,7 +54,8 @@ enum { ST_CONFLICT = 0, ST_FAILED, ST_CONTAIN, ST_OVERFLOW, ST_APPLIED, ST_UNRES
 // 0) compare smaller.
 constexpr uint64_t kLockFree = ~0ull;
 constexpr uint32_t kRoundWin = 0xFFFFFFFFu;
-enum : uint32_t { REC_NONE = 0, REC_PENDING = 1, REC_LOST = 2, REC_CONTAINED = 3, REC_WON = 4 };
+// The last three: the patch won its nodes.
+enum : uint32_t { REC_NONE = 0, REC_PENDING = 1, REC_LOST = 2, REC_CONTAINED = 3, REC_WON = 4, REC_APPLIED = 5 };
 
 __device__ __forceinline__ uint64_t lockKey(uint32_t round, uint32_t k) {
   return ((uint64_t)(0xFFFFFFFFu - round) << 32) | k;
@@ -527,7 +529,8 @@ __global__ __launch_bounds__(64) void k_search(const bvht_BVHNode *__restrict__ 
                                                const uint32_t *__restrict__ order, const uint32_t *__restrict__ inner,
                                                uint32_t numInner, uint32_t chunk, uint32_t numChunks, uint32_t K,
                                                uint32_t offsetAccess, uint32_t alt, PatchRec *__restrict__ recs,
-                                               uint64_t *locks, uint32_t *__restrict__ stats, RecordSink sink,
+                                               uint64_t *locks, uint32_t *__restrict__ marks,
+                                               uint32_t *__restrict__ stats, RecordSink sink,
                                                const uint32_t *__restrict__ sortErr) {
   __shared__ Patch P;
   __shared__ uint2 s_stk[kStackCap];  // node, induced cost
@@ -540,6 +543,10 @@ __global__ __launch_bounds__(64) void k_search(const bvht_BVHNode *__restrict__ 
     return;
   }
   const uint32_t nodeIdx = inner[pos];
+  if (!PROBE && lane < 2) {  // takes the marks of the chunk before away (any mark is old here)
+    const uint32_t was = rec->moved[lane];
+    if (rec->ok >= REC_CONTAINED && was < N) marks[was] = NONE;
+  }
   // The workgroup is one wave: everything below but the patch itself (lane 0
   // edits it) is computed by every lane alike.
   float cost[2] = {0.0f, 0.0f};
@@ -655,7 +662,7 @@ __device__ uint32_t decide(PatchRec *r, uint32_t k, uint32_t round, uint64_t *lo
 // are one round trip each instead of ten in a row (a chunk has a few hundred
 // to a few thousand patches, far too few to hide a chain of loads per
 // thread).  1M triangles, 627 patches: k_commitFirst 13.3 -> 4.8 us,
-// k_apply 11.1 -> 4.8 us.
+// writing the topology 11.1 -> 4.8 us (a launch of its own then).
 constexpr uint32_t kPatchLanes = 16, kPatchBlock = 256, kPatchesPerBlock = kPatchBlock / kPatchLanes;
 
 // An undecided patch after round 1, as k_resolveTail reads it: its nodes, its
@@ -669,7 +676,9 @@ __global__ __launch_bounds__(kPatchBlock) void k_commitFirst(PatchRec *__restric
                                                              uint32_t *__restrict__ skipped,
                                                              uint32_t *__restrict__ stats,
                                                              uint32_t *__restrict__ open,
-                                                             uint32_t *__restrict__ numPending) {
+                                                             uint32_t *__restrict__ numPending,
+                                                             uint32_t *__restrict__ deep) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *deep = 0;
   const uint32_t k = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes, j = threadIdx.x % kPatchLanes;
   const bool in = k < K;  // every lane stays for the ballots
   PatchRec *r = recs + (in ? k : 0);
@@ -727,7 +736,7 @@ __global__ __launch_bounds__(kPatchBlock) void k_commitFirst(PatchRec *__restric
 // patches of 65,536 triangles (10% per step) 48 -> 24 us in the mean; the
 // first chunks of a step, whose more than 1,024 undecided patches took the
 // global rounds before, 168 -> 47 us.
-// Global locks keep their round-1 values (k_apply releases them all).
+// Global locks keep their round-1 values (k_contain releases them all).
 constexpr int kTailBlock = 1024;
 constexpr uint32_t kTailSlotsLog = 14, kTailSlots = 1u << kTailSlotsLog;
 constexpr uint32_t kTailCap = kTailSlots / kNNode;  // patches: the table never overflows
@@ -748,6 +757,29 @@ __device__ __forceinline__ uint32_t tailInsert(uint32_t *keys, uint32_t n, uint3
   return 0;  // unreachable
 }
 
+// The nodes from patch k's insertion point w up to the root, for k_contain:
+// their number and then themselves.  A path that does not fit sets *deep.
+constexpr uint32_t kPathWords = 128;
+__device__ void walkPath(const PatchRec *__restrict__ recs, uint32_t k, uint32_t w,
+                         const bvht_BVHNode *__restrict__ nodes, uint32_t root, uint32_t *__restrict__ paths,
+                         uint32_t *__restrict__ deep) {
+  const uint32_t ok = recs[k].ok;  // another workgroup may be deciding it: undecided patches walk too
+  if (ok == REC_NONE || ok == REC_LOST) return;
+  uint32_t *path = paths + (2 * (size_t)k + w) * kPathWords;
+  uint32_t x = recs[k].best[w], len = 0;
+  while (true) {
+    const uint32_t p = nodes[x].parent;
+    path[++len] = x;
+    if (x == root) break;
+    if (len == kPathWords - 1) {
+      *deep = 1;
+      break;
+    }
+    x = p;
+  }
+  path[0] = len;
+}
+
 constexpr uint32_t kTailGroups = kTailBlock / kPatchLanes;                          // patches loaded at a time
 constexpr uint32_t kTailTrips = (kTailCap + kTailGroups - 1) / kTailGroups;
 
@@ -755,7 +787,10 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
                                                            uint32_t *__restrict__ marks,
                                                            uint32_t *__restrict__ skipped, uint32_t *__restrict__ stats,
                                                            const uint32_t *__restrict__ open, uint32_t *listA,
-                                                           uint32_t *listB, const uint32_t *__restrict__ numPending) {
+                                                           uint32_t *listB, const uint32_t *__restrict__ numPending,
+                                                           uint32_t K, const bvht_BVHNode *__restrict__ nodes,
+                                                           uint32_t root, uint32_t *__restrict__ paths,
+                                                           uint32_t walkers, uint32_t *__restrict__ deep) {
   // lowest reserving rank per slot, rounds alternate; at first [1] holds the
   // node ids and [0] the patches' slots (16 bits each)
   __shared__ __align__(16) uint32_t s_min[2][kTailSlots];
@@ -764,6 +799,11 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
   __shared__ uint32_t s_cnt;
   uint8_t *s_taken = reinterpret_cast<uint8_t *>(s_taken4);
   uint16_t *s_slot = reinterpret_cast<uint16_t *>(&s_min[0][0]);
+  if (blockIdx.x > 0) {  // workgroup-uniform
+    const uint32_t at = (blockIdx.x - 1) * walkers + threadIdx.x;
+    if (threadIdx.x < walkers && at / 2 < K) walkPath(recs, at / 2, at & 1, nodes, root, paths, deep);
+    return;
+  }
   static_assert(kTailSlots <= 65535 && kTailCap * kNNode * 2 <= sizeof(s_min[0]), "the slots fit s_min[0]");
   uint32_t num = *numPending;
   if (num == 0) return;
@@ -941,61 +981,27 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
   }
 }
 
-// Drops a winner whose insertion point lies below a node another winner moves.
-// Two lanes per patch, one for each insertion point; a level's mark and
-// parent link are loaded together, so a level costs one round trip (1M
-// triangles: 31.1 -> 12.4 us with the two walks one after the other and
-// two dependent loads per level before).
-constexpr uint32_t kContainBlock = 64;
-__global__ __launch_bounds__(kContainBlock) void k_contain(PatchRec *__restrict__ recs, uint32_t K,
-                                                           const bvht_BVHNode *__restrict__ nodes, uint32_t root,
-                                                           uint32_t N, const uint32_t *__restrict__ marks,
-                                                           uint32_t *__restrict__ skipped,
-                                                           uint32_t *__restrict__ stats) {
-  const uint32_t k = blockIdx.x * (kContainBlock / 2) + threadIdx.x / 2, w = threadIdx.x & 1;
-  const bool in = k < K;  // every lane stays for the shuffle
-  PatchRec *r = recs + (in ? k : 0);
-  const uint32_t ok = in ? r->ok : (uint32_t)REC_NONE;
-  uint32_t x = r->best[w];  // written for every patch that reserved; only read for winners
-  const bool won = ok == REC_WON;
-  bool bad = false;
-  if (won) {
-    for (uint32_t steps = 0; steps < N; ++steps) {
-      uint32_t m = marks[x], p = nodes[x].parent;
-      asm volatile("" : "+v"(m), "+v"(p));  // both loads go out before either is used
-      if (m != NONE && m != k) {
-        bad = true;
-        break;
-      }
-      if (x == root) break;
-      x = p;
-    }
-  }
-  const bool other = __shfl_xor((int)bad, 1, 64) != 0;
-  if (won && w == 0 && (bad || other)) {
-    r->ok = REC_CONTAINED;
-    skipped[k] += 1;
-    atomicAdd(stats + ST_CONTAIN, 1u);
-  }
+// Whether node x is a root that a winner other than k moves.  A mark of an
+// earlier chunk may be left at x (k_search takes most of them away): it counts
+// only if its patch is a winner now and moves x.
+__device__ __forceinline__ bool movedByOther(uint32_t m, uint32_t x, uint32_t k, uint32_t K, const PatchRec *recs) {
+  if (m == NONE || m == k || m >= K) return false;
+  const PatchRec *r = recs + m;
+  return r->ok >= REC_CONTAINED && (r->moved[0] == x || r->moved[1] == x);
 }
 
-// Winners write their topology; every patch releases its locks and marks.
-__global__ __launch_bounds__(kPatchBlock) void k_apply(PatchRec *__restrict__ recs, uint32_t K,
-                                                       bvht_BVHNode *__restrict__ nodes, uint64_t *__restrict__ locks,
-                                                       uint32_t *__restrict__ marks, uint32_t *__restrict__ fixStarts,
-                                                       uint32_t *__restrict__ numPending,
-                                                       uint32_t *__restrict__ stats) {
-  const uint32_t k = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes, j = threadIdx.x % kPatchLanes;
-  if (k >= K) return;
-  if (k == 0 && j == 0) *numPending = 0;
-  PatchRec *r = recs + k;
-  const uint32_t ok = r->ok;  // read by all 16 lanes (of one wave) before lane 0 writes it below
+// Writes patch k's node j (the caller's lane): a winner's topology, released
+// locks, the refit's starts.  Returns whether lane 0 of a patch dropped it (2)
+// or applied it (1).
+__device__ __forceinline__ uint32_t applyPatch(PatchRec *r, uint32_t k, uint32_t j, uint32_t ok, bool bad,
+                                           bvht_BVHNode *__restrict__ nodes, uint64_t *__restrict__ locks,
+                                           uint32_t *__restrict__ fixStarts, uint32_t *__restrict__ skipped) {
   const uint32_t jn = j < (uint32_t)kNNode ? j : 0u;
   const uint32_t n = r->node[jn], parent = r->parent[jn], left = r->left[jn], right = r->right[jn],
-                 isLeft = r->isLeft[jn], fix = r->fix[j < 3 ? j : 0u], moved = r->moved[j & 1];
-  const bool win = ok == REC_WON;
+                 isLeft = r->isLeft[jn], fix = r->fix[j < 3 ? j : 0u];
+  const bool win = ok == REC_WON && !bad;
   if (j < 3) fixStarts[3 * k + j] = win ? fix : NONE;
-  if (ok == REC_NONE) return;
+  if (ok == REC_NONE) return 0;
   if (j < (uint32_t)kNNode && n != NONE) {
     locks[n] = kLockFree;
     if (win) {  // MiniPatch::applyOne -- BVHPatch.hpp:72-80
@@ -1005,11 +1011,123 @@ __global__ __launch_bounds__(kPatchBlock) void k_apply(PatchRec *__restrict__ re
       nodes[n].isLeft = (uint16_t)isLeft;
     }
   }
-  if (j >= 14) marks[moved] = NONE;
-  if (j == 0) {
-    r->ok = REC_NONE;
-    if (win) atomicAdd(stats + ST_APPLIED, 1u);
+  if (j != 0 || ok != REC_WON) return 0;
+  r->ok = win ? REC_APPLIED : REC_CONTAINED;
+  if (!win) skipped[k] += 1;
+  return win ? 1 : 2;
+}
+
+// Drops a winner whose insertion point lies below a node another winner moves;
+// the other winners write their topology, and every patch releases its locks.
+// The paths above the insertion points were walked while the conflicts were
+// resolved (the tree does not change until here), so a patch's marks are one
+// round trip for its 16 lanes, and nothing is read that another patch writes.
+// Per chunk, with a launch for the walks and one to apply before: 627 patches
+// of 1M triangles 12.3 + 4.8 -> 5.1 us, 2,648 of 4.2M 13.7 + 9.9 -> 7.8 us.
+// A path longer than kPathWords leaves it all to one workgroup, which walks
+// every path before it writes anything.
+__global__ __launch_bounds__(kPatchBlock) void k_contain(PatchRec *__restrict__ recs, uint32_t K,
+                                                         bvht_BVHNode *__restrict__ nodes, uint32_t root, uint32_t N,
+                                                         const uint32_t *__restrict__ marks,
+                                                         const uint32_t *__restrict__ paths,
+                                                         const uint32_t *__restrict__ deep, uint64_t *__restrict__ locks,
+                                                         uint32_t *__restrict__ fixStarts,
+                                                         uint32_t *__restrict__ skipped,
+                                                         uint32_t *__restrict__ numPending,
+                                                         uint32_t *__restrict__ stats) {
+  const uint32_t j = threadIdx.x % kPatchLanes, group = threadIdx.x & 63u & ~(kPatchLanes - 1);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *numPending = 0;
+  const uint32_t k = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes;
+  const bool in = k < K;  // every lane stays for the exchanges
+  PatchRec *r = recs + (in ? k : 0);
+  const uint32_t *path = paths + 2 * (size_t)(in ? k : 0) * kPathWords;
+  constexpr uint32_t ROWS = 2;  // of 16 words, of each path, loaded before anything is known
+  uint32_t x[2][ROWS];
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+#pragma unroll
+    for (uint32_t i = 0; i < ROWS; ++i) x[w][i] = path[w * kPathWords + i * kPatchLanes + j];
+  const uint32_t ok = in ? r->ok : (uint32_t)REC_NONE;  // read before lane 0 of the patch writes it
+  if (*deep != 0) {
+    if (blockIdx.x > 0) return;
+    for (uint32_t q = threadIdx.x; q < K; q += kPatchBlock) {  // REC_LOST + 1 .. : decided here
+      if (recs[q].ok != REC_WON) continue;
+      bool bad = false;
+      for (int w = 0; w < 2 && !bad; ++w) {
+        uint32_t at = recs[q].best[w];
+        for (uint32_t steps = 0; steps < N; ++steps) {
+          if (movedByOther(marks[at], at, q, K, recs)) {
+            bad = true;
+            break;
+          }
+          if (at == root) break;
+          at = nodes[at].parent;
+        }
+      }
+      fixStarts[3 * (size_t)q] = bad ? 1 : 0;  // until the patch is applied below
+    }
+    __syncthreads();
+    for (uint32_t q = threadIdx.x / kPatchLanes; q < K; q += kPatchesPerBlock) {
+      const uint32_t okq = recs[q].ok;
+      const bool bad = okq == REC_WON && fixStarts[3 * (size_t)q] != 0;
+      const uint32_t did = applyPatch(recs + q, q, j, okq, bad, nodes, locks, fixStarts, skipped);
+      if (did) atomicAdd(stats + (did == 1 ? ST_APPLIED : ST_CONTAIN), 1u);
+    }
+    return;
   }
+  bool bad = false;
+  if (__ballot(ok == REC_WON) != 0) {
+    uint32_t len[2];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      len[w] = __shfl(x[w][0], 0, kPatchLanes);
+      if (ok != REC_WON) len[w] = 0;
+    }
+    uint32_t m[2][ROWS];
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (uint32_t i = 0; i < ROWS; ++i) {
+        const uint32_t at = i * kPatchLanes + j;
+        m[w][i] = at > 0 && at <= len[w] ? marks[x[w][i]] : NONE;
+      }
+    bool marked = false;
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (uint32_t i = 0; i < ROWS; ++i) {
+        if (m[w][i] == k || m[w][i] >= K) m[w][i] = NONE;
+        marked |= m[w][i] != NONE;
+      }
+    if (marked) {  // their patches' records, all in flight together
+      uint32_t state[2][ROWS], root0[2][ROWS], root1[2][ROWS];
+#pragma unroll
+      for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (uint32_t i = 0; i < ROWS; ++i) {
+          const PatchRec *o = recs + (m[w][i] != NONE ? m[w][i] : k);
+          state[w][i] = o->ok;
+          root0[w][i] = o->moved[0];
+          root1[w][i] = o->moved[1];
+        }
+#pragma unroll
+      for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (uint32_t i = 0; i < ROWS; ++i)
+          bad |= m[w][i] != NONE && state[w][i] >= REC_CONTAINED && (root0[w][i] == x[w][i] || root1[w][i] == x[w][i]);
+    }
+    for (int w = 0; w < 2; ++w)
+      for (uint32_t at = ROWS * kPatchLanes + j; at <= len[w]; at += kPatchLanes) {
+        const uint32_t y = path[w * kPathWords + at];
+        bad |= movedByOther(marks[y], y, k, K, recs);
+      }
+  }
+  bad = ((__ballot(bad) >> group) & 0xFFFFu) != 0;
+  const uint32_t did = in ? applyPatch(r, k, j, ok, bad, nodes, locks, fixStarts, skipped) : 0u;
+  // counted per workgroup: one word takes an atomic every few ns
+  const int applied = __syncthreads_count(did == 1), dropped = __syncthreads_count(did == 2);
+  if (threadIdx.x == 0 && applied) atomicAdd(stats + ST_APPLIED, (uint32_t)applied);
+  if (threadIdx.x == 0 && dropped) atomicAdd(stats + ST_CONTAIN, (uint32_t)dropped);
 }
 
 // ---- targeted refit (kFixTree3, Bittner13CUDA.cu:407-467) ------------------
@@ -1504,7 +1622,7 @@ struct Internal {
   size_t noneWords = 0, stateWords = 0;
   uint64_t *locks = nullptr;
   uint32_t *marks = nullptr, *cnt = nullptr, *refitCnt = nullptr;
-  uint32_t *pending[2] = {nullptr, nullptr}, *numPending = nullptr;
+  uint32_t *pending[2] = {nullptr, nullptr}, *numPending = nullptr, *deep = nullptr, *paths = nullptr;
   uint32_t *fixStarts = nullptr;
   uint64_t *refitSlots = nullptr;  // where two refit walks meet (all zero between launches)
   size_t refitSlotWords = 0;
@@ -1544,6 +1662,7 @@ void carveState(Internal *in, size_t &words) {
   in->skipped = take(in->K);
   in->stats = take(ST_WORDS);
   in->numPending = take(1);
+  in->deep = take(1);
   words = off;
 }
 
@@ -1688,6 +1807,7 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
             devMalloc(reinterpret_cast<void **>(&in->sortScratch), sortScratchBytes(in->plan), "bn13 sort") &&
             devAlloc(&in->recs, batchSize, "bn13 patches") && devAlloc(&in->state, in->stateWords, "bn13 state") &&
             devAlloc(&in->pending[0], (1 + kOpenWords) * (size_t)batchSize, "bn13 pending") && devAlloc(&in->pending[1], batchSize, "bn13 pending") &&
+            devAlloc(&in->paths, 2 * kPathWords * (size_t)batchSize, "bn13 paths") &&
             devAlloc(&in->selCounts, selBlocks, "bn13 select") && devAlloc(&in->partials, kSahBlocks, "bn13 SAH");
   if (!ok) {
     freeMemory(&m);
@@ -1714,6 +1834,7 @@ void freeMemory(bvht_GPUWorkingMemory *data) {
     devFree(in->state);
     devFree(in->pending[0]);
     devFree(in->pending[1]);
+    devFree(in->paths);
     devFree(in->selCounts);
     devFree(in->partials);
     devFree(in->feat);
@@ -1927,22 +2048,25 @@ void bn13_rmAndReinsChunk(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer
   // word is cleared with the sort state at the next selection)
   k_search<false><<<K, 64, 0, stream()>>>(bvh->nodes, in->root, in->N, in->sorted, in->inner, in->numInner, chunk,
                                           cfg.numChunks, K, cfg.offsetAccess ? 1u : 0u, cfg.altFindNode ? 1u : 0u,
-                                          in->recs, in->locks, in->stats, sinkOf(in),
+                                          in->recs, in->locks, in->marks, in->stats, sinkOf(in),
                                           chunk == 0 ? in->sortScratch + in->plan.errOff : nullptr);
   if (!checkLaunch("k_search")) return;
-  k_commitFirst<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped, in->stats,
-                                                     in->pending[0], in->numPending);
+  k_commitFirst<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped,
+                                                                          in->stats, in->pending[0], in->numPending,
+                                                                          in->deep);
   if (!checkLaunch("k_commitFirst")) return;
-  k_resolveTail<<<1, kTailBlock, 0, stream()>>>(in->recs, in->locks, in->marks, in->skipped, in->stats, in->pending[0],
-                                                in->pending[0] + kOpenWords * (size_t)in->K, in->pending[1],
-                                                in->numPending);
+  // one wave of walks a workgroup (a CU each: its LDS is the tail's) while the
+  // CUs take them all, else whole workgroups
+  const uint32_t walkers = divUp(2ull * K, 64) < (uint32_t)numCUs() ? 64 : kTailBlock;
+  k_resolveTail<<<1 + divUp(2ull * K, walkers), kTailBlock, 0, stream()>>>(
+      in->recs, in->locks, in->marks, in->skipped, in->stats, in->pending[0],
+      in->pending[0] + kOpenWords * (size_t)in->K, in->pending[1], in->numPending, K, bvh->nodes, in->root, in->paths,
+      walkers, in->deep);
   if (!checkLaunch("k_resolveTail")) return;
-  k_contain<<<divUp(K, kContainBlock / 2), kContainBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->root, in->N, in->marks, in->skipped,
-                                                 in->stats);
+  k_contain<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->root, in->N, in->marks,
+                                                                      in->paths, in->deep, in->locks, in->fixStarts,
+                                                                      in->skipped, in->numPending, in->stats);
   if (!checkLaunch("k_contain")) return;
-  k_apply<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->locks, in->marks, in->fixStarts,
-                                               in->numPending, in->stats);
-  if (!checkLaunch("k_apply")) return;
   refitFrom(in, bvh, in->fixStarts, 3 * K, false);
 }
 
@@ -2078,8 +2202,8 @@ bool bvht_bn13_probe(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bvh
   }
   if (!features(in, bvh)) return false;
   k_search<true><<<num, 64, 0, stream()>>>(bvh->nodes, in->root, in->N, devPositions, in->inner, in->numInner, 0, 1,
-                                          num, 0u, cfg.altFindNode ? 1u : 0u, in->recs, in->locks, in->stats,
-                                          sinkOf(in), nullptr);
+                                          num, 0u, cfg.altFindNode ? 1u : 0u, in->recs, in->locks, in->marks,
+                                          in->stats, sinkOf(in), nullptr);
   return checkLaunch("k_search (probe)");
 }
 

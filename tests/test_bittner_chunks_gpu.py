@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from test_bittner_gpu import replay_check
+from test_features_numbering_gpu import chain
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +55,24 @@ def test_refit_from_leaf_lists(bvh, orc, count):
     assert L.bvht_fixTreeFrom(ctypes.byref(mem), ctypes.byref(tree.ptr), d_starts.ptr, 1)
     L.doCudaDevSync()
     assert tree.download().tobytes() == want.tobytes()
+
+
+# Trees of one path: the nodes above an insertion point fit its stored path (127), or one workgroup
+# checks every patch of the chunk.
+@pytest.mark.parametrize("leaves", [40, 126, 127, 128, 129, 130, 700])
+def test_deep_trees_equal_replay(bvh, orc, leaves):
+    nodes = chain(bvh, leaves)
+    steps, chunks, percent = 3, 2, 12.0
+    rc, _, _, _, trees = orc.bittner_gpuref(nodes, percent, chunks, steps, search=1, chunk_trees=True)
+    assert rc == 0
+    tree = bvh.DeviceBVH.from_host(nodes)
+    opt = bvh.Bittner13GPU(maxNumStepps=steps, numChunks=chunks, batchPercent=percent)
+    opt.setup(tree, leaves)
+    cfg, L = opt.cfg(opt.chunk), bvh.lib()
+    for s in range(steps):
+        L.bn13_selectNodes(ctypes.byref(opt.mem), ctypes.byref(tree.ptr), cfg)
+        for c in range(chunks):
+            L.bn13_rmAndReinsChunk(ctypes.byref(opt.mem), ctypes.byref(tree.ptr), cfg, c)
+            assert tree.download().tobytes() == trees[s * chunks + c].tobytes(), (s, c)
+    st = opt.stats()
+    assert bvh.last_error() == "" and st["applied"] > 0 and st["unresolved"] == 0 and st["runaway"] == 0
