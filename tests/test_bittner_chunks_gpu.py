@@ -6,6 +6,7 @@ import pytest
 
 from test_bittner_gpu import replay_check
 from test_features_numbering_gpu import chain
+from test_mlp_gpu import features_ref
 
 pytestmark = pytest.mark.gpu
 
@@ -76,3 +77,24 @@ def test_deep_trees_equal_replay(bvh, orc, leaves):
             assert tree.download().tobytes() == trees[s * chunks + c].tobytes(), (s, c)
     st = opt.stats()
     assert bvh.last_error() == "" and st["applied"] > 0 and st["unresolved"] == 0 and st["runaway"] == 0
+
+
+# Node and leaf lists whose lengths lie at the edges of a wave (64 items) and of a block (4,096).
+@pytest.mark.parametrize("n", [2, 31, 32, 33, 2047, 2048, 2049, 4096, 4097, 10000])
+def test_ordered_selections(bvh, orc, n):
+    v, f = bvh.scene_soup(n, n)
+    mesh = bvh.DeviceMesh(v, f)
+    tree = bvh.lbvh_build(mesh)
+    nodes = tree.download()
+    opt = bvh.Bittner13GPU(maxNumStepps=1, numChunks=1, batchPercent=75.0)
+    opt.setup(tree, n)
+    ids = bvh.DeviceBuffer(4 * n)
+    num = ctypes.c_uint32()
+    leaves = np.nonzero(nodes["isLeafFlag"] != 0)[0]
+    for begin in (0, 1, n // 2, n - 1, n):
+        bvh.lib().selectDynamicLeafNodes(ctypes.byref(opt.mem), ctypes.byref(tree.ptr), ids.ptr, ctypes.byref(num), begin)
+        assert bvh.last_error() == ""
+        want = leaves[nodes["left"][leaves] >= begin]
+        assert num.value == len(want) and np.array_equal(ids.download(np.uint32, num.value), want)
+    ref = features_ref(nodes)  # by inner node id
+    assert np.allclose(opt.features(tree), ref, rtol=1e-5, atol=1e-6)
