@@ -1666,7 +1666,7 @@ struct Internal {
   uint32_t *leafCnt = nullptr;
   float *subSA = nullptr;
   bool subValid = false;  // leafCnt/subSA match the tree (kept by the refit)
-  uint32_t *anc[2] = {nullptr, nullptr}, *dep[2] = {nullptr, nullptr};
+  unsigned long long *up = nullptr;  // computeDepth's pairs; computeSubtree's list before
   PriorityModel *model = nullptr;
   float *recFeat = nullptr, *recGain = nullptr;
   uint32_t *recCount = nullptr;
@@ -1700,19 +1700,18 @@ bool features(Internal *in, const bvht_CUDAMemoryBVHPointer *bvh) {
   if (!in->feat) {
     if (!devAlloc(&in->feat, (size_t)in->numInner * kFeat, "bn13 features") ||
         !devAlloc(&in->leafCnt, in->N, "bn13 leaf counts") || !devAlloc(&in->subSA, in->N, "bn13 subtree SA") ||
-        !devAlloc(&in->anc[0], in->N, "bn13 ancestors") || !devAlloc(&in->anc[1], in->N, "bn13 ancestors") ||
-        !devAlloc(&in->dep[0], in->N, "bn13 depths") || !devAlloc(&in->dep[1], in->N, "bn13 depths"))
+        !devAlloc(&in->up, in->N, "bn13 depths"))
       return false;
   }
   if (!in->subValid) {
-    if (!computeSubtree(bvh->nodes, in->N, in->leaves, in->numLeaves, in->leafCnt, in->subSA, in->refitCnt, in->anc[0],
-                        in->anc[1]))
+    uint32_t *list = reinterpret_cast<uint32_t *>(in->up);
+    if (!computeSubtree(bvh->nodes, in->N, in->leaves, in->numLeaves, in->leafCnt, in->subSA, in->refitCnt, list,
+                        list + in->N))
       return false;
     in->subValid = true;
   }
-  const int d = computeDepth(bvh->nodes, in->N, in->root, in->anc, in->dep);
-  if (d < 0) return false;
-  return computeFeatures(bvh->nodes, in->N, in->root, in->inner, in->numInner, in->leafCnt, in->subSA, in->dep[d],
+  if (!computeDepth(bvh->nodes, in->N, in->root, in->inner, in->numInner, in->up)) return false;
+  return computeFeatures(bvh->nodes, in->N, in->root, in->inner, in->numInner, in->leafCnt, in->subSA, in->up,
                          in->feat);
 }
 
@@ -1871,10 +1870,7 @@ void freeMemory(bvht_GPUWorkingMemory *data) {
     devFree(in->feat);
     devFree(in->leafCnt);
     devFree(in->subSA);
-    for (int b = 0; b < 2; ++b) {
-      devFree(in->anc[b]);
-      devFree(in->dep[b]);
-    }
+    devFree(in->up);
     devFree(in->recFeat);
     devFree(in->recGain);
     devFree(in->recCount);
