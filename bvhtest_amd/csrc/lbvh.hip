@@ -166,50 +166,24 @@ __global__ __launch_bounds__(kBoxBlock) void k_sceneBox(const bvht_vec3 *__restr
 // and every block of the next kernel reduces all partials itself.
 // Block reduction of per-thread boxes; thread 0 writes partials[blockIdx.x].
 __device__ void writeBoxPartial(const float mn[3], const float mx[3], float *__restrict__ partials) {
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   __shared__ float s_red[6][kBoxBlock / 64];
-  for (int a = 0; a < 3; ++a) {
-    const float x = waveMin(mn[a]), y = waveMax(mx[a]);
-    if (lane == 0) {
-      s_red[a][wave] = x;
-      s_red[3 + a][wave] = y;
-    }
-  }
-  __syncthreads();
-  if (tid < 6) {
-    float x = s_red[tid][0];
-    for (uint32_t w = 1; w < blockDim.x / 64; ++w) x = tid < 3 ? mergeMin(x, s_red[tid][w]) : mergeMax(x, s_red[tid][w]);
-    partials[blockIdx.x * 6 + tid] = x;
-  }
+  float box[6];
+  blockBox(mn, mx, s_red, box);
+  if (threadIdx.x == 0)
+    for (int a = 0; a < 6; ++a) partials[blockIdx.x * 6 + a] = box[a];
 }
 
 // Union of `count` partial boxes (written by an earlier kernel), starting
 // from the all-zero box; every thread of the block receives it.
 __device__ void readBoxPartials(const float *__restrict__ partials, uint32_t count, float box[6]) {
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   __shared__ float s_red[6][kBoxBlock / 64];
-  __shared__ float s_box[6];
   float mn[3] = {0.0f, 0.0f, 0.0f}, mx[3] = {0.0f, 0.0f, 0.0f};
-  for (uint32_t b = tid; b < count; b += blockDim.x)
+  for (uint32_t b = threadIdx.x; b < count; b += blockDim.x)
     for (int a = 0; a < 3; ++a) {
       mn[a] = mergeMin(mn[a], partials[b * 6 + a]);
       mx[a] = mergeMax(mx[a], partials[b * 6 + 3 + a]);
     }
-  for (int a = 0; a < 3; ++a) {
-    const float x = waveMin(mn[a]), y = waveMax(mx[a]);
-    if (lane == 0) {
-      s_red[a][wave] = x;
-      s_red[3 + a][wave] = y;
-    }
-  }
-  __syncthreads();
-  if (tid < 6) {
-    float x = s_red[tid][0];
-    for (uint32_t w = 1; w < blockDim.x / 64; ++w) x = tid < 3 ? mergeMin(x, s_red[tid][w]) : mergeMax(x, s_red[tid][w]);
-    s_box[tid] = x;
-  }
-  __syncthreads();
-  for (int a = 0; a < 6; ++a) box[a] = s_box[a];
+  blockBox(mn, mx, s_red, box);
 }
 
 // Box of all vertices.  The vertex array is read as 16-byte words (float4

@@ -66,7 +66,7 @@ __device__ void blockBoxAtomics(const float mn[3], const float mx[3], uint32_t *
   __shared__ float s_red[6][kBuildBlock / 64];
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int a = 0; a < 3; ++a) {
-    const float x = waveMin(mn[a]), y = waveMax(mx[a]);
+    const float x = waveMinUniform(mn[a]), y = -waveMinUniform(-mx[a]);  // no NaN: fminf and fmaxf drop them
     if (lane == 0) {
       s_red[a][wave] = x;
       s_red[3 + a][wave] = y;

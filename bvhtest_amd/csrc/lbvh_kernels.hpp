@@ -27,6 +27,31 @@ __device__ __forceinline__ void shiftedBox(float mn[3], float mx[3]) {
   }
 }
 
+// The union of a workgroup's boxes, in every thread (no NaN; a zero's sign may
+// change).  DPP steps, and every wave reduces the waves' boxes itself: shuffles
+// and a serial loop over the waves took 36 LDS round trips and 16 more, twice
+// in the key pass (builds of 65k / 1M / 4.2M triangles 54.6 / 135.6 / 365.5 us
+// against 48.5 / 129 / 355.5).
+template <int WAVES>
+__device__ __forceinline__ void blockBox(const float mn[3], const float mx[3], float (&s_red)[6][WAVES], float box[6]) {
+  static_assert((WAVES & (WAVES - 1)) == 0 && WAVES <= 64, "a lane per wave");
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float lo = waveMinUniform(mn[a]), hi = -waveMinUniform(-mx[a]);
+    if (lane == 0) {
+      s_red[a][wave] = lo;
+      s_red[3 + a][wave] = hi;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    box[a] = waveMinUniform(s_red[a][lane & (WAVES - 1)]);
+    box[3 + a] = -waveMinUniform(-s_red[3 + a][lane & (WAVES - 1)]);
+  }
+}
+
 // LBVH_calcMortonCodes host part (LBVH_CUDA.cu:171-180), f32, IEEE division.
 __device__ __forceinline__ void mortonMapping(const float box[6], bvht_vec3 &off, bvht_vec3 &sc) {
   off = {0.0f - box[0], 0.0f - box[1], 0.0f - box[2]};

@@ -55,21 +55,8 @@ __global__ __launch_bounds__(kSmallBlock) void k_smallSort(const bvht_vec3 *__re
     mx[2] = fmaxf(mx[2], fmaxf(fmaxf(a.z, b.z), d.z));
   }
   shiftedBox(mn, mx);
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {  // no NaN: fminf and fmaxf drop them
-    const float lo = waveMinUniform(mn[a]), hi = -waveMinUniform(-mx[a]);
-    if (lane == 0) {
-      s_red[a][wave] = lo;
-      s_red[3 + a][wave] = hi;
-    }
-  }
-  __syncthreads();
   float box[6];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    box[a] = waveMinUniform(s_red[a][lane & (kSmallWaves - 1)]);
-    box[3 + a] = -waveMinUniform(-s_red[3 + a][lane & (kSmallWaves - 1)]);
-  }
+  blockBox(mn, mx, s_red, box);
   bvht_vec3 off, sc;
   mortonMapping(box, off, sc);
   if (tid == 0) {
