@@ -503,11 +503,7 @@ __global__ __launch_bounds__(kWideBlock, 8) void k_segOnesweepWide(
   // published at once (inclusive for the mesh's first tile)
   uint32_t count = 0;
   if (tid < R) {
-    for (int w = 0; w < WAVES; ++w) {
-      const uint32_t c = s_wave[w][tid];
-      s_wave[w][tid] = count;
-      count += c;
-    }
+    count = waveOffsets<WAVES, (ITEMS <= 8)>(s_wave, tid);
     storeRelaxedAgent(status + (size_t)g * R + tid, (lt == 0 ? kSegFlagInc : kSegFlagAgg) | count);
   }
   // exclusive scans over the digits: of the tile's counts and of the mesh's

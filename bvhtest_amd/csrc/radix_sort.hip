@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kSortBlock, 3) void k_onesweep(const K *__restrict_
   __shared__ uint32_t s_wave[WAVES][kSortRadix];
   __shared__ uint32_t s_bstart[kSortRadix];
   __shared__ uint32_t s_gstart[kSortRadix];
-  __shared__ uint32_t s_scan[WAVES];
+  __shared__ uint32_t s_scan[2 * WAVES];
   __shared__ uint32_t s_tile;
   // staging for the scatter: the keys, then the values in the same words,
   // so a 64-bit tile takes 32 KiB of LDS and four workgroups fit on a CU
@@ -113,8 +113,8 @@ __global__ __launch_bounds__(kSortBlock, 3) void k_onesweep(const K *__restrict_
   }
   uint32_t *st = status + (size_t)tile * kSortRadix + tid;
   storeRelaxedAgent(st, (tile == 0 ? kFlagInc : kFlagAgg) | total);
-  const uint32_t hbase = blockExclusiveScan<kSortBlock>(hist[tid], s_scan);
-  const uint32_t bstart = blockExclusiveScan<kSortBlock>(total, s_scan);
+  uint32_t hbase = hist[tid], bstart = total;
+  blockExclusiveScan2<kSortBlock>(hbase, bstart, s_scan);
   s_bstart[tid] = bstart;
   __syncthreads();
 
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__
   __shared__ uint32_t s_wave[WAVES][kSortRadix];  // per-wave digit counters, then prefix partials
   __shared__ uint32_t s_bstart[kSortRadix];
   __shared__ uint32_t s_gstart[kSortRadix];
-  __shared__ uint32_t s_scan[WAVES];
+  __shared__ uint32_t s_scan[2 * WAVES];
   __shared__ K s_buf[TILE];  // the staged keys, then the values in the same words
 
   const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -295,19 +295,20 @@ __global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__
   // published at once
   uint32_t total = 0;
   if (tid < kSortRadix) {
-    for (int w = 0; w < WAVES; ++w) {
-      const uint32_t c = s_wave[w][tid];
-      s_wave[w][tid] = total;
-      total += c;
-    }
+    total = waveOffsets<WAVES, (ITEMS <= 8)>(s_wave, tid);
     // two digits per word: 15-bit counts (at most 17,408
     // keys in a tile), each half flagged when published
-    const uint32_t odd = __shfl_xor(total, 1, 64);  // waves 0..3, all lanes
+    const uint32_t odd = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)total, 0xB1, 0xF, 0xF, false);  // the neighbour's
     if ((tid & 1u) == 0)
       storeRelaxedAgent(status + (size_t)tile * kWideStatusWords + tid / 2, kHalfFlags | total | (odd << 16));
   }
-  const uint32_t hbase = blockExclusiveScan<BLOCK>(histDigit, s_scan);
-  const uint32_t bstart = blockExclusiveScan<BLOCK>(total, s_scan);
+  uint32_t hbase = histDigit, bstart = total;
+  if constexpr (ITEMS <= 12) {
+    blockExclusiveScan2<BLOCK>(hbase, bstart, s_scan);
+  } else {  // one after the other: no registers for both
+    hbase = blockExclusiveScan<BLOCK>(hbase, s_scan);
+    bstart = blockExclusiveScan<BLOCK>(bstart, s_scan);
+  }
   if (tid < kSortRadix) s_bstart[tid] = bstart;
   __syncthreads();
 
