@@ -213,6 +213,14 @@ __global__ __launch_bounds__(256) void k_packNodes(const bvht_BVHNode *__restric
   }
 }
 
+// Rays of a wave that all have the same signs (most tiles of an image) are
+// walked by a loop made for them (OCT: the signs, x y z in bits 0 1 2): the near
+// and far planes of a box are then named instead of selected, 12 of about 75
+// instructions of a visit (primary rays, 1080p over 4.2M triangles 3.21 ->
+// 3.15 ms, a 1024x1024 image of 65k 245 -> 234 us).  kAnyOct: any signs.  (Scalar
+// loads where all of a wave's rays are at one node lost: 3.27 ms and 262 us.)
+constexpr int kAnyOct = 8;
+
 // A ray in registers; sx, sy, sz are its sign flags.
 struct WalkRay {
   bvht_vec3 pos, dir, inv;
@@ -226,11 +234,14 @@ __device__ __forceinline__ WalkRay walkRay(const bvht_Ray &r) {
 // (0.01, t1).  The reference starts from x and takes y and z where they
 // compare greater (near) or smaller (far): a NaN there is ignored, as max and
 // min do, and a NaN in x makes the box missed, which the ordered compare adds.
+template <int OCT>
 __device__ __forceinline__ bool hitBox6(float mnx, float mny, float mnz, float mxx, float mxy, float mxz,
                                         const WalkRay &r, float t1, float &tmin) {
-  const float nx = ((r.sx ? mxx : mnx) - r.pos.x) * r.inv.x, fx = ((r.sx ? mnx : mxx) - r.pos.x) * r.inv.x;
-  const float ny = ((r.sy ? mxy : mny) - r.pos.y) * r.inv.y, fy = ((r.sy ? mny : mxy) - r.pos.y) * r.inv.y;
-  const float nz = ((r.sz ? mxz : mnz) - r.pos.z) * r.inv.z, fz = ((r.sz ? mnz : mxz) - r.pos.z) * r.inv.z;
+  const bool sx = OCT == kAnyOct ? r.sx : (OCT & 1) != 0, sy = OCT == kAnyOct ? r.sy : (OCT & 2) != 0,
+             sz = OCT == kAnyOct ? r.sz : (OCT & 4) != 0;
+  const float nx = ((sx ? mxx : mnx) - r.pos.x) * r.inv.x, fx = ((sx ? mnx : mxx) - r.pos.x) * r.inv.x;
+  const float ny = ((sy ? mxy : mny) - r.pos.y) * r.inv.y, fy = ((sy ? mny : mxy) - r.pos.y) * r.inv.y;
+  const float nz = ((sz ? mxz : mnz) - r.pos.z) * r.inv.z, fz = ((sz ? mnz : mxz) - r.pos.z) * r.inv.z;
   tmin = fmaxf(fmaxf(nx, ny), nz);
   const float tmax = fminf(fminf(fx, fy), fz);
   return !__builtin_isunordered(nx, fx) & (tmin < fminf(tmax, t1)) & (tmax > 0.01f);
@@ -290,13 +301,14 @@ __device__ __forceinline__ bool walkPop(Walk &s, const uint32_t *stk) {
 // The two children of an inner node: which one is entered now and which one
 // waits (kNoChild: none).
 constexpr uint32_t kNoChild = 0xFFFFFFFEu;
+template <int OCT>
 __device__ __forceinline__ void innerChildren(const NodeRec *r, const WalkRay &ray, float t1, uint32_t &now,
                                               uint32_t &later) {
   const float4 a = r->a, b = r->b, c = r->c;
   const uint2 d = *reinterpret_cast<const uint2 *>(&r->d);
   float minL, minR;
-  const bool hl = hitBox6(a.x, a.y, a.z, a.w, b.x, b.y, ray, t1, minL);
-  const bool hr = hitBox6(b.z, b.w, c.x, c.y, c.z, c.w, ray, t1, minR);
+  const bool hl = hitBox6<OCT>(a.x, a.y, a.z, a.w, b.x, b.y, ray, t1, minL);
+  const bool hr = hitBox6<OCT>(b.z, b.w, c.x, c.y, c.z, c.w, ray, t1, minR);
   const bool both = hl & hr, left = hl & (!hr | (minL < minR));
   now = (hl | hr) ? (left ? d.x : d.y) : kNoChild;
   later = both ? (left ? d.y : d.x) : kNoChild;
@@ -304,9 +316,10 @@ __device__ __forceinline__ void innerChildren(const NodeRec *r, const WalkRay &r
 
 // Visits an inner node; false: the walk has ended or gone past the stack.
 // `stk` is this lane's column of a [kStackCap][64] LDS array.
+template <int OCT>
 __device__ __forceinline__ bool visitInner(Walk &s, const WalkRay &ray, const TraceCtx &cx, uint32_t *stk) {
   uint32_t now, later;
-  innerChildren(cx.recs + s.ref, ray, s.t1, now, later);
+  innerChildren<OCT>(cx.recs + s.ref, ray, s.t1, now, later);
   s.count++;
   if (later != kNoChild) {
     if (s.sp >= (uint32_t)kStackCap) {
@@ -361,10 +374,10 @@ __device__ __forceinline__ bool visitLeaf(Walk &s, const WalkRay &ray, const Tra
 }
 
 // One step of a wave's walks.  `active` lanes have a node to visit.
-template <int MODE>
+template <int MODE, int OCT>
 __device__ __forceinline__ void walkStep(bool &active, Walk &s, const WalkRay &ray, const TraceCtx &cx,
                                          float tMin, uint32_t skip, uint32_t *stk) {
-  if (active && (s.ref & kLeafRef) == 0) active = visitInner(s, ray, cx, stk);
+  if (active && (s.ref & kLeafRef) == 0) active = visitInner<OCT>(s, ray, cx, stk);
   if (active && (s.ref & kLeafRef) != 0) active = visitLeaf<MODE>(s, ray, cx, tMin, skip, stk);
 }
 
@@ -387,7 +400,7 @@ __device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx 
       leafTest<MODE>(s, ray, cx, tMin, skip);
     } else {
       uint32_t now, later;
-      innerChildren(cx.recs + s.ref, ray, s.t1, now, later);
+      innerChildren<kAnyOct>(cx.recs + s.ref, ray, s.t1, now, later);
       s.count++;
       if (now != kNoChild) {
         hi = (hi << 1) | (lo >> 63);
@@ -422,6 +435,16 @@ __device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx 
   return TraceOut{s.tri, s.nearest, (uint16_t)s.count};
 }
 
+template <int MODE, int OCT>
+__device__ __forceinline__ void walkLoop(bool active, Walk &s, const WalkRay &ray, const TraceCtx &cx, float tMin,
+                                         uint32_t skip, uint32_t *stk) {
+  for (uint32_t it = 1;; ++it) {
+    if (__ballot(active) == 0) break;
+    walkStep<MODE, OCT>(active, s, ray, cx, tMin, skip, stk);
+    if ((it & (kCheckSteps - 1)) == 0 && s.count >= kMaxSteps) active = false;
+  }
+}
+
 // Walks one ray per lane to its end (every lane of the wave calls).
 template <int MODE>
 __device__ __forceinline__ TraceOut walkAll(bool active, const bvht_Ray &r, const TraceCtx &cx, uint32_t root,
@@ -431,10 +454,21 @@ __device__ __forceinline__ TraceOut walkAll(bool active, const bvht_Ray &r, cons
   Walk s;
   walkReset(s, top);
   active = active && root < cx.bound;
-  for (uint32_t it = 1;; ++it) {
-    if (__ballot(active) == 0) break;
-    walkStep<MODE>(active, s, ray, cx, tMin, skip, stk);
-    if ((it & (kCheckSteps - 1)) == 0 && s.count >= kMaxSteps) active = false;
+  const uint64_t act = __ballot(active);
+  const uint64_t nx = __ballot(active && ray.sx), ny = __ballot(active && ray.sy), nz = __ballot(active && ray.sz);
+  uint32_t oct = kAnyOct;
+  if ((nx == 0 || nx == act) && (ny == 0 || ny == act) && (nz == 0 || nz == act))
+    oct = (nx != 0 ? 1 : 0) | (ny != 0 ? 2 : 0) | (nz != 0 ? 4 : 0);
+  switch (oct) {  // wave-uniform
+    case 0: walkLoop<MODE, 0>(active, s, ray, cx, tMin, skip, stk); break;
+    case 1: walkLoop<MODE, 1>(active, s, ray, cx, tMin, skip, stk); break;
+    case 2: walkLoop<MODE, 2>(active, s, ray, cx, tMin, skip, stk); break;
+    case 3: walkLoop<MODE, 3>(active, s, ray, cx, tMin, skip, stk); break;
+    case 4: walkLoop<MODE, 4>(active, s, ray, cx, tMin, skip, stk); break;
+    case 5: walkLoop<MODE, 5>(active, s, ray, cx, tMin, skip, stk); break;
+    case 6: walkLoop<MODE, 6>(active, s, ray, cx, tMin, skip, stk); break;
+    case 7: walkLoop<MODE, 7>(active, s, ray, cx, tMin, skip, stk); break;
+    default: walkLoop<MODE, kAnyOct>(active, s, ray, cx, tMin, skip, stk); break;
   }
   if (s.sp > (uint32_t)kStackCap) return slowWalk<MODE>(ray, cx, top, tMin, skip);
   return TraceOut{s.tri, s.nearest, (uint16_t)s.count};
@@ -507,9 +541,9 @@ __global__ __launch_bounds__(64) void k_traceImageBundle(const bvht_Ray *__restr
         const NodeRec pp = cx.recs[node];
         float minL = 0.0f, minR = 0.0f;
         const bool hl =
-            valid && hitBox6(pp.a.x, pp.a.y, pp.a.z, pp.a.w, pp.b.x, pp.b.y, wr, nearest + 0.01f, minL);
+            valid && hitBox6<kAnyOct>(pp.a.x, pp.a.y, pp.a.z, pp.a.w, pp.b.x, pp.b.y, wr, nearest + 0.01f, minL);
         const bool hr =
-            valid && hitBox6(pp.b.z, pp.b.w, pp.c.x, pp.c.y, pp.c.z, pp.c.w, wr, nearest + 0.01f, minR);
+            valid && hitBox6<kAnyOct>(pp.b.z, pp.b.w, pp.c.x, pp.c.y, pp.c.z, pp.c.w, wr, nearest + 0.01f, minR);
         const bool anyL = __ballot(hl) != 0, anyR = __ballot(hr) != 0;
         if (anyL || anyR) {
           hi = (hi << 1) | (lo >> 63);
@@ -654,7 +688,7 @@ __global__ __launch_bounds__(64) void k_traceRaysDyn(const bvht_Ray *__restrict_
       continue;
     }
     const bool was = active;
-    walkStep<MODE>(active, s, ray, cx, tMin, skipTri, stk);
+    walkStep<MODE, kAnyOct>(active, s, ray, cx, tMin, skipTri, stk);
     if ((it & (kCheckSteps - 1)) == 0 && s.count >= kMaxSteps) active = false;
     if (was && !active) {
       TraceOut o = {s.tri, s.nearest, (uint16_t)s.count};

@@ -85,3 +85,22 @@ def test_leaves_of_several_triangles(bvh, orc, most):
     d[:400] = np.eye(3, dtype=np.float32)[rng.integers(0, 3, 400)] * rng.choice([-1, 1], (400, 1)).astype(np.float32)
     pos[:600] -= d[:600] * np.float32(0.5)
     check(bvh, orc, nodes, 0, v, f, make_rays(bvh, pos, d))
+
+
+# Whole waves of rays with the same signs, in every octant, and a wave with one ray that differs.
+@pytest.mark.parametrize("octant", range(8))
+def test_waves_of_one_octant(bvh, orc, octant):
+    v, f = bvh.scene_spheres_soup(16, 2000, 77)
+    nodes = orc.lbvh(v, f)[2]
+    rng = np.random.default_rng(octant)
+    sign = np.float32([-1 if octant >> k & 1 else 1 for k in range(3)])
+    lo, hi = v.min(0), v.max(0)
+    d = (rng.random((640, 3), np.float32) + np.float32(0.05)) * sign
+    d[192:256] *= np.float32([0, 1, 1])  # along a plane: zeros of one sign, infinite inverses
+    pos = (lo + hi) / 2 - d * np.float32(2) + (rng.random((640, 3), np.float32) - np.float32(0.5)) * (hi - lo)
+    rays = make_rays(bvh, pos.astype(np.float32), d)
+    rays[100]["dir"] *= -1
+    rays[100]["invDir"] *= -1
+    rays["sign"] = rays["invDir"] < 0
+    hits = check(bvh, orc, nodes, 0, v, f, rays)
+    assert (hits["triId"] != 0xFFFFFFFF).any()
