@@ -11,7 +11,7 @@
 //               bound over the patched view (the reference's findNode1 keeps
 //               a 4096-entry heap per thread in local memory); the patch
 //               reserves its nodes (round 1);
-//     k_commitFirst / k_resolveTail  deterministic reservations: exactly the
+//     k_commit / k_resolveTail  deterministic reservations: exactly the
 //               patches a rank-ordered first-come locking applies (the
 //               reference's kCheckConflicts, timing-dependent there);
 //               (beside them, the paths above the insertion points are walked);
@@ -661,7 +661,7 @@ __device__ uint32_t decide(PatchRec *r, uint32_t k, uint32_t round, uint64_t *lo
 // lane j holds node j, so the patch's node ids, their locks and the writes
 // are one round trip each instead of ten in a row (a chunk has a few hundred
 // to a few thousand patches, far too few to hide a chain of loads per
-// thread).  1M triangles, 627 patches: k_commitFirst 13.3 -> 4.8 us,
+// thread).  1M triangles, 627 patches: round 1 13.3 -> 4.8 us,
 // writing the topology 11.1 -> 4.8 us (a launch of its own then).
 constexpr uint32_t kPatchLanes = 16, kPatchBlock = 256, kPatchesPerBlock = kPatchBlock / kPatchLanes;
 
@@ -669,25 +669,39 @@ constexpr uint32_t kPatchLanes = 16, kPatchBlock = 256, kPatchesPerBlock = kPatc
 // rank and the roots it moves, one word per lane.
 constexpr uint32_t kOpenWords = kPatchLanes, kOpenRank = 12, kOpenMoved = 13;
 static_assert(kNNode <= (int)kOpenRank, "a patch's nodes lie below its rank");
+constexpr uint32_t kCommitRounds = 3;  // k_commit launches of a chunk at most, an open list's length each
 
-// Round 1 over every patch (the reservations were made by k_search).
-__global__ __launch_bounds__(kPatchBlock) void k_commitFirst(PatchRec *__restrict__ recs, uint32_t K, uint64_t *locks,
-                                                             uint32_t *__restrict__ marks,
-                                                             uint32_t *__restrict__ skipped,
-                                                             uint32_t *__restrict__ stats,
-                                                             uint32_t *__restrict__ open,
-                                                             uint32_t *__restrict__ numPending,
-                                                             uint32_t *__restrict__ deep) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *deep = 0;
-  const uint32_t k = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes, j = threadIdx.x % kPatchLanes;
-  const bool in = k < K;  // every lane stays for the ballots
-  PatchRec *r = recs + (in ? k : 0);
-  const uint32_t ok = in ? r->ok : (uint32_t)REC_NONE;
-  const uint32_t n = in && j < (uint32_t)kNNode ? r->node[j] : NONE;
+// Round 1 over every patch (the reservations were made by k_search), or, LATER,
+// a further round over the entries that the one before left.  With `again` the
+// undecided patches reserve their nodes for the next round at once: a patch
+// that meets such a reservation in place of its own is only decided a round
+// later.
+template <bool LATER>
+__global__ __launch_bounds__(kPatchBlock) void k_commit(PatchRec *__restrict__ recs, uint32_t K, uint64_t *locks,
+                                                        uint32_t *__restrict__ marks, uint32_t *__restrict__ skipped,
+                                                        uint32_t *__restrict__ stats, const uint32_t *__restrict__ openIn,
+                                                        const uint32_t *__restrict__ numIn,
+                                                        uint32_t *__restrict__ open, uint32_t *__restrict__ numPending,
+                                                        uint32_t round, bool again, uint32_t *__restrict__ deep) {
+  if (!LATER && blockIdx.x == 0 && threadIdx.x == 0) *deep = 0;
+  const uint32_t at = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes, j = threadIdx.x % kPatchLanes;
+  const bool in = at < (LATER ? *numIn : K);  // every lane stays for the ballots
   const bool mover = j == kOpenMoved || j == kOpenMoved + 1;
-  const uint32_t moved = in && mover ? r->moved[j - kOpenMoved] : NONE;
-  const bool undecided = ok == REC_PENDING, use = undecided && n != NONE;
-  const uint64_t mine = lockKey(1, k);
+  uint32_t k = at, n, moved;
+  bool undecided = in;
+  if (LATER) {
+    const uint32_t word = in ? openIn[(size_t)at * kOpenWords + j] : NONE;
+    k = __shfl(word, kOpenRank, kPatchLanes);
+    n = j < (uint32_t)kNNode ? word : NONE;
+    moved = word;
+  } else {
+    PatchRec *r = recs + (in ? at : 0);
+    n = in && j < (uint32_t)kNNode ? r->node[j] : NONE;
+    moved = in && mover ? r->moved[j - kOpenMoved] : NONE;
+    undecided = in && r->ok == REC_PENDING;
+  }
+  const bool use = undecided && n != NONE;
+  const uint64_t mine = lockKey(round, k);
   const uint64_t v = use ? __hip_atomic_load(locks + n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : mine;
   const uint32_t group = threadIdx.x & 63u & ~(kPatchLanes - 1);
   const bool lost = ((__ballot((v >> 32) == 0) >> group) & 0xFFFFu) != 0;  // node of an applied patch
@@ -697,22 +711,24 @@ __global__ __launch_bounds__(kPatchBlock) void k_commitFirst(PatchRec *__restric
     if (use)
       atomicMin(reinterpret_cast<unsigned long long *>(locks + n), (unsigned long long)lockKey(kRoundWin, k));
     if (mover) marks[moved] = k;  // moved roots are patch nodes: one applied patch each
-    if (j == 0) r->ok = REC_WON;
+    if (j == 0) recs[k].ok = REC_WON;
   } else if (lost) {
     if (j == 0) {
-      r->ok = REC_LOST;
+      recs[k].ok = REC_LOST;
       skipped[k] += 1;
       atomicAdd(stats + ST_CONFLICT, 1u);
     }
   } else {
+    if (again && use)
+      atomicMin(reinterpret_cast<unsigned long long *>(locks + n), (unsigned long long)lockKey(round + 1, k));
     uint32_t slot = 0;
     if (j == 0) slot = atomicAdd(numPending, 1u);
     slot = __shfl(slot, 0, kPatchLanes);
-    open[slot * kOpenWords + j] = j == kOpenRank ? k : mover ? moved : n;
+    open[(size_t)slot * kOpenWords + j] = j == kOpenRank ? k : mover ? moved : n;
   }
 }
 
-// Rounds 2.. over the (few) undecided patches, in one workgroup.  At most
+// The further rounds over the (few) undecided patches, in one workgroup.  At most
 // `num + 1` rounds are needed; patches still undecided after that bound
 // (never, unless memory ordering is broken) are dropped and counted.
 //
@@ -722,7 +738,7 @@ __global__ __launch_bounds__(kPatchBlock) void k_commitFirst(PatchRec *__restric
 // it (round 1's from its global lock, read once) and the lowest rank
 // reserving it this round, and each thread keeps its patches' table slots in
 // registers.  The table is built by 16 lanes a patch, from the entries that
-// k_commitFirst left (a line each): a node a lane, every load and every first
+// k_commit left (a line each): a node a lane, every load and every first
 // probe of a thread in flight together (one thread a patch, node by node from
 // its record: 22.0 against 13.3 us before the first round with 772 patches,
 // 7.2 against 4.7 with 50).  A round is two barriers: a patch with a taken node loses, the
@@ -790,7 +806,8 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
                                                            uint32_t *listB, const uint32_t *__restrict__ numPending,
                                                            uint32_t K, const bvht_BVHNode *__restrict__ nodes,
                                                            uint32_t root, uint32_t *__restrict__ paths,
-                                                           uint32_t walkers, uint32_t *__restrict__ deep) {
+                                                           uint32_t walkers, uint32_t *__restrict__ deep,
+                                                           uint32_t firstRound) {
   // lowest reserving rank per slot, rounds alternate; at first [1] holds the
   // node ids and [0] the patches' slots (16 bits each)
   __shared__ __align__(16) uint32_t s_min[2][kTailSlots];
@@ -807,7 +824,7 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
   static_assert(kTailSlots <= 65535 && kTailCap * kNNode * 2 <= sizeof(s_min[0]), "the slots fit s_min[0]");
   uint32_t num = *numPending;
   if (num == 0) return;
-  const uint32_t maxRound = num + 2;
+  const uint32_t maxRound = num + firstRound;
   if (num <= kTailCap) {
     // 16 lanes per patch: a lane loads one node of each of up to kTailTrips
     // patches and its lock, all in flight together, and inserts it
@@ -957,7 +974,7 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
   for (uint32_t i = threadIdx.x; i < num; i += kTailBlock) listA[i] = open[i * kOpenWords + kOpenRank];
   __syncthreads();
   uint32_t *cur = listA, *nxt = listB;
-  for (uint32_t round = 2; num > 0 && round <= maxRound; ++round) {
+  for (uint32_t round = firstRound; num > 0 && round <= maxRound; ++round) {
     for (uint32_t i = threadIdx.x; i < num; i += kTailBlock) reserve(recs + cur[i], cur[i], round, locks);
     if (threadIdx.x == 0) s_cnt = 0;
     __syncthreads();
@@ -1036,7 +1053,7 @@ __global__ __launch_bounds__(kPatchBlock) void k_contain(PatchRec *__restrict__ 
                                                          uint32_t *__restrict__ numPending,
                                                          uint32_t *__restrict__ stats) {
   const uint32_t j = threadIdx.x % kPatchLanes, group = threadIdx.x & 63u & ~(kPatchLanes - 1);
-  if (blockIdx.x == 0 && threadIdx.x == 0) *numPending = 0;
+  if (blockIdx.x == 0 && threadIdx.x < kCommitRounds) numPending[threadIdx.x] = 0;
   const uint32_t k = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes;
   const bool in = k < K;  // every lane stays for the exchanges
   PatchRec *r = recs + (in ? k : 0);
@@ -1691,7 +1708,7 @@ void carveState(Internal *in, size_t &words) {
   in->refitCnt = take(in->N);
   in->skipped = take(in->K);
   in->stats = take(ST_WORDS);
-  in->numPending = take(1);
+  in->numPending = take(kCommitRounds);
   in->deep = take(1);
   words = off;
 }
@@ -1835,7 +1852,7 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
             devAlloc(&in->vals[0], in->numInner, "bn13 vals") && devAlloc(&in->vals[1], in->numInner, "bn13 vals") &&
             devMalloc(reinterpret_cast<void **>(&in->sortScratch), sortScratchBytes(in->plan), "bn13 sort") &&
             devAlloc(&in->recs, batchSize, "bn13 patches") && devAlloc(&in->state, in->stateWords, "bn13 state") &&
-            devAlloc(&in->pending[0], (1 + kOpenWords) * (size_t)batchSize, "bn13 pending") && devAlloc(&in->pending[1], batchSize, "bn13 pending") &&
+            devAlloc(&in->pending[0], (1 + kOpenWords) * (size_t)batchSize, "bn13 pending") && devAlloc(&in->pending[1], (1 + kOpenWords) * (size_t)batchSize, "bn13 pending") &&
             devAlloc(&in->paths, 2 * kPathWords * (size_t)batchSize, "bn13 paths") &&
             devAlloc(&in->selBits, (kSelWords + 1) * (size_t)selBlocks, "bn13 select") && devAlloc(&in->partials, kSahBlocks, "bn13 SAH");
   if (!ok) {
@@ -2057,6 +2074,19 @@ void bn13_selectNodes(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bv
   in->selected = true;
 }
 
+// Rounds over the whole GPU before the rest goes to one workgroup, which takes
+// about 20 us for 800 undecided patches and more than its LDS holds much worse;
+// a round costs a launch, 5 us.  Many patches, or many for the tree, leave enough
+// of them.  Per chunk, us, with 1 / 2 / 3 rounds: K = 386 of N = 154k nodes
+// 88.9 / 90.4 / 91.2, 965 of 154k 107.6 / 106.2 / 107.2, 1,134 of 1.8M
+// 109.5 / 111.9 / 114.4, 2,269 of 1.8M 129.1 / 125.3 / 127.1, 5,105 of 8.2M
+// 201 / 188 / 190, 10,210 of 8.2M 440 / 301 / 306, 11,349 of 1.8M 669 / 355 / 278.
+static uint32_t commitRounds(uint32_t K, uint32_t N) {
+  if (K >= 4096 && K >= N / 256) return 3;
+  return K >= 2048 || (K >= 768 && K >= N / 512) ? 2 : 1;
+}
+static_assert(kCommitRounds >= 3, "a list length for every round");
+
 void bn13_rmAndReinsChunk(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bvh, bvht_AlgoCFG cfg, uint32_t chunk) {
   Internal *in = inOf(data);
   if (!in || !validBVH(bvh, "bn13_rmAndReinsChunk")) return;
@@ -2077,17 +2107,26 @@ void bn13_rmAndReinsChunk(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer
                                           in->recs, in->locks, in->marks, in->stats, sinkOf(in),
                                           chunk == 0 ? in->sortScratch + in->plan.errOff : nullptr);
   if (!checkLaunch("k_search")) return;
-  k_commitFirst<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped,
-                                                                          in->stats, in->pending[0], in->numPending,
-                                                                          in->deep);
-  if (!checkLaunch("k_commitFirst")) return;
+  const uint32_t commitBlocks = divUp(K, kPatchesPerBlock), rounds = commitRounds(K, in->N);
+  k_commit<false><<<commitBlocks, kPatchBlock, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped, in->stats,
+                                                              nullptr, nullptr, in->pending[0], in->numPending, 1u,
+                                                              rounds > 1, in->deep);
+  if (!checkLaunch("k_commit")) return;
+  for (uint32_t r = 2; r <= rounds; ++r) {
+    k_commit<true><<<commitBlocks, kPatchBlock, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped, in->stats,
+                                                               in->pending[r & 1], in->numPending + r - 2,
+                                                               in->pending[(r & 1) ^ 1], in->numPending + r - 1, r,
+                                                               r < rounds, in->deep);
+    if (!checkLaunch("k_commit")) return;
+  }
+  const size_t lists = kOpenWords * (size_t)in->K;  // behind the open entries: room for k_resolveTail's lists
   // one wave of walks a workgroup (a CU each: its LDS is the tail's) while the
   // CUs take them all, else whole workgroups
   const uint32_t walkers = divUp(2ull * K, 64) < (uint32_t)numCUs() ? 64 : kTailBlock;
   k_resolveTail<<<1 + divUp(2ull * K, walkers), kTailBlock, 0, stream()>>>(
-      in->recs, in->locks, in->marks, in->skipped, in->stats, in->pending[0],
-      in->pending[0] + kOpenWords * (size_t)in->K, in->pending[1], in->numPending, K, bvh->nodes, in->root, in->paths,
-      walkers, in->deep);
+      in->recs, in->locks, in->marks, in->skipped, in->stats, in->pending[(rounds & 1) ^ 1],
+      in->pending[0] + lists, in->pending[1] + lists, in->numPending + rounds - 1, K, bvh->nodes, in->root, in->paths,
+      walkers, in->deep, rounds + 1);
   if (!checkLaunch("k_resolveTail")) return;
   k_contain<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->root, in->N, in->marks,
                                                                       in->paths, in->deep, in->locks, in->fixStarts,

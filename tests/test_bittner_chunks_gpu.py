@@ -20,6 +20,16 @@ def test_conflict_rounds_equal_replay(bvh, orc, percent):
     replay_check(bvh, orc, v, f, 2, 1, percent, search=1)
 
 
+# Chunks with one, two and three rounds over the whole GPU (767 and 768 patches, 4,095 and 4,096), and one
+# that leaves more undecided patches than the workgroup's table holds.
+@pytest.mark.parametrize("grid,percent", [((48, 40), 9.993), ((48, 40), 10.008), ((128, 64), 12.499), ((128, 64), 12.503),
+                                          ((256, 128), 20.0)])
+def test_round_counts_equal_replay(bvh, orc, grid, percent):
+    v, f = bvh.scene_heightfield(*grid, 53, 0.2)
+    print(f"K={int(np.float32(percent) / np.float32(100.0) * np.float32(2 * len(f) - 1))}", flush=True)
+    replay_check(bvh, orc, v, f, 1, 1, percent, search=1)
+
+
 # Refits from lists of leaves: one walk, a workgroup's edge (256), more than the
 # meeting places of one launch (a quarter of the leaves), all leaves, all of
 # them twice over and some inner nodes among them.
