@@ -11,11 +11,14 @@
 //                only the face indices when the topology does not need keys.
 //   k_buildLevel0 tiles of 2^kTileLog positions: gathers each sorted
 //                triangle, writes the leaf, reduces the tile's subtree
-//                (wave shuffles, then LDS) and writes each inner node once
+//                (lane exchanges, then LDS) and writes each inner node once
 //                (box, topology, SA) from the lane of its index;
 //   k_buildLevelUp further launches reduce the tile roots in LDS.
 // The reference topology is a closed form of n (see types.hpp), so no key is
 // read to build it and no global atomic is needed for the refit.
+// The full build takes the box from the vertices instead (k_vertBox, checked
+// by k_mortonFix), and meshes of up to 8,192 triangles take box, keys and sort
+// in one workgroup (lbvh_small.hip).
 #include "lbvh.hpp"
 #include "lbvh_kernels.hpp"
 #include "lbvh_small.hpp"

@@ -275,8 +275,8 @@ bool bvht_sortKeyIndexPairs(const void *keys, uint32_t n, uint32_t keyBits, uint
                             uint32_t *valsOut);
 /* Per-kernel device times (ms, HIP events on the library stream) of the last
  * bvht_LBVH_build when timing is on; bvht_LBVH_stageName(i) names kernel i
- * (k_sceneBox, k_morton or k_mortonMsd, the sort's kernels, k_buildLevel0,
- * k_buildLevelUp).
+ * (k_smallSort, or k_vertBox or k_sceneBox, k_morton, k_mortonFix or
+ * k_mortonMsd and the sort's kernels; then k_buildLevel0, k_buildLevelUp).
  * Returns the number of entries written. */
 void bvht_LBVH_setTiming(bool enable);
 /* With group on, the onesweep digit passes of a timed build are one entry,
