@@ -131,7 +131,10 @@ constexpr int kStackCap = 24;  // pending children per lane: 6 KiB of LDS a wave
 // 1080p over 4.2M triangles, 685, 600, 608, 602 us at 512x512 over 65k (beyond
 // 20 the waves displace each other's records from the L1).
 constexpr uint32_t kTraceWavesPerCU = 20;
-constexpr uint32_t kRefillAt = 16;  // idle lanes that make a k_traceRaysDyn wave fetch rays
+// Idle lanes that make a k_traceRaysDyn wave fetch rays.  8, 12, 16, 24, 32, 48: 4.37,
+// 3.97, 3.98, 3.93, 3.94, 4.03 ms at 1080p over 4.2M triangles, 622, 612, 601, 585,
+// 575, 554 us at 1024x1024 over 65k.
+constexpr uint32_t kRefillAt = 32;
 
 // One node's record.  A child index at or past `bound` becomes an empty leaf
 // (a reference past the records) and raises *bad (the traversal then never
