@@ -4,7 +4,8 @@
 // Every segment's output equals the standalone build of that mesh (own scene
 // box, local face and node indices): the reference build of
 // lib/builder/LBVH_CUDA.cu applied per mesh.  Stages:
-//   k_segInit    zeroes the sort scratch, initialises the mesh boxes;
+//   k_segInit    zeroes the sort scratch, initialises the mesh boxes, once:
+//                every build's level 0 leaves them so for the next;
 //   k_segVertBox per run of one mesh's vertices: block reduce, 6 atomic
 //                min/max (order-preserving u32 encoding) into the mesh's
 //                vertex box (the reference's triangle box once shifted by
@@ -46,10 +47,7 @@ namespace {
 // second pair shifted (f32 rounding is monotone); the keys are made from
 // the first, which equals it unless an unreferenced vertex lies outside
 // the triangles' box, and k_segFix repairs such meshes.
-constexpr int kBoxWords = 12;
 constexpr uint32_t kVertChunk = 4096;  // vertices per k_segVertBox workgroup
-
-__device__ __forceinline__ uint32_t boxInitWord(uint32_t w) { return (w % 6) < 3 ? f2o(HUGE_VALF) : f2o(-HUGE_VALF); }
 
 // The reference's box from a raw vertex min / max pair (6 words at w):
 // -+FLT_EPSILON, then the origin.
@@ -84,16 +82,10 @@ __device__ void blockBoxAtomics(const float mn[3], const float mx[3], uint32_t *
   }
 }
 
-// Zeroes the sort scratch and initialises the per-mesh boxes (one launch).
-__global__ void k_segInit(uint32_t *__restrict__ scratch, size_t scratchWords, uint32_t *__restrict__ boxOrd,
-                          size_t boxWords) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < scratchWords + boxWords;
-       i += (size_t)gridDim.x * blockDim.x) {
-    if (i < scratchWords)
-      scratch[i] = 0;
-    else
-      boxOrd[i - scratchWords] = boxInitWord((uint32_t)((i - scratchWords) % kBoxWords));
-  }
+// The state as every build needs it: before the first, and after one that did
+// not launch all of its kernels.
+__global__ void k_segInit(BatchState state) {
+  clearBatchState(state, blockIdx.x * (size_t)blockDim.x + threadIdx.x, (size_t)gridDim.x * blockDim.x);
 }
 
 // Min / max of a run of up to kVertChunk vertices of one mesh (vchunks:
@@ -127,6 +119,7 @@ constexpr int kSegWideSizes = 5;
 // against 2.57), or 2^10, one trip, while those are at most four workgroups
 // per CU (64 meshes, 700k triangles: 107.8 us against 109.8; 2^9: 113)
 constexpr int kChunkLog = 11, kChunkLogSmall = 10;
+constexpr int kSegHistWord = 16;                            // first histogram word of the sort scratch
 constexpr int kSegMaxHist = 3 * 1024;                       // passes x radix, both digit widths
 constexpr uint32_t kSegFlagAgg = 1u << 30, kSegFlagInc = 2u << 30, kSegCountMask = (1u << 30) - 1;
 
@@ -154,6 +147,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_segMorton(const bvht_vec3 *__re
   static_assert(P * R <= kSegMaxHist, "histogram fits the LDS array");
   __shared__ uint32_t s_hist[P * R];
   for (int i = threadIdx.x; i < P * R; i += kBuildBlock) s_hist[i] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) segHist[(int)kSegErrWord - kSegHistWord] = 0;  // of this build from here on
   const uint2 c = chunks[blockIdx.x];
   const SegDesc sd = segs[c.x];
   bvht_vec3 off, sc;
@@ -648,6 +642,7 @@ struct BatchInternal {
   uint32_t *keys[2] = {nullptr, nullptr};
   uint32_t *vals[2] = {nullptr, nullptr};
   float2 *rec = nullptr;  // leaf box per triangle (three float2), written by k_segMorton
+  bool dirty = false;     // a build stopped half way: the state has to be cleared first
   int radixBits = 8;
   uint2 *chunks = nullptr;     // (mesh, chunk) of the Morton pass
   uint32_t numChunks = 0;
@@ -661,7 +656,8 @@ struct BatchInternal {
   int wideItems = 0;  // keys per thread of those tiles
   // sort scratch: [0, 16) pass counters + error word, then the mesh
   // histograms / prefixes (M x passes x radix), then the look-back status
-  // (passes x sort tiles x radix); all of it is zeroed before every build
+  // (passes x sort tiles x radix); all of it but the error word is zero
+  // between builds
   uint32_t *sortScratch = nullptr;
   size_t histWords = 0, statusWords = 0;
   hipStream_t capStream = nullptr;
@@ -701,7 +697,7 @@ bool useWideSegSort(const BatchInternal *in) { return in->radixBits == 8 && in->
 template <int RB>
 bool segSort(BatchInternal *in, int &result) {
   constexpr int R = 1 << RB, P = segPasses(RB);
-  uint32_t *counters = in->sortScratch, *hist = in->sortScratch + 16;
+  uint32_t *counters = in->sortScratch, *hist = in->sortScratch + kSegHistWord;
   uint32_t *status = hist + (size_t)in->M * P * R;
   const bool wide = RB == 8 && useWideSegSort(in);  // the wide passes scan the counts themselves
   if (!wide) {
@@ -716,7 +712,7 @@ bool segSort(BatchInternal *in, int &result) {
         k_segOnesweepWide<decltype(items)::value><<<in->numWideTiles, kWideBlock, 0, stream()>>>(
             in->keys[cur], pass == 0 ? nullptr : in->vals[cur], last ? nullptr : in->keys[cur ^ 1], in->vals[cur ^ 1],
             in->wideTiles, in->segs, in->totalFaces, (uint32_t)(pass * RB), hist + (size_t)pass * R, P,
-            status + (size_t)pass * in->numWideTiles * R, counters + pass, counters + 15);
+            status + (size_t)pass * in->numWideTiles * R, counters + pass, counters + kSegErrWord);
       };
       switch (in->wideItems) {
         case 1: launch(std::integral_constant<int, 1>()); break;
@@ -732,7 +728,7 @@ bool segSort(BatchInternal *in, int &result) {
     k_segOnesweep<RB><<<in->numSortTiles, kSortBlock, 0, stream()>>>(
         in->keys[cur], pass == 0 ? nullptr : in->vals[cur], last ? nullptr : in->keys[cur ^ 1], in->vals[cur ^ 1],
         in->sortTiles, in->segs, (uint32_t)(pass * RB), hist + (size_t)pass * R, P,
-        status + (size_t)pass * in->numSortTiles * R, counters + pass, counters + 15);
+        status + (size_t)pass * in->numSortTiles * R, counters + pass, counters + kSegErrWord);
     if (!checkLaunch("k_segOnesweep")) return false;
     cur ^= 1;
   }
@@ -740,15 +736,30 @@ bool segSort(BatchInternal *in, int &result) {
   return true;
 }
 
+bool streamCapturing() {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream(), &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+// Clears the whole state.
+bool clearState(BatchInternal *in) {
+  const BatchState all = {in->sortScratch, in->boxOrd, kSegHistWord + in->histWords + in->statusWords,
+                          (size_t)kBoxWords * in->M};
+  const uint32_t blocks = (uint32_t)std::min<size_t>(divUp(all.scratchWords + all.boxWords, 256), (size_t)numCUs() * 8);
+  k_segInit<<<blocks, 256, 0, stream()>>>(all);
+  return checkLaunch("k_segInit");
+}
+
 template <int TLOG>
 bool batchStagesT(BatchInternal *in, const bvht_vec3 *vert, const bvht_Triangle *faces, bvht_BVHNode *nodes) {
   const int P = segPasses(in->radixBits), R = 1 << in->radixBits;
   const uint32_t sortTiles = useWideSegSort(in) ? in->numWideTiles : in->numSortTiles;
-  const size_t scratchWords = 16 + (size_t)in->M * P * R + (size_t)P * sortTiles * R;
-  const size_t boxWords = (size_t)kBoxWords * in->M;
-  const uint32_t initBlocks = (uint32_t)std::min<size_t>(divUp(scratchWords + boxWords, 256), (size_t)numCUs() * 8);
-  k_segInit<<<initBlocks, 256, 0, stream()>>>(in->sortScratch, scratchWords, in->boxOrd, boxWords);
-  if (!checkLaunch("k_segInit")) return false;
+  // every build leaves the words that it used clear (k_buildLevel0)
+  const BatchState state = {in->sortScratch, in->boxOrd, kSegHistWord + (size_t)in->M * P * R + (size_t)P * sortTiles * R,
+                            (size_t)kBoxWords * in->M};
+  const bool recorded = in->dirty && streamCapturing();  // a graph that may never run clears nothing for the next build
+  if (in->dirty && !clearState(in)) return false;
+  in->dirty = true;
   if (in->numVChunks) {
     k_segVertBox<<<in->numVChunks, kBuildBlock, 0, stream()>>>(vert, in->vchunks, in->boxOrd);
     if (!checkLaunch("k_segVertBox")) return false;
@@ -756,21 +767,24 @@ bool batchStagesT(BatchInternal *in, const bvht_vec3 *vert, const bvht_Triangle 
   int r = 0;
   if (in->radixBits == 10) {
     k_segMorton<10><<<in->numChunks, kBuildBlock, 0, stream()>>>(vert, faces, in->segs, in->chunks, in->boxOrd,
-                                                                 in->keys[0], in->rec, in->sortScratch + 16, in->chunkLog);
+                                                                 in->keys[0], in->rec, in->sortScratch + kSegHistWord, in->chunkLog);
     if (!checkLaunch("k_segMorton")) return false;
     k_segFix<10><<<in->numChunks, kBuildBlock, 0, stream()>>>(vert, faces, in->segs, in->chunks, in->boxOrd,
-                                                              in->keys[0], in->sortScratch + 16, in->chunkLog);
+                                                              in->keys[0], in->sortScratch + kSegHistWord, in->chunkLog);
     if (!checkLaunch("k_segFix") || !segSort<10>(in, r)) return false;
   } else {
     k_segMorton<8><<<in->numChunks, kBuildBlock, 0, stream()>>>(vert, faces, in->segs, in->chunks, in->boxOrd,
-                                                                in->keys[0], in->rec, in->sortScratch + 16, in->chunkLog);
+                                                                in->keys[0], in->rec, in->sortScratch + kSegHistWord, in->chunkLog);
     if (!checkLaunch("k_segMorton")) return false;
     k_segFix<8><<<in->numChunks, kBuildBlock, 0, stream()>>>(vert, faces, in->segs, in->chunks, in->boxOrd,
-                                                             in->keys[0], in->sortScratch + 16, in->chunkLog);
+                                                             in->keys[0], in->sortScratch + kSegHistWord, in->chunkLog);
     if (!checkLaunch("k_segFix") || !segSort<8>(in, r)) return false;
   }
-  return launchTreeLevelsBatch(TLOG, nodes, in->vals[r], faces, vert, in->rec, in->segs, in->tiles.data(),
-                               in->tileCounts.data(), (int)in->tiles.size());
+  if (!launchTreeLevelsBatch(TLOG, nodes, in->vals[r], faces, vert, in->rec, in->segs, in->tiles.data(),
+                               in->tileCounts.data(), (int)in->tiles.size(), state))
+    return false;
+  in->dirty = recorded;
+  return true;
 }
 
 bool batchStages(BatchInternal *in, const bvht_vec3 *vert, const bvht_Triangle *faces, bvht_BVHNode *nodes) {
@@ -931,8 +945,9 @@ bvht_LBVH_BatchWorkingMemory bvht_LBVH_allocateBatch(uint32_t numMeshes, const u
       !devAlloc(&in->keys[1], in->totalFaces, "batch keys") || !devAlloc(&in->vals[0], in->totalFaces, "batch values") ||
       !devAlloc(&in->vals[1], in->totalFaces, "batch values") ||
       !devAlloc(&in->rec, 3ull * in->totalFaces, "batch leaf boxes") ||
-      !devAlloc(&in->sortScratch, 16 + in->histWords + in->statusWords, "batch sort") ||
-      !fillU32(in->sortScratch, 0u, 16) ||  // the error word reads 0 before the first build
+      !devAlloc(&in->sortScratch, kSegHistWord + in->histWords + in->statusWords, "batch sort") ||
+      !fillU32(in->sortScratch, 0u, kSegHistWord) ||  // the error word reads 0 before the first build
+      !clearState(in) || !check(hipStreamSynchronize(stream()), "batch state") ||
       !check(hipStreamCreateWithFlags(&in->capStream, hipStreamNonBlocking), "batch capture stream")) {
     bvht_LBVH_freeBatch(&m);
     return m;
@@ -1032,7 +1047,7 @@ uint32_t bvht_LBVH_batchStatus(const bvht_LBVH_BatchWorkingMemory *mem) {
   }
   const BatchInternal *in = reinterpret_cast<const BatchInternal *>(mem->internal);
   uint32_t v = 0xFFFFFFFFu;
-  if (!check(hipMemcpyAsync(&v, in->sortScratch + 15, 4, hipMemcpyDeviceToHost, stream()), "bvht_LBVH_batchStatus") ||
+  if (!check(hipMemcpyAsync(&v, in->sortScratch + kSegErrWord, 4, hipMemcpyDeviceToHost, stream()), "bvht_LBVH_batchStatus") ||
       !check(hipStreamSynchronize(stream()), "bvht_LBVH_batchStatus sync"))
     return 0xFFFFFFFFu;
   return v;

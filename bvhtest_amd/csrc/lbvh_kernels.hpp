@@ -134,6 +134,24 @@ __device__ __forceinline__ float o2f(uint32_t o) {
   return __uint_as_float((o & 0x80000000u) ? (o & 0x7FFFFFFFu) : ~o);
 }
 
+// The sort scratch and mesh boxes of a batched build (lbvh_batch.hip), which
+// every build leaves as the next one needs them: zeroes and empty boxes.
+constexpr int kBoxWords = 12;  // two boxes a mesh, order-preserving words: min, max
+__device__ __forceinline__ uint32_t boxInitWord(uint32_t w) { return (w % 6) < 3 ? f2o(HUGE_VALF) : f2o(-HUGE_VALF); }
+struct BatchState {
+  uint32_t *scratch, *boxOrd;
+  size_t scratchWords, boxWords;
+};
+constexpr uint32_t kSegErrWord = 15;  // of the scratch: kept for the caller to read
+__device__ __forceinline__ void clearBatchState(const BatchState &st, size_t first, size_t stride) {
+  for (size_t i = first; i < st.scratchWords + st.boxWords; i += stride) {
+    if (i >= st.scratchWords)
+      st.boxOrd[i - st.scratchWords] = boxInitWord((uint32_t)((i - st.scratchWords) % kBoxWords));
+    else if (i != kSegErrWord)
+      st.scratch[i] = 0;
+  }
+}
+
 // Inner node whose index is position p of a segment with N1 + 1 leaves
 // (p < N1), in the closed form of the reference topology: an odd p is the
 // last position of a left child (a full aligned block), an even p > 0 the
@@ -241,7 +259,7 @@ template <int TLOG, bool BATCH, bool REC>
 __global__ __launch_bounds__(level0Block(TLOG), (1 << TLOG) > 1024 ? 4 : 8) void k_buildLevel0(
     bvht_BVHNode *__restrict__ nodesAll, const uint32_t *__restrict__ sorted, const bvht_Triangle *__restrict__ faces,
     const bvht_vec3 *__restrict__ vertAll, const float2 *__restrict__ rec, SegDesc single,
-    const SegDesc *__restrict__ segs, const uint2 *__restrict__ tiles) {
+    const SegDesc *__restrict__ segs, const uint2 *__restrict__ tiles, BatchState state) {
   constexpr int BLOCK = level0Block(TLOG);
   constexpr uint32_t T = 1u << TLOG;
   constexpr int R = T / BLOCK;
@@ -267,7 +285,7 @@ __global__ __launch_bounds__(level0Block(TLOG), (1 << TLOG) > 1024 ? 4 : 8) void
   bvht_BVHNode *__restrict__ nodes = nodesAll + sd.nodeBase;
   const bvht_vec3 *__restrict__ vert = vertAll + sd.vertBase;
   const uint32_t u0 = group << TLOG;
-  if (u0 >= n) return;  // block-uniform: a group past the last position owns nothing
+  if (!BATCH && u0 >= n) return;  // block-uniform: a group past the last position owns nothing (a table lists none)
   const uint32_t cnt = min(T, n - u0);
 
   // Every sorted index, face and vertex gather of the thread's leaves is
@@ -383,6 +401,9 @@ __global__ __launch_bounds__(level0Block(TLOG), (1 << TLOG) > 1024 ? 4 : 8) void
     for (int c = 0; c < 6; ++c) b[c] = s_box[at][c];
     storeInner(nodes, l, r, N1, b);
   }
+  // the sort is over: its state is cleared here for the next build (a launch of
+  // its own before every build otherwise: 64 meshes 108.1 us against 104.1)
+  if constexpr (BATCH) clearBatchState(state, blockIdx.x * (size_t)BLOCK + threadIdx.x, (size_t)gridDim.x * BLOCK);
 }
 
 // One upper level of the tile hierarchy.  Units are aligned runs of
@@ -472,6 +493,7 @@ bool launchTreeLevels(int tlog, bvht_BVHNode *nodes, const uint32_t *sorted, con
 // rec (if not null) holds every triangle's leaf box (k_buildLevel0's REC).
 bool launchTreeLevelsBatch(int tlog, bvht_BVHNode *nodes, const uint32_t *sorted, const bvht_Triangle *faces,
                            const bvht_vec3 *vert, const float2 *rec, const SegDesc *segs,
-                           const uint2 *const *tilesPerLevel, const uint32_t *tilesCount, int levels);
+                           const uint2 *const *tilesPerLevel, const uint32_t *tilesCount, int levels,
+                           const BatchState &state);
 
 }  // namespace bvht
