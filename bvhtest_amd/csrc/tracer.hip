@@ -119,7 +119,7 @@ struct TraceOut {
 // One node, 64 bytes.  Inner: a b c hold the left child's box, then the
 // right's (min.xyz max.xyz each), d.x and d.y the children's references.
 // Leaf: a = v0 and the first face, b = e1 = v1 - v0 and the face count,
-// c = e2 = v2 - v0 (of that face).
+// c = e2 = v2 - v0 (of that face).  d.z is 0.
 struct NodeRec {
   float4 a, b, c;
   uint4 d;
@@ -280,12 +280,13 @@ struct Walk {
   uint32_t sp;     // pending children on the stack; kStackCap + 1: one too many, see slowWalk
   uint32_t count;  // inner nodes visited
   uint32_t tri;
+  uint32_t ahead;  // AHEAD: 0, from the children's records, taken at the next visit
   float nearest, t1;  // t1 = nearest + 0.01: boxes beyond are not entered
 };
 
 __device__ __forceinline__ void walkReset(Walk &s, uint32_t rootRef) {
   s.ref = rootRef;
-  s.sp = s.count = 0;
+  s.sp = s.count = s.ahead = 0;
   s.tri = kNoHit;
   s.nearest = s.t1 = HUGE_VALF;
 }
@@ -319,10 +320,22 @@ __device__ __forceinline__ void innerChildren(const NodeRec *r, const WalkRay &r
 
 // Visits an inner node; false: the walk has ended or gone past the stack.
 // `stk` is this lane's column of a [kStackCap][64] LDS array.
-template <int OCT>
+// AHEAD: both children's records are asked for as soon as their references are
+// known, beside the box tests (a word that is 0 in every record, added to the
+// count a visit later), so the one that is visited next is on its way to the
+// L1.  For launches that leave the GPU room, whose time is their longest walk's;
+// see walksAhead.
+template <int OCT, bool AHEAD>
 __device__ __forceinline__ bool visitInner(Walk &s, const WalkRay &ray, const TraceCtx &cx, uint32_t *stk) {
   uint32_t now, later;
-  innerChildren<OCT>(cx.recs + s.ref, ray, s.t1, now, later);
+  const NodeRec *r = cx.recs + s.ref;
+  if constexpr (AHEAD) {
+    const uint2 d = *reinterpret_cast<const uint2 *>(&r->d);
+    const uint32_t before = s.ahead, most = cx.bound - 1;
+    s.ahead = cx.recs[min(d.x & ~kLeafRef, most)].d.z | cx.recs[min(d.y & ~kLeafRef, most)].d.z;
+    s.count += before;
+  }
+  innerChildren<OCT>(r, ray, s.t1, now, later);
   s.count++;
   if (later != kNoChild) {
     if (s.sp >= (uint32_t)kStackCap) {
@@ -377,10 +390,10 @@ __device__ __forceinline__ bool visitLeaf(Walk &s, const WalkRay &ray, const Tra
 }
 
 // One step of a wave's walks.  `active` lanes have a node to visit.
-template <int MODE, int OCT>
+template <int MODE, int OCT, bool AHEAD>
 __device__ __forceinline__ void walkStep(bool &active, Walk &s, const WalkRay &ray, const TraceCtx &cx,
                                          float tMin, uint32_t skip, uint32_t *stk) {
-  if (active && (s.ref & kLeafRef) == 0) active = visitInner<OCT>(s, ray, cx, stk);
+  if (active && (s.ref & kLeafRef) == 0) active = visitInner<OCT, AHEAD>(s, ray, cx, stk);
   if (active && (s.ref & kLeafRef) != 0) active = visitLeaf<MODE>(s, ray, cx, tMin, skip, stk);
 }
 
@@ -438,18 +451,18 @@ __device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx 
   return TraceOut{s.tri, s.nearest, (uint16_t)s.count};
 }
 
-template <int MODE, int OCT>
+template <int MODE, int OCT, bool AHEAD>
 __device__ __forceinline__ void walkLoop(bool active, Walk &s, const WalkRay &ray, const TraceCtx &cx, float tMin,
                                          uint32_t skip, uint32_t *stk) {
   for (uint32_t it = 1;; ++it) {
     if (__ballot(active) == 0) break;
-    walkStep<MODE, OCT>(active, s, ray, cx, tMin, skip, stk);
+    walkStep<MODE, OCT, AHEAD>(active, s, ray, cx, tMin, skip, stk);
     if ((it & (kCheckSteps - 1)) == 0 && s.count >= kMaxSteps) active = false;
   }
 }
 
 // Walks one ray per lane to its end (every lane of the wave calls).
-template <int MODE>
+template <int MODE, bool AHEAD>
 __device__ __forceinline__ TraceOut walkAll(bool active, const bvht_Ray &r, const TraceCtx &cx, uint32_t root,
                                             float tMin, uint32_t skip, uint32_t *stk) {
   const WalkRay ray = walkRay(r);
@@ -463,15 +476,15 @@ __device__ __forceinline__ TraceOut walkAll(bool active, const bvht_Ray &r, cons
   if ((nx == 0 || nx == act) && (ny == 0 || ny == act) && (nz == 0 || nz == act))
     oct = (nx != 0 ? 1 : 0) | (ny != 0 ? 2 : 0) | (nz != 0 ? 4 : 0);
   switch (oct) {  // wave-uniform
-    case 0: walkLoop<MODE, 0>(active, s, ray, cx, tMin, skip, stk); break;
-    case 1: walkLoop<MODE, 1>(active, s, ray, cx, tMin, skip, stk); break;
-    case 2: walkLoop<MODE, 2>(active, s, ray, cx, tMin, skip, stk); break;
-    case 3: walkLoop<MODE, 3>(active, s, ray, cx, tMin, skip, stk); break;
-    case 4: walkLoop<MODE, 4>(active, s, ray, cx, tMin, skip, stk); break;
-    case 5: walkLoop<MODE, 5>(active, s, ray, cx, tMin, skip, stk); break;
-    case 6: walkLoop<MODE, 6>(active, s, ray, cx, tMin, skip, stk); break;
-    case 7: walkLoop<MODE, 7>(active, s, ray, cx, tMin, skip, stk); break;
-    default: walkLoop<MODE, kAnyOct>(active, s, ray, cx, tMin, skip, stk); break;
+    case 0: walkLoop<MODE, 0, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
+    case 1: walkLoop<MODE, 1, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
+    case 2: walkLoop<MODE, 2, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
+    case 3: walkLoop<MODE, 3, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
+    case 4: walkLoop<MODE, 4, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
+    case 5: walkLoop<MODE, 5, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
+    case 6: walkLoop<MODE, 6, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
+    case 7: walkLoop<MODE, 7, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
+    default: walkLoop<MODE, kAnyOct, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
   }
   if (s.sp > (uint32_t)kStackCap) return slowWalk<MODE>(ray, cx, top, tMin, skip);
   return TraceOut{s.tri, s.nearest, (uint16_t)s.count};
@@ -502,6 +515,7 @@ __device__ __forceinline__ uint32_t tileX(uint32_t l) { return (l & 1) | ((l >> 
 __device__ __forceinline__ uint32_t tileY(uint32_t l) { return tileX(l >> 1); }
 
 // Image path: 8x8 pixel tiles per wave (kTraceRay launch shape, CUDAKernels.cu:409-416).
+template <bool AHEAD>
 __global__ __launch_bounds__(64) void k_traceImage(const bvht_Ray *__restrict__ rays,
                                                       bvht_CUDAPixel *__restrict__ img, TraceCtx cx, uint32_t root,
                                                       bvht_vec3 light, uint32_t w, uint32_t h) {
@@ -511,7 +525,7 @@ __global__ __launch_bounds__(64) void k_traceImage(const bvht_Ray *__restrict__ 
   const bool in = x < w && y < h;
   const size_t i = in ? (size_t)y * w + x : 0;
   const bvht_Ray ray = rays[i];
-  const TraceOut o = walkAll<0>(in, ray, cx, root, 0.0f, kNoHit, s_stk + threadIdx.x);
+  const TraceOut o = walkAll<0, AHEAD>(in, ray, cx, root, 0.0f, kNoHit, s_stk + threadIdx.x);
   if (in) img[i] = shade(o, ray, cx.vert, cx.faces, light);
 }
 
@@ -604,7 +618,7 @@ __global__ __launch_bounds__(64) void k_traceImageBundle(const bvht_Ray *__restr
   if (valid) img[(size_t)y * w + x] = shade(o, ray, cx.vert, cx.faces, light);
 }
 
-template <int MODE>
+template <int MODE, bool AHEAD>
 __global__ __launch_bounds__(64) void k_traceRays(const bvht_Ray *__restrict__ rays, uint32_t num, TraceCtx cx,
                                                      uint32_t root, bvht_vec3 light, float tMin,
                                                      const uint32_t *__restrict__ skip, bvht_Hit *__restrict__ hits,
@@ -633,7 +647,7 @@ __global__ __launch_bounds__(64) void k_traceRays(const bvht_Ray *__restrict__ r
   if (!in) i = 0;
   const bvht_Ray ray = rays[i];
   const bool still = ray.dir.x == 0.0f && ray.dir.y == 0.0f && ray.dir.z == 0.0f;
-  const TraceOut o = walkAll<MODE>(in && !still, ray, cx, root, tMin, skip ? skip[i] : kNoHit, s_stk + threadIdx.x);
+  const TraceOut o = walkAll<MODE, AHEAD>(in && !still, ray, cx, root, tMin, skip ? skip[i] : kNoHit, s_stk + threadIdx.x);
   if (!in) return;
   if (hits) hits[i] = bvht_Hit{o.tri, o.t};
   if (img) img[i] = shade(o, ray, cx.vert, cx.faces, light);
@@ -691,7 +705,7 @@ __global__ __launch_bounds__(64) void k_traceRaysDyn(const bvht_Ray *__restrict_
       continue;
     }
     const bool was = active;
-    walkStep<MODE, kAnyOct>(active, s, ray, cx, tMin, skipTri, stk);
+    walkStep<MODE, kAnyOct, false>(active, s, ray, cx, tMin, skipTri, stk);
     if ((it & (kCheckSteps - 1)) == 0 && s.count >= kMaxSteps) active = false;
     if (was && !active) {
       TraceOut o = {s.tri, s.nearest, (uint16_t)s.count};
@@ -883,6 +897,14 @@ bool prepareTrace(const bvht_BVHNode *nodes, const bvht_MeshRaw &mesh, TraceCtx 
   return true;
 }
 
+// Whether a launch of so many waves has its walks load ahead (visitInner): up
+// to ten waves per CU.  Plain against ahead, us, 65k triangles / 0.9M: 1 wave per
+// CU 180 / 658 against 145 / 536, 4 waves 195 / 650 against 166 / 582, 10 waves
+// 202 / 728 against 179 / 712, 18 waves 193 / 746 against 177 / 860, 64 waves
+// 232 / 1,667 against 274 / 2,484 (the L1 is busy then).  Switching to it after a
+// number of steps, or where few of a wave's lanes are left, lost everywhere.
+bool walksAhead(uint64_t waves) { return waves <= (uint64_t)numCUs() * 10; }
+
 // Sorts the rays by k_rayKeys and returns the trace order (nullptr on
 // failure, with the error recorded).
 const uint32_t *rayOrder(const bvht_Ray *rays, uint32_t num, const bvht_BVHNode *nodes, uint32_t root) {
@@ -983,8 +1005,10 @@ void tracerImage(bvht_Ray *rays, bvht_CUDAPixel *img, bvht_BVHNode *nodes, uint3
   dim3 grid(divUp(w, 8), divUp(h, 8));
   if (bundle)
     k_traceImageBundle<<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
+  else if (walksAhead((uint64_t)grid.x * grid.y))
+    k_traceImage<true><<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
   else
-    k_traceImage<<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
+    k_traceImage<false><<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
   checkLaunch(bundle ? "k_traceImageBundle" : "k_traceImage");
 }
 
@@ -1026,8 +1050,13 @@ bool bvht_traceRays(const bvht_Ray *rays, uint32_t num, bvht_BVHNode *nodes, uin
     const TraceCache &c = traceCache();
     const bool image = rays == c.imgRays && (uint64_t)num == (uint64_t)c.imgW * c.imgH;
     const uint32_t blocks = image ? divUp(c.imgW, 8) * divUp(c.imgH, 8) : divUp(num, 64);
-    k_traceRays<0><<<blocks, 64, 0, stream()>>>(rays, num, cx, rootNode, light, tMin, skipTri,
-                                                hits, img, order, image ? c.imgW : 0u);
+    const uint32_t width = image ? c.imgW : 0u;
+    if (walksAhead(blocks))
+      k_traceRays<0, true><<<blocks, 64, 0, stream()>>>(rays, num, cx, rootNode, light, tMin, skipTri, hits, img, order,
+                                                        width);
+    else
+      k_traceRays<0, false><<<blocks, 64, 0, stream()>>>(rays, num, cx, rootNode, light, tMin, skipTri, hits, img, order,
+                                                         width);
     return checkLaunch("k_traceRays");
   }
   // secondary rays: resident waves refill idle lanes (walk lengths vary widely)

@@ -104,3 +104,17 @@ def test_waves_of_one_octant(bvh, orc, octant):
     rays["sign"] = rays["invDir"] < 0
     hits = check(bvh, orc, nodes, 0, v, f, rays)
     assert (hits["triId"] != 0xFFFFFFFF).any()
+
+
+# The last launch whose walks load ahead (2,560 waves on 256 CUs) and the first whose do not, as image and as rays.
+@pytest.mark.parametrize("w,h", [(512, 320), (512, 321), (640, 400)])
+def test_walks_ahead_and_plain(bvh, orc, w, h):
+    v, f = bvh.scene_spheres_soup(16, 2000, 77)
+    mesh = bvh.DeviceMesh(v, f)
+    tree = bvh.lbvh_build(mesh)
+    cam = ((0.5, 0.5, 2.0), (0.5, 0.5, 0.5), (0, 1, 0), 45.0)
+    rays = bvh.generate_rays(w, h, *cam)
+    opix, ohits = orc.trace(rays, tree.download(), 0, v, f)
+    pix, hits = bvh.trace_rays(tree, mesh, rays)
+    assert hits.tobytes() == ohits.tobytes() and pix.tobytes() == opix.tobytes()
+    assert bvh.trace_image(tree, mesh, w, h, *cam).tobytes() == opix.tobytes()
