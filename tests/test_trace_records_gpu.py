@@ -118,3 +118,14 @@ def test_walks_ahead_and_plain(bvh, orc, w, h):
     pix, hits = bvh.trace_rays(tree, mesh, rays)
     assert hits.tobytes() == ohits.tobytes() and pix.tobytes() == opix.tobytes()
     assert bvh.trace_image(tree, mesh, w, h, *cam).tobytes() == opix.tobytes()
+
+
+# Bundles: 12,288 waves on 256 CUs and more.
+@pytest.mark.parametrize("w,h", [(1024, 768), (1024, 776)])
+def test_bundles_ahead_and_plain(bvh, orc, w, h):
+    v, f = bvh.scene_heightfield(64, 32, 5, 0.2)
+    mesh = bvh.DeviceMesh(v, f)
+    tree = bvh.lbvh_build(mesh)
+    cam = ((0.5, 1.0, 1.25), (0.5, 0.1, 0.25), (0, 1, 0), 45.0)
+    opix, _ = orc.trace_bundle(bvh.generate_rays(w, h, *cam), w, h, tree.download(), 0, v, f)
+    assert bvh.trace_image(tree, mesh, w, h, *cam, bundle=True).tobytes() == opix.tobytes()
