@@ -4,8 +4,8 @@
 // Every segment's output equals the standalone build of that mesh (own scene
 // box, local face and node indices): the reference build of
 // lib/builder/LBVH_CUDA.cu applied per mesh.  Stages:
-//   k_segInit    zeroes the sort scratch, initialises the mesh boxes, once:
-//                every build's level 0 leaves them so for the next;
+//   k_segInit    zeroes the sort scratch, initialises the mesh boxes;
+//                then every build leaves them so (level 0);
 //   k_segVertBox per run of one mesh's vertices: block reduce, 6 atomic
 //                min/max (order-preserving u32 encoding) into the mesh's
 //                vertex box (the reference's triangle box once shifted by
@@ -642,7 +642,7 @@ struct BatchInternal {
   uint32_t *keys[2] = {nullptr, nullptr};
   uint32_t *vals[2] = {nullptr, nullptr};
   float2 *rec = nullptr;  // leaf box per triangle (three float2), written by k_segMorton
-  bool dirty = false;     // a build stopped half way: the state has to be cleared first
+  bool dirty = true;      // before the first build, after one that stopped half way: the state has to be cleared
   int radixBits = 8;
   uint2 *chunks = nullptr;     // (mesh, chunk) of the Morton pass
   uint32_t numChunks = 0;
@@ -947,7 +947,6 @@ bvht_LBVH_BatchWorkingMemory bvht_LBVH_allocateBatch(uint32_t numMeshes, const u
       !devAlloc(&in->rec, 3ull * in->totalFaces, "batch leaf boxes") ||
       !devAlloc(&in->sortScratch, kSegHistWord + in->histWords + in->statusWords, "batch sort") ||
       !fillU32(in->sortScratch, 0u, kSegHistWord) ||  // the error word reads 0 before the first build
-      !clearState(in) || !check(hipStreamSynchronize(stream()), "batch state") ||
       !check(hipStreamCreateWithFlags(&in->capStream, hipStreamNonBlocking), "batch capture stream")) {
     bvht_LBVH_freeBatch(&m);
     return m;
@@ -992,6 +991,10 @@ bool bvht_LBVH_buildBatch(bvht_LBVH_BatchWorkingMemory *mem, const bvht_vec3 *ve
   if (!useGraph) return batchStages(in, vert, faces, nodes);
   if (in->exec && (in->capVert != vert || in->capFaces != faces || in->capNodes != nodes)) dropGraph(in);
   if (!in->exec) {
+    if (in->dirty) {  // ahead of the graph, not in it
+      if (!clearState(in)) return false;
+      in->dirty = streamCapturing();
+    }
     hipStream_t user = rt().stream;
     rt().stream = in->capStream;
     bool ok = check(hipStreamBeginCapture(in->capStream, hipStreamCaptureModeThreadLocal), "batch capture");
