@@ -537,7 +537,6 @@ __global__ __launch_bounds__(64) void k_traceImage(const bvht_Ray *__restrict__ 
 // reference's shared-memory flags and reduction.  Every ray still finds its
 // nearest hit (the shared walk covers its own); among triangles at exactly
 // the same distance the first one met may differ from the per-ray order.
-template <bool AHEAD>
 __global__ __launch_bounds__(64) void k_traceImageBundle(const bvht_Ray *__restrict__ rays,
                                                          bvht_CUDAPixel *__restrict__ img, TraceCtx cx, uint32_t root,
                                                          bvht_vec3 light, uint32_t w, uint32_t h) {
@@ -555,13 +554,14 @@ __global__ __launch_bounds__(64) void k_traceImageBundle(const bvht_Ray *__restr
     for (uint32_t steps = 0; steps < (1u << 26); ++steps) {
       const uint32_t node = ref & ~kLeafRef;
       if ((ref & kLeafRef) == 0) {
-        if constexpr (AHEAD) {  // as in visitInner; here it is one address a wave
-          const uint2 d = *reinterpret_cast<const uint2 *>(&cx.recs[node].d);
-          const uint32_t before = ahead, most = cx.bound - 1;
-          ahead = cx.recs[min(d.x & ~kLeafRef, most)].d.z | cx.recs[min(d.y & ~kLeafRef, most)].d.z;
-          o.intCount += before;
-        }
-        o.intCount++;
+        // both children's records are asked for beside the box tests, as in
+        // visitInner; here it is one address a wave, and pays at every size: 65k / 0.9M
+        // triangles, 160x120 1,059 / 2,796 -> 828 / 2,181 us, 640x480 395 / 1,422 ->
+        // 322 / 1,207, 1024x1024 283 / 2,865 -> 277 / 2,532, 1920x1080 290 / 2,614 -> 289 / 2,367
+        const uint2 d = *reinterpret_cast<const uint2 *>(&cx.recs[node].d);
+        const uint32_t before = ahead, most = cx.bound - 1;
+        ahead = cx.recs[min(d.x & ~kLeafRef, most)].d.z | cx.recs[min(d.y & ~kLeafRef, most)].d.z;
+        o.intCount += 1 + before;
         const NodeRec pp = cx.recs[node];
         float minL = 0.0f, minR = 0.0f;
         const bool hl =
@@ -905,16 +905,12 @@ bool prepareTrace(const bvht_BVHNode *nodes, const bvht_MeshRaw &mesh, TraceCtx 
 }
 
 // Whether a launch of so many waves has its walks load ahead (visitInner): up
-// to `perCU` waves per CU.  Rays: plain against ahead, us, 65k triangles / 0.9M: 1 wave per
+// to ten waves per CU.  Plain against ahead, us, 65k triangles / 0.9M: 1 wave per
 // CU 180 / 658 against 145 / 536, 4 waves 195 / 650 against 166 / 582, 10 waves
 // 202 / 728 against 179 / 712, 18 waves 193 / 746 against 177 / 860, 64 waves
 // 232 / 1,667 against 274 / 2,484 (the L1 is busy then).  Switching to it after a
 // number of steps, or where few of a wave's lanes are left, lost everywhere.
-// Bundles (one address a wave): 1 wave 1,059 / 2,796 against 828 / 2,181, 18 waves
-// 395 / 1,422 against 322 / 1,207, 48 waves 326 / 2,240 against 305 / 2,000, 64 waves
-// 280 / 2,870 against 286 / 2,524.
-constexpr uint32_t kAheadRays = 10, kAheadBundles = 48;
-bool walksAhead(uint64_t waves, uint32_t perCU) { return waves <= (uint64_t)numCUs() * perCU; }
+bool walksAhead(uint64_t waves) { return waves <= (uint64_t)numCUs() * 10; }
 
 // Sorts the rays by k_rayKeys and returns the trace order (nullptr on
 // failure, with the error recorded).
@@ -1014,12 +1010,9 @@ void tracerImage(bvht_Ray *rays, bvht_CUDAPixel *img, bvht_BVHNode *nodes, uint3
   TraceCtx cx;
   if (!prepareTrace(nodes, mesh, cx, "tracerImage")) return;
   dim3 grid(divUp(w, 8), divUp(h, 8));
-  const uint64_t waves = (uint64_t)grid.x * grid.y;
-  if (bundle && walksAhead(waves, kAheadBundles))
-    k_traceImageBundle<true><<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
-  else if (bundle)
-    k_traceImageBundle<false><<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
-  else if (walksAhead(waves, kAheadRays))
+  if (bundle)
+    k_traceImageBundle<<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
+  else if (walksAhead((uint64_t)grid.x * grid.y))
     k_traceImage<true><<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
   else
     k_traceImage<false><<<grid, 64, 0, stream()>>>(rays, img, cx, rootNode, light, w, h);
@@ -1065,7 +1058,7 @@ bool bvht_traceRays(const bvht_Ray *rays, uint32_t num, bvht_BVHNode *nodes, uin
     const bool image = rays == c.imgRays && (uint64_t)num == (uint64_t)c.imgW * c.imgH;
     const uint32_t blocks = image ? divUp(c.imgW, 8) * divUp(c.imgH, 8) : divUp(num, 64);
     const uint32_t width = image ? c.imgW : 0u;
-    if (walksAhead(blocks, kAheadRays))
+    if (walksAhead(blocks))
       k_traceRays<0, true><<<blocks, 64, 0, stream()>>>(rays, num, cx, rootNode, light, tMin, skipTri, hits, img, order,
                                                         width);
     else
