@@ -990,11 +990,12 @@ bool bvht_LBVH_buildBatch(bvht_LBVH_BatchWorkingMemory *mem, const bvht_vec3 *ve
   }
   if (!useGraph) return batchStages(in, vert, faces, nodes);
   if (in->exec && (in->capVert != vert || in->capFaces != faces || in->capNodes != nodes)) dropGraph(in);
+  // ahead of the graph, not in it: every replay too may follow a build that stopped half way
+  if (in->dirty) {
+    if (!clearState(in)) return false;
+    in->dirty = streamCapturing();
+  }
   if (!in->exec) {
-    if (in->dirty) {  // ahead of the graph, not in it
-      if (!clearState(in)) return false;
-      in->dirty = streamCapturing();
-    }
     hipStream_t user = rt().stream;
     rt().stream = in->capStream;
     bool ok = check(hipStreamBeginCapture(in->capStream, hipStreamCaptureModeThreadLocal), "batch capture");
@@ -1015,7 +1016,9 @@ bool bvht_LBVH_buildBatch(bvht_LBVH_BatchWorkingMemory *mem, const bvht_vec3 *ve
     in->capFaces = faces;
     in->capNodes = nodes;
   }
-  return check(hipGraphLaunch(in->exec, rt().stream), "batch graph launch");
+  if (check(hipGraphLaunch(in->exec, rt().stream), "batch graph launch")) return true;
+  in->dirty = true;
+  return false;
 }
 
 void bvht_LBVH_freeBatch(bvht_LBVH_BatchWorkingMemory *mem) {

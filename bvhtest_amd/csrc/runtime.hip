@@ -28,6 +28,15 @@ bool check(hipError_t e, const char *what) {
   return false;
 }
 
+bool checkLaunch(const char *what) {
+  Runtime &r = rt();
+  if (r.launchFailAfter > 0 && --r.launchFailAfter == 0) {
+    setError("%s: injected launch failure", what);
+    return false;
+  }
+  return check(hipGetLastError(), what);
+}
+
 bool devMalloc(void **p, size_t bytes, const char *what) {
   *p = nullptr;
   Runtime &r = rt();
@@ -80,6 +89,7 @@ void *bvht_getStream(void) { return rt().stream; }
 const char *bvht_getLastError(void) { return rt().lastError.c_str(); }
 void bvht_clearError(void) { rt().lastError.clear(); }
 void bvht_setAllocFailAfter(int n) { rt().allocFailAfter = n < 0 ? 0 : n; }
+void bvht_setLaunchFailAfter(int n) { rt().launchFailAfter = n < 0 ? 0 : n; }
 const char *bvht_version(void) { return "bvhtest_amd 0.1 (gfx950)"; }
 int bvht_deviceCount(void) {
   int n = 0;

@@ -1,5 +1,5 @@
 // Library runtime: the stream all work goes to, the last-error record, the
-// allocation hook used by host tests, and small launch helpers.
+// failure hooks used by host tests, and small launch helpers.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -16,6 +16,7 @@ struct Runtime {
   hipStream_t stream = nullptr;
   std::string lastError;
   int allocFailAfter = 0;  // 0: off; n: the n-th allocation from now fails
+  int launchFailAfter = 0;  // the same for checked kernel launches
 };
 
 Runtime &rt();
@@ -26,8 +27,8 @@ void setError(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
 
 // Returns true on hipSuccess; otherwise records "<what>: <hip error>".
 bool check(hipError_t e, const char *what);
-// Checks the last kernel launch.
-inline bool checkLaunch(const char *what) { return check(hipGetLastError(), what); }
+// Checks the last kernel launch, honouring the failure-injection hook.
+bool checkLaunch(const char *what);
 
 // Device allocation honouring the failure-injection hook; *p = nullptr on failure.
 bool devMalloc(void **p, size_t bytes, const char *what);

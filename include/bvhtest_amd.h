@@ -136,6 +136,9 @@ void bvht_clearError(void);
 /* Host-test hook: make the n-th device allocation from now fail (n >= 1);
  * 0 disables.  Exercises the CUDA_ERROR paths, e.g. lib/builder/LBVH.cpp:29-35. */
 void bvht_setAllocFailAfter(int n);
+/* The same for kernel launches: the n-th checked launch from now is reported
+ * as failed (its kernel has run), so a call stops half way. */
+void bvht_setLaunchFailAfter(int n);
 /* Library version string and the gfx target it was built for. */
 const char *bvht_version(void);
 /* Number of visible HIP devices (0 when none; never fails). */
