@@ -87,6 +87,7 @@ SIGNATURES = {
     "bvht_clearError": (None, []),
     "bvht_setAllocFailAfter": (None, [ctypes.c_int]),
     "bvht_setLaunchFailAfter": (None, [ctypes.c_int]),
+    "bvht_setSortPolls": (None, [ctypes.c_int]),
     "bvht_version": (ctypes.c_char_p, []),
     "bvht_deviceCount": (ctypes.c_int, []),
     "runMalloc": (c_bool, [P(c_vp), c_size]),

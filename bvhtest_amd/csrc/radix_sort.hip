@@ -230,19 +230,35 @@ __global__ __launch_bounds__(kSortBlock, 3) void k_onesweep(const K *__restrict_
 //    of a chained look-back.  The counts are published two digits to a word
 //    (15 bits each), so a 16-byte load brings eight digits and, with 8 loads
 //    in flight per thread, one round trip covers 64 to 256 predecessors.
-//  - The tile is the workgroup's id.  Workgroups start in id order on each
-//    XCD and a CU holds one of any tile size, so the lowest tile that has not
-//    started yet only waits for tiles that have, and they do not wait for it;
-//    the wait for a count is bounded all the same and raises the error flag.
-//    (Tile ids from an atomic counter: 1.5 to 3.4 us at the start of a pass.)
+//  - The tile is the workgroup's id (ids from an atomic counter took 1.5 to
+//    3.4 us at the start of a pass), so a tile may wait for one that has not
+//    started, as where sorts on several streams or of several processes hold
+//    each other's CUs.  Its wait is bounded: after `polls` looks the thread
+//    counts the missing tile's digits from the pass's input itself, so every
+//    workgroup ends whatever has started, and no order of starting is assumed.
 enum { kValsLoaded = 0, kValsIdentity = 1, kValsNone = 2 };
+
+// The status words of digits 8q .. 8q + 7 of a whole tile, counted from its
+// keys (TILE loads in a row, about 2 ms for 17,408: only where a wait gave up).
+template <uint32_t TILE, int BYTES>
+__device__ BufferU32x4 countTile(BufferRsrc keys, uint32_t tile, uint32_t word, uint32_t dshift, uint32_t q) {
+  BufferU32x4 w = {kHalfFlags, kHalfFlags, kHalfFlags, kHalfFlags};
+  for (uint32_t i = 0; i < TILE; ++i) {
+    const uint32_t d = bufferLoadU32(keys, (tile * TILE + i) * BYTES + word * 4u) >> dshift & (kSortRadix - 1);
+    const uint32_t o = d - 8 * q, one = (o & 1) ? 1u << 16 : 1u;
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c) w[c] += o / 2 == c ? one : 0u;
+  }
+  return w;
+}
+
 template <typename K, int VALS, int BLOCK, int ITEMS>
 __global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__ keysIn,
                                                            const uint32_t *__restrict__ valsIn,
                                                            K *__restrict__ keysOut, uint32_t *__restrict__ valsOut,
                                                            uint32_t n, uint32_t shift,
                                                            const uint32_t *__restrict__ hist, uint32_t *status,
-                                                           uint32_t *err) {
+                                                           uint32_t polls) {
   constexpr int WAVES = BLOCK / 64;
   constexpr uint32_t TILE = BLOCK * ITEMS;
   static_assert(BLOCK >= kSortRadix && TILE <= kHalfCount, "a thread per digit; a tile's count of one digit fits 15 bits");
@@ -354,6 +370,7 @@ __global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__
     static_assert(QG == 2 * WAVES, "two look-back groups per row of s_wave");
     const uint32_t q = tid % OCTS, g = tid / OCTS;
     const BufferRsrc st = bufferRsrc(status, tile * kWideStatusWords * 4u);  // the earlier tiles' words
+    const uint32_t ready = polls ? kHalfFlags : ~0u;  // without polls no word will do: every tile is counted
     uint32_t sum[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u}, spins = 0;
     for (uint32_t j0 = g; j0 < tile; j0 += QG * QB) {
       BufferU32x4 sv[QB];
@@ -367,16 +384,16 @@ __global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__
       for (uint32_t b = 0; b < QB; ++b) {
         const uint32_t j = j0 + b * QG;
         BufferU32x4 v = sv[b];
-        // not yet published (j < tile: tile 0 never waits); the wait is bounded
-        while (((v[0] & v[1] & v[2] & v[3]) & kHalfFlags) != kHalfFlags) {
-          if (++spins > (1u << 24)) {
-            atomicOr(err, 1u);
-            v = BufferU32x4{kHalfFlags, kHalfFlags, kHalfFlags, kHalfFlags};
-            break;
-          }
+        // not yet published (tile 0 never waits); after so many looks in all, one more look each
+        while (__builtin_expect(((v[0] & v[1] & v[2] & v[3]) & ready) != ready, 0)) {
+          if (j >= tile) break;
           __builtin_amdgcn_s_sleep(1);
           memoryChanged();
           v = bufferLoadU32x4Coherent(st, (j * kWideStatusWords + 4 * q) * 4u);
+          if (++spins >= polls && ((v[0] & v[1] & v[2] & v[3]) & ready) != ready) {
+            v = countTile<TILE, sizeof(K)>(keys, j, dw, dshift, q);
+            break;
+          }
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -416,7 +433,7 @@ __global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__
       const K kk = s_buf[j];
       const uint32_t d = (uint32_t)(kk >> shift) & (kSortRadix - 1);
       out[k] = s_gstart[d] + (j - s_bstart[d]);
-      if (out[k] >= n) out[k] = n;  // only reachable after a bounded-wait error
+      if (out[k] >= n) out[k] = n;  // never past the arrays, whatever the histogram held
       if (keysOut && out[k] < n) bufferStore(kk, kout, out[k] * (uint32_t)sizeof(K));
     }
   }
@@ -445,13 +462,14 @@ struct WidePass {
   uint32_t *valsOut;
   uint32_t n, shift;
   const uint32_t *hist;
-  uint32_t *status, *err;
+  uint32_t *status;
+  uint32_t polls;
 };
 template <typename K, int VALS, int BLOCK, int ITEMS>
 void launchWideSize(const SortPlan &p, const WidePass &w) {
   k_onesweepWide<K, VALS, BLOCK, ITEMS><<<p.numTiles, BLOCK, 0, stream()>>>(
       static_cast<const K *>(w.keysIn), w.valsIn, static_cast<K *>(w.keysOut), w.valsOut, w.n, w.shift, w.hist,
-      w.status, w.err);
+      w.status, w.polls);
 }
 template <typename K, int VALS>
 void launchWide(const SortPlan &p, const WidePass &w) {
@@ -535,7 +553,7 @@ int sortRun(const SortPlan &p, void *keys[2], uint32_t *vals[2], bool identityVa
     bool last = pass == p.passes - 1;
     void *kout = (last && !keepKeys) ? nullptr : keys[cur ^ 1];
     uint32_t shift = pass * kSortRadixBits;
-    const WidePass w = {keys[cur], vin, kout, keysOnly ? nullptr : vals[cur ^ 1], p.n, shift, hist, status, err};
+    const WidePass w = {keys[cur], vin, kout, keysOnly ? nullptr : vals[cur ^ 1], p.n, shift, hist, status, rt().sortPolls};
     if (keysOnly)
       launchWide<uint64_t, kValsNone>(p, w);
     else if (p.wide && p.keyBytes == 8 && !vin)

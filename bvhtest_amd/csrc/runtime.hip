@@ -90,6 +90,7 @@ const char *bvht_getLastError(void) { return rt().lastError.c_str(); }
 void bvht_clearError(void) { rt().lastError.clear(); }
 void bvht_setAllocFailAfter(int n) { rt().allocFailAfter = n < 0 ? 0 : n; }
 void bvht_setLaunchFailAfter(int n) { rt().launchFailAfter = n < 0 ? 0 : n; }
+void bvht_setSortPolls(int n) { rt().sortPolls = n < 0 ? kSortPolls : (uint32_t)n; }
 const char *bvht_version(void) { return "bvhtest_amd 0.1 (gfx950)"; }
 int bvht_deviceCount(void) {
   int n = 0;

@@ -12,11 +12,16 @@
 
 namespace bvht {
 
+// Looks (about 1 us each) that a sort workgroup waits for another's counts
+// before it counts that tile's keys itself (radix_sort.hip).
+constexpr uint32_t kSortPolls = 1u << 12;
+
 struct Runtime {
   hipStream_t stream = nullptr;
   std::string lastError;
   int allocFailAfter = 0;  // 0: off; n: the n-th allocation from now fails
   int launchFailAfter = 0;  // the same for checked kernel launches
+  uint32_t sortPolls = kSortPolls;
 };
 
 Runtime &rt();

@@ -139,6 +139,10 @@ void bvht_setAllocFailAfter(int n);
 /* The same for kernel launches: the n-th checked launch from now is reported
  * as failed (its kernel has run), so a call stops half way. */
 void bvht_setLaunchFailAfter(int n);
+/* Host-test hook: how often a workgroup of the one-round sort passes looks for
+ * another's counts before it makes them itself (0: always itself, slow;
+ * negative: the default).  The results are the same. */
+void bvht_setSortPolls(int n);
 /* Library version string and the gfx target it was built for. */
 const char *bvht_version(void);
 /* Number of visible HIP devices (0 when none; never fails). */
@@ -253,8 +257,9 @@ bool bvht_LBVH_build(bvht_LBVH_WorkingMemory *mem, const bvht_MeshRaw *mesh, bvh
  * to completion (also before the first build).  MSD sort: 1 = histogram
  * does not match the keys, 2 = a bucket ran out of key bits, 4 = a piece
  * exceeded the in-LDS limit;
- * onesweep: 1 = a look-back wait gave up; 63-bit keys also 8 = the list of
- * long groups of equal top bits overflowed.
+ * onesweep: 1 = a look-back wait gave up (sorts of more than 17,408 keys per
+ * CU; smaller ones cannot); 63-bit keys also 8 = the list of long groups of
+ * equal top bits overflowed.
  * 0xFFFFFFFF on a bad argument or a failed copy. */
 uint32_t bvht_LBVH_sortStatus(bvht_LBVH_WorkingMemory *mem);
 /* LBVH build that allocates nothing (no counterpart in the reference).  For
