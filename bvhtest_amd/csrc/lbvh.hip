@@ -594,6 +594,14 @@ size_t sortZeroWords(const Internal *in) {
   return in->plan.totalWords;
 }
 
+// The words of the sort scratch that bvht_LBVH_sortStatus reads: the sort's
+// error word, and the split sort's for long groups (without it, the same).
+void sortErrWords(const bvht_LBVH_WorkingMemory *mem, const Internal *in, uint32_t *words[2]) {
+  uint32_t *sc = (uint32_t *)mem->sortScratch;
+  words[0] = sc + (in->useMsd ? in->msd.ctrlOff + 2 : (in->useSplit ? in->split.plan.errOff : in->plan.errOff));
+  words[1] = in->useSplit ? sc + in->split.ctrlOff + 2 : words[0];
+}
+
 // check: the keys are made from k_vertBox's box; verify it against the
 // triangles' box and repair the keys if it differs (k_mortonFix).
 bool launchMorton(bvht_LBVH_WorkingMemory *mem, const bvht_MeshRaw *mesh, bool check) {
@@ -717,7 +725,9 @@ bool buildAll(bvht_LBVH_WorkingMemory *mem, const bvht_MeshRaw *mesh, bvht_CUDAM
   tm.record("begin");
   if (!in->useMsd && mesh->numFaces <= kSmallSortMax) {
     void *keys = mem->opts.topology == 1 ? mem->keys[0] : nullptr;
-    if (!smallSort(*mesh, (int)mem->opts.mortonBits, (BuildParams *)mem->params, keys, mem->values[0])) return false;
+    uint32_t *err[2];
+    sortErrWords(mem, in, err);
+    if (!smallSort(*mesh, (int)mem->opts.mortonBits, (BuildParams *)mem->params, keys, mem->values[0], err)) return false;
     tm.record("k_smallSort");
     in->resultBuf = 0;
     mem->sortedValues = mem->values[0];
@@ -1055,12 +1065,11 @@ uint32_t bvht_LBVH_sortStatus(bvht_LBVH_WorkingMemory *mem) {
     return 0xFFFFFFFFu;
   }
   const Internal *in = internalOf(mem);
-  const uint32_t *sc = (const uint32_t *)mem->sortScratch;
-  const size_t word = in->useMsd ? in->msd.ctrlOff + 2 : (in->useSplit ? in->split.plan.errOff : in->plan.errOff);
-  uint32_t v = 0xFFFFFFFFu, w = 0;
-  if (!check(hipMemcpyAsync(&v, sc + word, 4, hipMemcpyDeviceToHost, stream()), "bvht_LBVH_sortStatus") ||
+  uint32_t *words[2], v = 0xFFFFFFFFu, w = 0;
+  sortErrWords(mem, in, words);
+  if (!check(hipMemcpyAsync(&v, words[0], 4, hipMemcpyDeviceToHost, stream()), "bvht_LBVH_sortStatus") ||
       (in->useSplit &&
-       !check(hipMemcpyAsync(&w, sc + in->split.ctrlOff + 2, 4, hipMemcpyDeviceToHost, stream()), "bvht_LBVH_sortStatus")) ||
+       !check(hipMemcpyAsync(&w, words[1], 4, hipMemcpyDeviceToHost, stream()), "bvht_LBVH_sortStatus")) ||
       !check(hipStreamSynchronize(stream()), "bvht_LBVH_sortStatus sync"))
     return 0xFFFFFFFFu;
   return v | (w << 3);

@@ -3,7 +3,7 @@
 // A mesh of up to a few thousand triangles does not fill a launch of the
 // large build's kernels: eight launches, each a workgroup or a few waiting on
 // its own loads.  Here one workgroup of 1,024 threads keeps everything in
-// registers and LDS: it loads the triangles (kItems per thread), reduces the
+// registers and LDS: it loads the triangles (ITEMS per thread), reduces the
 // box of the vertices they reference (the reference's box, so there is
 // nothing to repair), makes the keys and sorts (key, index) with one stable
 // 8-bit pass per digit; the indices leave in sorted order.
@@ -27,7 +27,8 @@ template <typename K, int PASSES, int ITEMS>
 __global__ __launch_bounds__(kSmallBlock) void k_smallSort(const bvht_vec3 *__restrict__ vert,
                                                            const bvht_Triangle *__restrict__ faces, uint32_t n,
                                                            BuildParams *__restrict__ prm, K *__restrict__ keysOut,
-                                                           uint32_t *__restrict__ valsOut) {
+                                                           uint32_t *__restrict__ valsOut, uint32_t *err,
+                                                           uint32_t *errLong) {
   __shared__ K s_key[kSmallBlock * ITEMS];
   __shared__ uint16_t s_idx[kSmallBlock * ITEMS];
   __shared__ uint32_t s_wave[kSmallWaves][kSortRadix];
@@ -60,6 +61,7 @@ __global__ __launch_bounds__(kSmallBlock) void k_smallSort(const bvht_vec3 *__re
   bvht_vec3 off, sc;
   mortonMapping(box, off, sc);
   if (tid == 0) {
+    *err = *errLong = 0;  // an earlier staged sort's: this one has no wait to give up
     for (int a = 0; a < 3; ++a) {
       prm->sceneMin[a] = box[a];
       prm->sceneMax[a] = box[3 + a];
@@ -142,22 +144,23 @@ __global__ __launch_bounds__(kSmallBlock) void k_smallSort(const bvht_vec3 *__re
 }
 
 template <typename K, int PASSES, int ITEMS>
-void launchSmall(const bvht_MeshRaw &mesh, BuildParams *prm, void *keysOut, uint32_t *valsOut) {
+void launchSmall(const bvht_MeshRaw &mesh, BuildParams *prm, void *keysOut, uint32_t *valsOut, uint32_t *const err[2]) {
   k_smallSort<K, PASSES, ITEMS><<<1, kSmallBlock, 0, stream()>>>(mesh.vert, mesh.faces, mesh.numFaces, prm,
-                                                                 static_cast<K *>(keysOut), valsOut);
+                                                                 static_cast<K *>(keysOut), valsOut, err[0], err[1]);
 }
 
 }  // namespace
 
-bool smallSort(const bvht_MeshRaw &mesh, int mortonBits, BuildParams *prm, void *keysOut, uint32_t *valsOut) {
+bool smallSort(const bvht_MeshRaw &mesh, int mortonBits, BuildParams *prm, void *keysOut, uint32_t *valsOut,
+               uint32_t *const err[2]) {
   const bool wide = mortonBits == 63;
   switch (divUp(mesh.numFaces, kSmallBlock)) {
 #define BVHT_SMALL(I)                                                   \
   case I:                                                               \
     if (wide)                                                           \
-      launchSmall<uint64_t, 8, I>(mesh, prm, keysOut, valsOut);         \
+      launchSmall<uint64_t, 8, I>(mesh, prm, keysOut, valsOut, err);    \
     else                                                                \
-      launchSmall<uint32_t, 4, I>(mesh, prm, keysOut, valsOut);         \
+      launchSmall<uint32_t, 4, I>(mesh, prm, keysOut, valsOut, err);    \
     break;
     BVHT_SMALL(1)
     BVHT_SMALL(2)

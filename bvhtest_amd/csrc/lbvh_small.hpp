@@ -13,7 +13,8 @@ constexpr uint32_t kSmallSortMax = 8192;
 
 // Scene box (into prm), Morton keys and their stable sort: valsOut[p] is the
 // triangle at sorted position p, keysOut (may be null) its key (uint64 for 63
-// bits, uint32 for 30).  numFaces in [1, kSmallSortMax].
-bool smallSort(const bvht_MeshRaw &mesh, int mortonBits, BuildParams *prm, void *keysOut, uint32_t *valsOut);
+// bits, uint32 for 30).  numFaces in [1, kSmallSortMax].  The words err become 0.
+bool smallSort(const bvht_MeshRaw &mesh, int mortonBits, BuildParams *prm, void *keysOut, uint32_t *valsOut,
+               uint32_t *const err[2]);
 
 }  // namespace bvht
