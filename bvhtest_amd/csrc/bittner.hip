@@ -682,8 +682,7 @@ __global__ __launch_bounds__(kPatchBlock) void k_commit(PatchRec *__restrict__ r
                                                         uint32_t *__restrict__ stats, const uint32_t *__restrict__ openIn,
                                                         const uint32_t *__restrict__ numIn,
                                                         uint32_t *__restrict__ open, uint32_t *__restrict__ numPending,
-                                                        uint32_t round, bool again, uint32_t *__restrict__ deep) {
-  if (!LATER && blockIdx.x == 0 && threadIdx.x == 0) *deep = 0;
+                                                        uint32_t round, bool again) {
   const uint32_t at = blockIdx.x * kPatchesPerBlock + threadIdx.x / kPatchLanes, j = threadIdx.x % kPatchLanes;
   const bool in = at < (LATER ? *numIn : K);  // every lane stays for the ballots
   const bool mover = j == kOpenMoved || j == kOpenMoved + 1;
@@ -774,26 +773,29 @@ __device__ __forceinline__ uint32_t tailInsert(uint32_t *keys, uint32_t n, uint3
 }
 
 // The nodes from patch k's insertion point w up to the root, for k_contain:
-// their number and then themselves.  A path that does not fit sets *deep.
+// their number and then themselves, and of a path that does not fit, from its
+// last stored node on, each node's parent at the node's place in `above` (a
+// word per node; walks that share nodes write the same).
 constexpr uint32_t kPathWords = 128;
 __device__ void walkPath(const PatchRec *__restrict__ recs, uint32_t k, uint32_t w,
-                         const bvht_BVHNode *__restrict__ nodes, uint32_t root, uint32_t *__restrict__ paths,
-                         uint32_t *__restrict__ deep) {
+                         const bvht_BVHNode *__restrict__ nodes, uint32_t root, uint32_t N,
+                         uint32_t *__restrict__ paths, uint32_t *above) {
   const uint32_t ok = recs[k].ok;  // another workgroup may be deciding it: undecided patches walk too
   if (ok == REC_NONE || ok == REC_LOST) return;
   uint32_t *path = paths + (2 * (size_t)k + w) * kPathWords;
   uint32_t x = recs[k].best[w], len = 0;
-  while (true) {
+  while (true) {  // a store a level and no other: the wait for the next parent then leaves it in flight
     const uint32_t p = nodes[x].parent;
     path[++len] = x;
-    if (x == root) break;
-    if (len == kPathWords - 1) {
-      *deep = 1;
-      break;
-    }
+    if (x == root || len == kPathWords - 1) break;
     x = p;
   }
   path[0] = len;
+  for (; x != root && len < N; ++len) {
+    const uint32_t p = nodes[x].parent;
+    above[x] = p;
+    x = p < N ? p : root;
+  }
 }
 
 constexpr uint32_t kTailGroups = kTailBlock / kPatchLanes;                          // patches loaded at a time
@@ -805,9 +807,8 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
                                                            const uint32_t *__restrict__ open, uint32_t *listA,
                                                            uint32_t *listB, const uint32_t *__restrict__ numPending,
                                                            uint32_t K, const bvht_BVHNode *__restrict__ nodes,
-                                                           uint32_t root, uint32_t *__restrict__ paths,
-                                                           uint32_t walkers, uint32_t *__restrict__ deep,
-                                                           uint32_t firstRound) {
+                                                           uint32_t root, uint32_t N, uint32_t *__restrict__ paths,
+                                                           uint32_t *above, uint32_t walkers, uint32_t firstRound) {
   // lowest reserving rank per slot, rounds alternate; at first [1] holds the
   // node ids and [0] the patches' slots (16 bits each)
   __shared__ __align__(16) uint32_t s_min[2][kTailSlots];
@@ -818,7 +819,7 @@ __global__ __launch_bounds__(kTailBlock) void k_resolveTail(PatchRec *__restrict
   uint16_t *s_slot = reinterpret_cast<uint16_t *>(&s_min[0][0]);
   if (blockIdx.x > 0) {  // workgroup-uniform
     const uint32_t at = (blockIdx.x - 1) * walkers + threadIdx.x;
-    if (threadIdx.x < walkers && at / 2 < K) walkPath(recs, at / 2, at & 1, nodes, root, paths, deep);
+    if (threadIdx.x < walkers && at / 2 < K) walkPath(recs, at / 2, at & 1, nodes, root, N, paths, above);
     return;
   }
   static_assert(kTailSlots <= 65535 && kTailCap * kNNode * 2 <= sizeof(s_min[0]), "the slots fit s_min[0]");
@@ -1041,13 +1042,15 @@ __device__ __forceinline__ uint32_t applyPatch(PatchRec *r, uint32_t k, uint32_t
 // round trip for its 16 lanes, and nothing is read that another patch writes.
 // Per chunk, with a launch for the walks and one to apply before: 627 patches
 // of 1M triangles 12.3 + 4.8 -> 5.1 us, 2,648 of 4.2M 13.7 + 9.9 -> 7.8 us.
-// A path longer than kPathWords leaves it all to one workgroup, which walks
-// every path before it writes anything.
+// A path longer than kPathWords goes on in `above`, the parents before this
+// launch wrote any: two lanes of the patch, a round trip per level.  (One
+// workgroup for a whole chunk with such a path: 7,503 patches below a path of
+// 150 nodes 16.3 ms a step of four chunks, now 2.83.)
 __global__ __launch_bounds__(kPatchBlock) void k_contain(PatchRec *__restrict__ recs, uint32_t K,
                                                          bvht_BVHNode *__restrict__ nodes, uint32_t root, uint32_t N,
                                                          const uint32_t *__restrict__ marks,
                                                          const uint32_t *__restrict__ paths,
-                                                         const uint32_t *__restrict__ deep, uint64_t *__restrict__ locks,
+                                                         const uint32_t *__restrict__ above, uint64_t *__restrict__ locks,
                                                          uint32_t *__restrict__ fixStarts,
                                                          uint32_t *__restrict__ skipped,
                                                          uint32_t *__restrict__ numPending,
@@ -1065,33 +1068,6 @@ __global__ __launch_bounds__(kPatchBlock) void k_contain(PatchRec *__restrict__ 
 #pragma unroll
     for (uint32_t i = 0; i < ROWS; ++i) x[w][i] = path[w * kPathWords + i * kPatchLanes + j];
   const uint32_t ok = in ? r->ok : (uint32_t)REC_NONE;  // read before lane 0 of the patch writes it
-  if (*deep != 0) {
-    if (blockIdx.x > 0) return;
-    for (uint32_t q = threadIdx.x; q < K; q += kPatchBlock) {  // REC_LOST + 1 .. : decided here
-      if (recs[q].ok != REC_WON) continue;
-      bool bad = false;
-      for (int w = 0; w < 2 && !bad; ++w) {
-        uint32_t at = recs[q].best[w];
-        for (uint32_t steps = 0; steps < N; ++steps) {
-          if (movedByOther(marks[at], at, q, K, recs)) {
-            bad = true;
-            break;
-          }
-          if (at == root) break;
-          at = nodes[at].parent;
-        }
-      }
-      fixStarts[3 * (size_t)q] = bad ? 1 : 0;  // until the patch is applied below
-    }
-    __syncthreads();
-    for (uint32_t q = threadIdx.x / kPatchLanes; q < K; q += kPatchesPerBlock) {
-      const uint32_t okq = recs[q].ok;
-      const bool bad = okq == REC_WON && fixStarts[3 * (size_t)q] != 0;
-      const uint32_t did = applyPatch(recs + q, q, j, okq, bad, nodes, locks, fixStarts, skipped);
-      if (did) atomicAdd(stats + (did == 1 ? ST_APPLIED : ST_CONTAIN), 1u);
-    }
-    return;
-  }
   bool bad = false;
   if (__ballot(ok == REC_WON) != 0) {
     uint32_t len[2];
@@ -1138,6 +1114,15 @@ __global__ __launch_bounds__(kPatchBlock) void k_contain(PatchRec *__restrict__ 
         const uint32_t y = path[w * kPathWords + at];
         bad |= movedByOther(marks[y], y, k, K, recs);
       }
+    if (j < 2 && (j == 0 ? len[0] : len[1]) == kPathWords - 1) {
+      uint32_t y = path[j * kPathWords + kPathWords - 1];  // its mark is done
+      for (uint32_t steps = 0; steps < N && y != root; ++steps) {
+        y = above[y];
+        if (y >= N) break;  // not a tree
+        const uint32_t m = marks[y];
+        bad |= movedByOther(m, y, k, K, recs);
+      }
+    }
   }
   bad = ((__ballot(bad) >> group) & 0xFFFFu) != 0;
   const uint32_t did = in ? applyPatch(r, k, j, ok, bad, nodes, locks, fixStarts, skipped) : 0u;
@@ -1654,7 +1639,7 @@ struct Internal {
   uint32_t N = 0, numLeaves = 0, numInner = 0, K = 0;
   uint32_t root = 0;
   uint32_t *inner = nullptr, *leaves = nullptr;
-  uint32_t *keys[2] = {nullptr, nullptr};
+  uint32_t *keys[2] = {nullptr, nullptr};  // one allocation; once sorted, k_contain's `above`
   uint32_t *vals[2] = {nullptr, nullptr};
   uint32_t *keysAlt = nullptr;    // altSort: the keys the sort consumes (keys[0] keeps the unsorted costs)
   uint32_t *altCounts = nullptr;  // altSort: per-tile counts / offsets
@@ -1668,7 +1653,7 @@ struct Internal {
   size_t noneWords = 0, stateWords = 0;
   uint64_t *locks = nullptr;
   uint32_t *marks = nullptr, *cnt = nullptr, *refitCnt = nullptr;
-  uint32_t *pending[2] = {nullptr, nullptr}, *numPending = nullptr, *deep = nullptr, *paths = nullptr;
+  uint32_t *pending[2] = {nullptr, nullptr}, *numPending = nullptr, *paths = nullptr;
   uint32_t *fixStarts = nullptr;
   uint64_t *refitSlots = nullptr;  // where two refit walks meet (all zero between launches)
   size_t refitSlotWords = 0;
@@ -1709,7 +1694,6 @@ void carveState(Internal *in, size_t &words) {
   in->skipped = take(in->K);
   in->stats = take(ST_WORDS);
   in->numPending = take(kCommitRounds);
-  in->deep = take(1);
   words = off;
 }
 
@@ -1841,6 +1825,7 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
   in->refitSlotWords = std::max<size_t>(6 * 3 * (size_t)batchSize, 4 * (size_t)divUp(numFaces, 4));
   carveState(in, in->stateWords);
   const uint32_t selBlocks = divUp(in->N, kSelTile);
+  const size_t keyStride = ((size_t)in->numInner + 4) & ~(size_t)3;  // both halves: at least N words, for k_contain
   m.numLeafNodes = in->numLeaves;
   m.numInnerNodes = in->numInner;
   m.numPatches = batchSize;
@@ -1848,7 +1833,7 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
   m.numNodesToFix = 3 * batchSize;
   m.numFlags = in->N;
   bool ok = devAlloc(&in->inner, in->numInner, "bn13 inner") && devAlloc(&in->leaves, in->numLeaves, "bn13 leaves") &&
-            devAlloc(&in->keys[0], in->numInner, "bn13 keys") && devAlloc(&in->keys[1], in->numInner, "bn13 keys") &&
+            devAlloc(&in->keys[0], 2 * keyStride, "bn13 keys") &&
             devAlloc(&in->vals[0], in->numInner, "bn13 vals") && devAlloc(&in->vals[1], in->numInner, "bn13 vals") &&
             devMalloc(reinterpret_cast<void **>(&in->sortScratch), sortScratchBytes(in->plan), "bn13 sort") &&
             devAlloc(&in->recs, batchSize, "bn13 patches") && devAlloc(&in->state, in->stateWords, "bn13 state") &&
@@ -1860,6 +1845,7 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
     return m;
   }
   carveState(in, in->stateWords);
+  in->keys[1] = in->keys[0] + keyStride;
   in->selCounts = reinterpret_cast<uint32_t *>(in->selBits + kSelWords * (size_t)selBlocks);
   m.result = true;
   return m;
@@ -1871,7 +1857,6 @@ void freeMemory(bvht_GPUWorkingMemory *data) {
     devFree(in->inner);
     devFree(in->leaves);
     devFree(in->keys[0]);
-    devFree(in->keys[1]);
     devFree(in->keysAlt);
     devFree(in->altCounts);
     devFree(in->vals[0]);
@@ -2110,13 +2095,13 @@ void bn13_rmAndReinsChunk(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer
   const uint32_t commitBlocks = divUp(K, kPatchesPerBlock), rounds = commitRounds(K, in->N);
   k_commit<false><<<commitBlocks, kPatchBlock, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped, in->stats,
                                                               nullptr, nullptr, in->pending[0], in->numPending, 1u,
-                                                              rounds > 1, in->deep);
+                                                              rounds > 1);
   if (!checkLaunch("k_commit")) return;
   for (uint32_t r = 2; r <= rounds; ++r) {
     k_commit<true><<<commitBlocks, kPatchBlock, 0, stream()>>>(in->recs, K, in->locks, in->marks, in->skipped, in->stats,
                                                                in->pending[r & 1], in->numPending + r - 2,
                                                                in->pending[(r & 1) ^ 1], in->numPending + r - 1, r,
-                                                               r < rounds, in->deep);
+                                                               r < rounds);
     if (!checkLaunch("k_commit")) return;
   }
   const size_t lists = kOpenWords * (size_t)in->K;  // behind the open entries: room for k_resolveTail's lists
@@ -2125,11 +2110,11 @@ void bn13_rmAndReinsChunk(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer
   const uint32_t walkers = divUp(2ull * K, 64) < (uint32_t)numCUs() ? 64 : kTailBlock;
   k_resolveTail<<<1 + divUp(2ull * K, walkers), kTailBlock, 0, stream()>>>(
       in->recs, in->locks, in->marks, in->skipped, in->stats, in->pending[(rounds & 1) ^ 1],
-      in->pending[0] + lists, in->pending[1] + lists, in->numPending + rounds - 1, K, bvh->nodes, in->root, in->paths,
-      walkers, in->deep, rounds + 1);
+      in->pending[0] + lists, in->pending[1] + lists, in->numPending + rounds - 1, K, bvh->nodes, in->root, in->N,
+      in->paths, in->keys[0], walkers, rounds + 1);
   if (!checkLaunch("k_resolveTail")) return;
   k_contain<<<divUp(K, kPatchesPerBlock), kPatchBlock, 0, stream()>>>(in->recs, K, bvh->nodes, in->root, in->N, in->marks,
-                                                                      in->paths, in->deep, in->locks, in->fixStarts,
+                                                                      in->paths, in->keys[0], in->locks, in->fixStarts,
                                                                       in->skipped, in->numPending, in->stats);
   if (!checkLaunch("k_contain")) return;
   refitFrom(in, bvh, in->fixStarts, 3 * K, false);
