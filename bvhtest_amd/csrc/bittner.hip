@@ -135,6 +135,8 @@ __device__ __forceinline__ void storeBox(bvht_BVHNode *nd, const float b[6], flo
   nd->surfaceArea = sa;
 }
 
+__device__ __forceinline__ bvht_AABB boxOf(const float b[6]) { return bvht_AABB{{{b[0], b[1], b[2]}, {b[3], b[4], b[5]}}}; }
+
 __device__ __forceinline__ float sa6(const float b[6]) { return surfaceArea(b[0], b[1], b[2], b[3], b[4], b[5]); }
 __device__ __forceinline__ void merge6(float a[6], const float b[6]) {
   a[0] = mergeMin(a[0], b[0]);
@@ -1157,9 +1159,13 @@ __global__ __launch_bounds__(kPatchBlock) void k_contain(PatchRec *__restrict__ 
 // both children's boxes and coherent stores that were waited for, three round
 // trips past the L2: 1,881 starts in 1M triangles 59 -> 23 us, 100,000
 // leaves of them 57 -> 37 us.
-constexpr uint32_t kRefitChildren = 3u, kRefitStart = 4u, kRefitDup = 8u, kRefitSlotShift = 4u;
+//
+// Lists of more starts than there are slots take none: bit 4 of a word then
+// says that a walk has arrived (kRefitArrived).
+constexpr uint32_t kRefitChildren = 3u, kRefitStart = 4u, kRefitDup = 8u, kRefitSlotShift = 4u, kRefitArrived = 16u;
 constexpr uint32_t kRefitBlock = 256;
 
+template <bool SLOTS>
 __global__ __launch_bounds__(kRefitBlock) void k_refitCount(const uint32_t *__restrict__ starts, uint32_t num,
                                                             uint32_t walks, const bvht_BVHNode *__restrict__ nodes, uint32_t N,
                                                             uint32_t *__restrict__ cnt) {
@@ -1176,7 +1182,7 @@ __global__ __launch_bounds__(kRefitBlock) void k_refitCount(const uint32_t *__re
     node = p;
     p = loadRelaxedAgent(&nodes[node].parent);
     old = atomicAdd(cnt + node, 1u);
-    if ((old & kRefitChildren) == 1) atomicOr(cnt + node, i << kRefitSlotShift);
+    if (SLOTS && (old & kRefitChildren) == 1) atomicOr(cnt + node, i << kRefitSlotShift);
   }
 }
 
@@ -1226,34 +1232,55 @@ __device__ __forceinline__ void unpackSlot(const uint64_t (&w)[WORDS], uint32_t 
 // workgroup has stopped, those whose box nobody took meet other workgroups'
 // walks in the slots.  Exchanging everything in the slots instead is bound
 // by the exchanges themselves (100,000 leaves of 1M: 52 us against 37).
-constexpr uint32_t kNearSlots = 2 * kRefitBlock;  // LDS table, at most half full
-template <bool FEAT, bool NEAR>
-__global__ __launch_bounds__(kRefitBlock) void k_refitApply(const uint32_t *__restrict__ starts, uint32_t num,
+//
+// By ids (NEAR lists of more than a quarter of the leaves): every node is a
+// candidate, in the order of the ids, and the marked starts walk, so
+// neighbours meet in LDS in whatever order the list names them.
+//
+// ARRIVE (by ids, more starts than slots): walks of two workgroups meet by
+// arrival: the box is stored past the L2, then the arrival marked; the second
+// loads the first one's box.  Three round trips, and no limit on the starts;
+// workgroups of 1,024 leave fewer such meetings (4M leaves 530 -> 388 us).
+//
+// All of 20,000 leaves in order / mixed 38 / 40 us (40 / 63 with an arrival at
+// every level, 101 / 199 in pieces of a quarter of the leaves), 100,000 48 / 56
+// (59 / 113, 113 / 246), 1M 174 / 242 (316 / 472, 225 / 988), 4M 647 / 904
+// (1,437 / 2,188, 623 / 4,114).
+enum { kRefitScattered = 0, kRefitNear = 1, kRefitIds = 2, kRefitArrive = 3 };
+constexpr uint32_t kSlotListMin = 1u << 17;
+constexpr uint32_t refitBlock(int list) { return list == kRefitArrive ? 1024 : kRefitBlock; }
+template <bool FEAT, int LIST>
+__global__ __launch_bounds__(refitBlock(LIST)) void k_refitApply(const uint32_t *__restrict__ starts, uint32_t num,
                                                             uint32_t walks, bvht_BVHNode *__restrict__ nodes,
                                                             uint32_t N, uint32_t *__restrict__ cnt, uint64_t *slots,
                                                             uint32_t *__restrict__ leafCnt,
                                                             float *__restrict__ subSA, uint32_t *__restrict__ stats) {
+  constexpr bool NEAR = LIST != kRefitScattered, IDS = LIST >= kRefitIds, ARRIVE = LIST == kRefitArrive;
   static_assert(!(FEAT && NEAR), "a near list keeps no features");
   constexpr int WORDS = FEAT ? 6 : 4;
+  constexpr uint32_t BLOCK = refitBlock(LIST), kNearSlots = 2 * BLOCK;  // LDS table, at most half full
   __shared__ unsigned long long s_key[NEAR ? kNearSlots : 1];  // node id << 32 | thread that left its box
-  __shared__ uint32_t s_box[6][NEAR ? kRefitBlock : 1];
-  __shared__ uint32_t s_taken[NEAR ? kRefitBlock : 1];
+  __shared__ uint32_t s_box[6][NEAR ? BLOCK : 1];
+  __shared__ uint32_t s_taken[NEAR ? BLOCK : 1];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
-  if (NEAR) {
-    for (uint32_t k = tid; k < kNearSlots; k += kRefitBlock) s_key[k] = ~0ull;
+  const auto clearTable = [&] {
+    for (uint32_t k = tid; k < kNearSlots; k += BLOCK) s_key[k] = ~0ull;
     s_taken[tid] = 0;
     __syncthreads();
-  }
-  const uint32_t i = (blockIdx.x * (kRefitBlock / 64) + tid / 64) * walks + lane;
-  uint32_t child = lane < walks && i < num ? starts[i] : NONE;
+  };
+  if (NEAR && !IDS) clearTable();  // ahead of the loads: a barrier behind them would wait for them
+  const uint32_t i = (blockIdx.x * (BLOCK / 64) + tid / 64) * walks + lane;
+  uint32_t child = IDS ? i : lane < walks && i < num ? starts[i] : NONE;
   bool go = child < N;
   if (!go) child = 0;
-  NodeView nv = globalView(nodes, child);
   uint32_t c = cnt[child];
   // a walk from below recomputes the node (or has: its word is cleared)
   go = go && c != 0 && (c & kRefitChildren) == 0;
+  if (IDS && __syncthreads_or(go) == 0) return;
+  if (IDS) clearTable();
+  NodeView nv = globalView(nodes, child);
   // one occurrence of a start named more than once goes on
-  if (go && (c & kRefitDup)) go = atomicExch(cnt + child, 0u) != 0;
+  if (!IDS && go && (c & kRefitDup)) go = atomicExch(cnt + child, 0u) != 0;
   if (!NEAR && !go) return;
   uint32_t node = nv.parent;
   bool end = node == child || node >= N;
@@ -1309,8 +1336,9 @@ __global__ __launch_bounds__(kRefitBlock) void k_refitApply(const uint32_t *__re
       }
       uint64_t w[WORDS];
       uint64_t *slot = slots + (size_t)at * WORDS;
-      const bool bad = meet && at >= num;  // not a tree (more than two children on a path)
-      if (phase == 1 && meet && !bad) {
+      const bool bad = !ARRIVE && meet && at >= num;  // not a tree (more than two children on a path)
+      const bool arrive = ARRIVE && phase == 1 && meet;
+      if (!ARRIVE && phase == 1 && meet && !bad) {
         uint32_t v[6 + 2 * (WORDS - 4) / 2];
 #pragma unroll
         for (int k = 0; k < 6; ++k) v[k] = __float_as_uint(b[k]);
@@ -1323,13 +1351,28 @@ __global__ __launch_bounds__(kRefitBlock) void k_refitApply(const uint32_t *__re
         for (int k = 0; k < WORDS; ++k)
           w[k] = __hip_atomic_exchange(slot + k, w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-      storeBox(nodes + child, b, sa);
+      if (arrive)
+        storeBoxAgent(nodes + child, boxOf(b), sa);
+      else
+        storeBox(nodes + child, b, sa);
       if (FEAT) {
         leafCnt[child] = leaves;
         subSA[child] = sub;
       }
       cnt[child] = 0;
       if (end || bad) break;
+      if (arrive) {
+        waitVectorMemory();  // the box is out before the arrival
+        const uint32_t seen = __hip_atomic_fetch_or(cnt + node, kRefitArrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((seen & kRefitArrived) == 0) break;  // first: the other walk goes on
+        const bvht_AABB o = loadBoxAgent(nodes + sib);
+        s[0] = o.minMax[0].x;
+        s[1] = o.minMax[0].y;
+        s[2] = o.minMax[0].z;
+        s[3] = o.minMax[1].x;
+        s[4] = o.minMax[1].y;
+        s[5] = o.minMax[1].z;
+      }
       if (phase == 0 && meet) {
 #pragma unroll
         for (int k = 0; k < 6; ++k)
@@ -1357,7 +1400,7 @@ __global__ __launch_bounds__(kRefitBlock) void k_refitApply(const uint32_t *__re
           s[k] = __uint_as_float(
               __hip_atomic_load(&s_box[k][from], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
       }
-      if (phase == 1 && meet) {
+      if (!ARRIVE && phase == 1 && meet) {
         if ((w[0] >> 48) == 0) break;  // first: the other walk goes on
         const uint32_t other = left ? 2u : 1u;
         for (uint32_t spins = 0;; ++spins) {
@@ -1719,27 +1762,37 @@ bool features(Internal *in, const bvht_CUDAMemoryBVHPointer *bvh) {
 // Refit from `num` device start nodes.  near: a list of leaves in their order
 // (no features kept); otherwise a chunk's scattered starts, 8 walks a wave
 // (1,881 starts in 1M triangles: 23.2, 25.0, 26.3, 29.2 us with 8, 16, 32, 64),
-// with the subtree features kept when they are in use.  A list longer than
-// the slots is done in pieces: a node above starts of two pieces is
-// recomputed by each, last with both its children final.
+// with the subtree features kept when they are in use.  More of those than
+// slots are done in pieces: a node above starts of two pieces is recomputed by
+// each, last with both its children final.
 bool refitFrom(Internal *in, const bvht_CUDAMemoryBVHPointer *bvh, const uint32_t *starts, uint32_t num, bool near) {
   const bool feat = !near && in->subValid;
   const uint32_t walks = near ? 64 : 8;
   const uint32_t most = (uint32_t)std::min<size_t>(in->refitSlotWords / (feat ? 6 : 4), 1u << (32 - kRefitSlotShift));
+  if (near && num > most) {
+    k_refitCount<false><<<divUp(num, kRefitBlock), kRefitBlock, 0, stream()>>>(starts, num, walks, bvh->nodes, in->N, in->cnt);
+    if (!checkLaunch("k_refitCount")) return false;
+    constexpr uint32_t block = refitBlock(kRefitArrive);
+    k_refitApply<false, kRefitArrive><<<divUp(in->N, block), block, 0, stream()>>>(
+        nullptr, num, walks, bvh->nodes, in->N, in->cnt, nullptr, nullptr, nullptr, in->stats);
+    return checkLaunch("k_refitApply");
+  }
   for (uint32_t at = 0; at < num;) {
     const uint32_t n = std::min(most, num - at), blocks = divUp(n, walks * (kRefitBlock / 64));
-    k_refitCount<<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N, in->cnt);
+    k_refitCount<true><<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N, in->cnt);
     if (!checkLaunch("k_refitCount")) return false;
-    if (near)
-      k_refitApply<false, true><<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N, in->cnt,
-                                                                      in->refitSlots, nullptr, nullptr, in->stats);
+    auto apply = [&](auto feat, auto list, uint32_t grid, uint32_t *leafCnt, float *subSA) {
+      k_refitApply<decltype(feat)::value, decltype(list)::value><<<grid, kRefitBlock, 0, stream()>>>(
+          starts + at, n, walks, bvh->nodes, in->N, in->cnt, in->refitSlots, leafCnt, subSA, in->stats);
+    };
+    if (near && n > in->numLeaves / 4)
+      apply(std::false_type(), std::integral_constant<int, kRefitIds>(), divUp(in->N, kRefitBlock), nullptr, nullptr);
+    else if (near)
+      apply(std::false_type(), std::integral_constant<int, kRefitNear>(), blocks, nullptr, nullptr);
     else if (feat)
-      k_refitApply<true, false><<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N, in->cnt,
-                                                                      in->refitSlots, in->leafCnt, in->subSA, in->stats);
+      apply(std::true_type(), std::integral_constant<int, kRefitScattered>(), blocks, in->leafCnt, in->subSA);
     else
-      k_refitApply<false, false><<<blocks, kRefitBlock, 0, stream()>>>(starts + at, n, walks, bvh->nodes, in->N,
-                                                                       in->cnt, in->refitSlots, nullptr, nullptr,
-                                                                       in->stats);
+      apply(std::false_type(), std::integral_constant<int, kRefitScattered>(), blocks, nullptr, nullptr);
     if (!checkLaunch("k_refitApply")) return false;
     at += n;
   }
@@ -1821,8 +1874,9 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
   in->numInner = bvh->numNodes - numFaces;
   in->K = batchSize;
   in->plan = makeSortPlan(in->numInner, 4, 32);
-  // a chunk's 3 starts per patch in one piece, and lists of up to a quarter of the leaves
-  in->refitSlotWords = std::max<size_t>(6 * 3 * (size_t)batchSize, 4 * (size_t)divUp(numFaces, 4));
+  // a chunk's 3 starts per patch in one piece, and lists of up to a quarter of the leaves or 131,072 of them
+  in->refitSlotWords = std::max<size_t>(6 * 3 * (size_t)batchSize,
+                                        4 * (size_t)std::max(divUp(numFaces, 4), std::min(numFaces, kSlotListMin)));
   carveState(in, in->stateWords);
   const uint32_t selBlocks = divUp(in->N, kSelTile);
   const size_t keyStride = ((size_t)in->numInner + 4) & ~(size_t)3;  // both halves: at least N words, for k_contain
