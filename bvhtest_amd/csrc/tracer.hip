@@ -126,6 +126,10 @@ struct NodeRec {
 };
 static_assert(sizeof(NodeRec) == 64, "one record per visit");
 constexpr uint32_t kLeafRef = 0x80000000u;  // the other bits: node id
+// No child: past every reference, since prepareTrace takes fewer than kLeafRef
+// nodes (up to 2^30 triangles).
+constexpr uint32_t kNoChild = 0xFFFFFFFFu;
+static_assert(((kLeafRef - 2) | kLeafRef) < kNoChild, "the last node of the largest tree has a reference of its own");
 constexpr int kStackCap = 24;  // pending children per lane: 6 KiB of LDS a wave, 26 waves on a CU
 // k_traceRaysDyn waves on a CU.  16, 20, 24, 26: 4.11, 3.99, 4.14, 4.13 ms at
 // 1080p over 4.2M triangles, 685, 600, 608, 602 us at 512x512 over 65k (beyond
@@ -136,9 +140,9 @@ constexpr uint32_t kTraceWavesPerCU = 20;
 // 575, 554 us at 1024x1024 over 65k.
 constexpr uint32_t kRefillAt = 32;
 
-// One node's record.  A child index at or past `bound` becomes an empty leaf
-// (a reference past the records) and raises *bad (the traversal then never
-// reads past the arrays).
+// One node's record.  A child index at or past `bound` becomes kNoChild with
+// an empty box and raises *bad (the traversal then never reads past the
+// arrays).
 __device__ __forceinline__ NodeRec packNode(uint32_t i, const bvht_BVHNode *__restrict__ nodes, uint32_t bound,
                                             const bvht_Triangle *__restrict__ faces,
                                             const bvht_vec3 *__restrict__ vert, uint32_t numFaces,
@@ -170,7 +174,7 @@ __device__ __forceinline__ NodeRec packNode(uint32_t i, const bvht_BVHNode *__re
       } else {
         *bad = 1;
         box[k] = {{{0.f, 0.f, 0.f}, {-1.f, -1.f, -1.f}}};
-        child[k] = 0xFFFFFFFFu;
+        child[k] = kNoChild;
       }
     }
     p.a = make_float4(box[0].minMax[0].x, box[0].minMax[0].y, box[0].minMax[0].z, box[0].minMax[1].x);
@@ -304,7 +308,6 @@ __device__ __forceinline__ bool walkPop(Walk &s, const uint32_t *stk) {
 
 // The two children of an inner node: which one is entered now and which one
 // waits (kNoChild: none).
-constexpr uint32_t kNoChild = 0xFFFFFFFEu;
 template <int OCT>
 __device__ __forceinline__ void innerChildren(const NodeRec *r, const WalkRay &ray, float t1, uint32_t &now,
                                               uint32_t &later) {
@@ -418,6 +421,10 @@ __device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx 
       uint32_t now, later;
       innerChildren<kAnyOct>(cx.recs + s.ref, ray, s.t1, now, later);
       s.count++;
+      if (now == kNoChild) {  // a missing child's empty box, met by a ray with wrong signs
+        now = later;
+        later = kNoChild;
+      }
       if (now != kNoChild) {
         hi = (hi << 1) | (lo >> 63);
         lo = (lo << 1) | (later != kNoChild ? 1u : 0u);

@@ -503,6 +503,8 @@ void freeRays(bvht_Ray **rays);                                   /* CUDAKernels
 void freeImage(bvht_CUDAPixel *img);                              /* CUDAKernels.hpp:42 */
 /* generateRays -- lib/tracer/CUDAKernels.cu:386-397 (pinhole camera). */
 void generateRays(bvht_Ray *rays, uint32_t w, uint32_t h, bvht_vec3 pos, bvht_vec3 lookAt, bvht_vec3 up, float fov);
+/* Traces take meshes of at most 2^30 triangles (more are refused with an error:
+ * node ids carry 31 bits). */
 /* tracerImage -- lib/tracer/CUDAKernels.cu:399-417.  bundle selects the
  * wave-coherent traversal (reference kTraceRayBundle). */
 void tracerImage(bvht_Ray *rays, bvht_CUDAPixel *img, bvht_BVHNode *nodes, uint32_t rootNode, bvht_MeshRaw mesh,
