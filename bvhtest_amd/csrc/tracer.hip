@@ -407,11 +407,20 @@ constexpr uint32_t kMaxSteps = 1u << 26, kCheckSteps = 1u << 20;
 
 // The walk of a ray that had more than kStackCap children pending, from the
 // start: the reference's 128-bit trail (a 1 marks a level whose second child
-// is still pending) and its parent links instead of a stack.  Same visits.
+// is still pending) and, where the stack has dropped a child, its parent links.
+// The stack keeps the last kStackCap of the pending children (a ring: `end`
+// is the place of the next, `kept` of them are there).  Same visits.  (Trees of
+// one path over 32, 64 and 120 triangles, one above the other, 640x480: 45, 114
+// and 189 us, without the ring 45, 130 and 208, with a ring in every walk 57,
+// 103 and 182.  A stack that goes on in scratch memory needs no start over, but
+// took 490 us instead of 290 for a 1024x1024 image of 65k triangles and 12.7 ms
+// instead of 7.1 for a 1080p frame of 4.2M.)
 template <int MODE>
-__device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx &cx, uint32_t top, float tMin, uint32_t skip) {
+__device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx &cx, uint32_t top, float tMin,
+                                             uint32_t skip, uint32_t *stk) {
   Walk s;
   walkReset(s, top);
+  uint32_t end = 0, kept = 0;
   uint64_t lo = 0, hi = 0;
   while (s.count < kMaxSteps) {
     const bool leaf = (s.ref & kLeafRef) != 0;
@@ -427,7 +436,13 @@ __device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx 
       }
       if (now != kNoChild) {
         hi = (hi << 1) | (lo >> 63);
-        lo = (lo << 1) | (later != kNoChild ? 1u : 0u);
+        lo <<= 1;
+        if (later != kNoChild) {
+          lo |= 1;
+          stk[end * 64] = later;
+          end = end + 1 == (uint32_t)kStackCap ? 0u : end + 1;
+          kept = min(kept + 1, (uint32_t)kStackCap);
+        }
         s.ref = now;
         continue;
       }
@@ -446,6 +461,12 @@ __device__ __forceinline__ TraceOut slowWalk(const WalkRay &ray, const TraceCtx 
       hi = 0;
     }
     lo ^= 1;
+    if (kept > 0) {
+      --kept;
+      end = end == 0 ? (uint32_t)kStackCap - 1 : end - 1;
+      s.ref = stk[end * 64];
+      continue;
+    }
     uint32_t node = s.ref & ~kLeafRef;
     for (uint32_t k = 0; k < up && node < cx.bound; ++k) node = cx.nodes[node].parent;
     if (node >= cx.bound) break;
@@ -493,7 +514,7 @@ __device__ __forceinline__ TraceOut walkAll(bool active, const bvht_Ray &r, cons
     case 7: walkLoop<MODE, 7, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
     default: walkLoop<MODE, kAnyOct, AHEAD>(active, s, ray, cx, tMin, skip, stk); break;
   }
-  if (s.sp > (uint32_t)kStackCap) return slowWalk<MODE>(ray, cx, top, tMin, skip);
+  if (s.sp > (uint32_t)kStackCap) return slowWalk<MODE>(ray, cx, top, tMin, skip, stk);
   return TraceOut{s.tri, s.nearest, (uint16_t)s.count};
 }
 
@@ -723,7 +744,7 @@ __global__ __launch_bounds__(64) void k_traceRaysDyn(const bvht_Ray *__restrict_
     if ((it & (kCheckSteps - 1)) == 0 && s.count >= kMaxSteps) active = false;
     if (was && !active) {
       TraceOut o = {s.tri, s.nearest, (uint16_t)s.count};
-      if (s.sp > (uint32_t)kStackCap) o = slowWalk<MODE>(ray, cx, top, tMin, skipTri);
+      if (s.sp > (uint32_t)kStackCap) o = slowWalk<MODE>(ray, cx, top, tMin, skipTri, stk);
       if (hits) hits[i] = bvht_Hit{o.tri, o.t};
       if (img) {
         bvht_Ray r = {};
