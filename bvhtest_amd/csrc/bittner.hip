@@ -777,22 +777,25 @@ __device__ __forceinline__ uint32_t tailInsert(uint32_t *keys, uint32_t n, uint3
 // The nodes from patch k's insertion point w up to the root, for k_contain:
 // their number and then themselves, and of a path that does not fit, from its
 // last stored node on, each node's parent at the node's place in `above` (a
-// word per node; walks that share nodes write the same).
+// word per node; walks that share nodes write the same).  Without `paths`
+// (allocateMemory), the parents from the insertion point on.
 constexpr uint32_t kPathWords = 128;
 __device__ void walkPath(const PatchRec *__restrict__ recs, uint32_t k, uint32_t w,
                          const bvht_BVHNode *__restrict__ nodes, uint32_t root, uint32_t N,
                          uint32_t *__restrict__ paths, uint32_t *above) {
   const uint32_t ok = recs[k].ok;  // another workgroup may be deciding it: undecided patches walk too
   if (ok == REC_NONE || ok == REC_LOST) return;
-  uint32_t *path = paths + (2 * (size_t)k + w) * kPathWords;
   uint32_t x = recs[k].best[w], len = 0;
-  while (true) {  // a store a level and no other: the wait for the next parent then leaves it in flight
-    const uint32_t p = nodes[x].parent;
-    path[++len] = x;
-    if (x == root || len == kPathWords - 1) break;
-    x = p;
+  if (paths) {
+    uint32_t *path = paths + (2 * (size_t)k + w) * kPathWords;
+    while (true) {  // a store a level and no other: the wait for the next parent then leaves it in flight
+      const uint32_t p = nodes[x].parent;
+      path[++len] = x;
+      if (x == root || len == kPathWords - 1) break;
+      x = p;
+    }
+    path[0] = len;
   }
-  path[0] = len;
   for (; x != root && len < N; ++len) {
     const uint32_t p = nodes[x].parent;
     above[x] = p;
@@ -1068,7 +1071,7 @@ __global__ __launch_bounds__(kPatchBlock) void k_contain(PatchRec *__restrict__ 
 #pragma unroll
   for (int w = 0; w < 2; ++w)
 #pragma unroll
-    for (uint32_t i = 0; i < ROWS; ++i) x[w][i] = path[w * kPathWords + i * kPatchLanes + j];
+    for (uint32_t i = 0; i < ROWS; ++i) x[w][i] = paths ? path[w * kPathWords + i * kPatchLanes + j] : 0u;
   const uint32_t ok = in ? r->ok : (uint32_t)REC_NONE;  // read before lane 0 of the patch writes it
   bool bad = false;
   if (__ballot(ok == REC_WON) != 0) {
@@ -1116,8 +1119,9 @@ __global__ __launch_bounds__(kPatchBlock) void k_contain(PatchRec *__restrict__ 
         const uint32_t y = path[w * kPathWords + at];
         bad |= movedByOther(marks[y], y, k, K, recs);
       }
-    if (j < 2 && (j == 0 ? len[0] : len[1]) == kPathWords - 1) {
-      uint32_t y = path[j * kPathWords + kPathWords - 1];  // its mark is done
+    if (j < 2 && (paths ? (j == 0 ? len[0] : len[1]) == kPathWords - 1 : ok == REC_WON)) {
+      uint32_t y = paths ? path[j * kPathWords + kPathWords - 1] : r->best[j];
+      if (!paths) bad |= movedByOther(marks[y], y, k, K, recs);  // a stored node's mark is done
       for (uint32_t steps = 0; steps < N && y != root; ++steps) {
         y = above[y];
         if (y >= N) break;  // not a tree
@@ -1879,6 +1883,8 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
                                         4 * (size_t)std::max(divUp(numFaces, 4), std::min(numFaces, kSlotListMin)));
   carveState(in, in->stateWords);
   const uint32_t selBlocks = divUp(in->N, kSelTile);
+  // 1 KB a patch: not where they would take more than two thirds of the nodes' own 48 bytes each
+  const bool storePaths = batchSize <= in->N / 32;
   const size_t keyStride = ((size_t)in->numInner + 4) & ~(size_t)3;  // both halves: at least N words, for k_contain
   m.numLeafNodes = in->numLeaves;
   m.numInnerNodes = in->numInner;
@@ -1892,7 +1898,7 @@ bvht_GPUWorkingMemory allocateMemory(bvht_CUDAMemoryBVHPointer *bvh, uint32_t ba
             devMalloc(reinterpret_cast<void **>(&in->sortScratch), sortScratchBytes(in->plan), "bn13 sort") &&
             devAlloc(&in->recs, batchSize, "bn13 patches") && devAlloc(&in->state, in->stateWords, "bn13 state") &&
             devAlloc(&in->pending[0], (1 + kOpenWords) * (size_t)batchSize, "bn13 pending") && devAlloc(&in->pending[1], (1 + kOpenWords) * (size_t)batchSize, "bn13 pending") &&
-            devAlloc(&in->paths, 2 * kPathWords * (size_t)batchSize, "bn13 paths") &&
+            (!storePaths || devAlloc(&in->paths, 2 * kPathWords * (size_t)batchSize, "bn13 paths")) &&
             devAlloc(&in->selBits, (kSelWords + 1) * (size_t)selBlocks, "bn13 select") && devAlloc(&in->partials, kSahBlocks, "bn13 SAH");
   if (!ok) {
     freeMemory(&m);

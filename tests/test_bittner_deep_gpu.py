@@ -35,10 +35,12 @@ def grafted(bvh, n, c):
     return nodes
 
 
-# 127 nodes of a path are stored; the last two: more patches than a workgroup has, on either side of the
-# sizes where the conflict rounds change
-@pytest.mark.parametrize("n,c,percent,chunks", [(2000, 100, 10.0, 2), (2000, 113, 10.0, 2), (2000, 128, 10.0, 2),
-                                                (2000, 600, 10.0, 2), (4000, 150, 9.0, 1), (30000, 200, 20.0, 2)])
+# 127 nodes of a path are stored where a chunk has at most a 32nd of the nodes (the first line), none where
+# it has more; the last of each: more patches than a workgroup has
+@pytest.mark.parametrize("n,c,percent,chunks", [(2000, c, 10.0, 4) for c in (100, 113, 114, 115, 116, 117, 600)] +
+                                               [(30000, 200, 12.0, 4)] +
+                                               [(2000, c, 10.0, 2) for c in (100, 128, 600)] +
+                                               [(4000, 150, 9.0, 1), (30000, 200, 20.0, 2)])
 def test_deep_paths_equal_replay(bvh, orc, n, c, percent, chunks):
     nodes = grafted(bvh, n, c)
     rc, _, _, st, trees = orc.bittner_gpuref(nodes, percent, chunks, 2, search=1, chunk_trees=True)
@@ -56,3 +58,30 @@ def test_deep_paths_equal_replay(bvh, orc, n, c, percent, chunks):
     got = opt.stats()
     assert bvh.last_error() == "" and got["applied"] > 0 and got["unresolved"] == 0
     assert got["contained"] == int(st[2]) and got["contained"] > 0
+
+
+def test_memory_of_a_large_chunk(bvh):
+    """A patch of a chunk with half of the nodes takes no stored path: its record, entries, slots and starts
+    are 528 bytes."""
+    L = bvh.lib()
+    with open("/proc/self/maps") as maps:  # the HIP runtime that the library uses
+        hip = ctypes.CDLL(next(l.split()[-1] for l in maps if "libamdhip64" in l))
+
+    def free():
+        got, total = ctypes.c_size_t(), ctypes.c_size_t()
+        L.doCudaDevSync()
+        assert hip.hipMemGetInfo(ctypes.byref(got), ctypes.byref(total)) == 0
+        return got.value
+
+    n = 500000
+    v, f = bvh.scene_soup(n, 3)
+    tree = bvh.lbvh_build(bvh.DeviceMesh(v, f))
+    used = []
+    for K in (1, n - 1):
+        before = free()
+        mem = L.allocateMemory(ctypes.byref(tree.ptr), K, n)
+        assert mem.result
+        used.append(before - free())
+        L.freeMemory(ctypes.byref(mem))
+    print(f"{used[0]} bytes with 1 patch, {(used[1] - used[0]) / n:.1f} more per patch", flush=True)
+    assert used[1] - used[0] < 528 * n + (64 << 20)  # allocations are rounded up
