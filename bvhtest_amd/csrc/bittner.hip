@@ -1745,12 +1745,12 @@ void carveState(Internal *in, size_t &words) {
 }
 
 bool features(Internal *in, const bvht_CUDAMemoryBVHPointer *bvh) {
-  if (!in->feat) {
-    if (!devAlloc(&in->feat, (size_t)in->numInner * kFeat, "bn13 features") ||
-        !devAlloc(&in->leafCnt, in->N, "bn13 leaf counts") || !devAlloc(&in->subSA, in->N, "bn13 subtree SA") ||
-        !devAlloc(&in->up, in->N, "bn13 depths"))
-      return false;
-  }
+  // each for itself: a call that failed half way may be made again
+  if ((!in->feat && !devAlloc(&in->feat, (size_t)in->numInner * kFeat, "bn13 features")) ||
+      (!in->leafCnt && !devAlloc(&in->leafCnt, in->N, "bn13 leaf counts")) ||
+      (!in->subSA && !devAlloc(&in->subSA, in->N, "bn13 subtree SA")) ||
+      (!in->up && !devAlloc(&in->up, in->N, "bn13 depths")))
+    return false;
   if (!in->subValid) {
     uint32_t *list = reinterpret_cast<uint32_t *>(in->up);
     if (!computeSubtree(bvh->nodes, in->N, in->leaves, in->numLeaves, in->leafCnt, in->subSA, in->refitCnt, list,
@@ -2074,9 +2074,8 @@ void bn13_selectNodes(bvht_GPUWorkingMemory *data, bvht_CUDAMemoryBVHPointer *bv
     return;
   }
   const uint32_t altTiles = divUp(in->numInner, kAltTile);
-  if (alt && !in->keysAlt &&
-      (!devAlloc(&in->keysAlt, in->numInner, "bn13 altSort keys") ||
-       !devAlloc(&in->altCounts, altTiles, "bn13 altSort counts")))
+  if (alt && ((!in->keysAlt && !devAlloc(&in->keysAlt, in->numInner, "bn13 altSort keys")) ||
+              (!in->altCounts && !devAlloc(&in->altCounts, altTiles, "bn13 altSort counts"))))
     return;
   uint32_t *scratch = in->sortScratch;
   if (!sortReset(in->plan, scratch)) return;
