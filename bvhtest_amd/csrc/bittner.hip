@@ -540,7 +540,7 @@ __global__ __launch_bounds__(64) void k_search(const bvht_BVHNode *__restrict__ 
   if (sortErr && k == 0 && lane == 0 && *sortErr) atomicAdd(stats + ST_SORTERR, 1u);
   PatchRec *rec = recs + k;
   const uint32_t pos = PROBE ? order[k] : order[offsetAccess ? k * numChunks + chunk : chunk * K + k];
-  if (pos >= numInner) {  // block-uniform; only a bad probe list gets here
+  if (pos >= numInner) {  // block-uniform: altSort's entries past the selected, or a bad probe list
     if (!PROBE && lane == 0) rec->ok = REC_NONE;
     return;
   }

@@ -14,11 +14,12 @@
 //     to be entered are kept in a 24-entry per-lane LDS stack of them.  A ray
 //     that needs a 25th starts over with the reference's 128-bit trail and its
 //     parent links (slowWalk), so the common walk carries neither;
-//   * the walk is bound by vector issue and by the L1's accesses (74% and 65
-//     to 83% busy on primary rays at 1080p over 4.2M triangles), so a step
-//     visits an inner node and, if that leads to one, the leaf: a ray's last
-//     box test and its triangle test take one step of the wave.  A lane's own
-//     sequence of visits does not change.
+//   * the walk is bound by the L1's accesses and by vector issue (75% and 59%
+//     of the cycles on primary rays at 1080p over 4.2M triangles, with 29 of 64
+//     lanes active; 49%, 49% and 26 on secondary rays), so a step visits an
+//     inner node and, if that leads to one, the leaf: a ray's last box test and
+//     its triangle test take one step of the wave.  A lane's own sequence of
+//     visits does not change.
 // Measured against separate pair and triangle records, a 16-entry ring and a
 // trail in every walk, one visit a step (1080p, 4.2M triangles; 512x512, 65k):
 // primary rays 3.65 -> 3.27 ms and 278 -> 240 us, secondary rays 4.05 -> 4.00 ms
