@@ -374,6 +374,7 @@ __global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__
     uint32_t sum[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u}, spins = 0;
     for (uint32_t j0 = g; j0 < tile; j0 += QG * QB) {
       BufferU32x4 sv[QB];
+      uint32_t missing = 0;  // a bit per tile to be counted
 #pragma unroll
       for (uint32_t b = 0; b < QB; ++b) {
         const uint32_t j = j0 + b * QG;
@@ -391,10 +392,19 @@ __global__ __launch_bounds__(BLOCK, 1) void k_onesweepWide(const K *__restrict__
           memoryChanged();
           v = bufferLoadU32x4Coherent(st, (j * kWideStatusWords + 4 * q) * 4u);
           if (++spins >= polls && ((v[0] & v[1] & v[2] & v[3]) & ready) != ready) {
-            v = countTile<TILE, sizeof(K)>(keys, j, dw, dshift, q);
+            v = BufferU32x4{kHalfFlags, kHalfFlags, kHalfFlags, kHalfFlags};
+            missing |= 1u << b;
             break;
           }
         }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          sum[2 * c] += v[c] & kHalfCount;
+          sum[2 * c + 1] += (v[c] >> 16) & kHalfCount;
+        }
+      }
+      for (; __builtin_expect(missing != 0, 0); missing &= missing - 1) {
+        const BufferU32x4 v = countTile<TILE, sizeof(K)>(keys, j0 + (uint32_t)__builtin_ctz(missing) * QG, dw, dshift, q);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           sum[2 * c] += v[c] & kHalfCount;
